@@ -226,8 +226,8 @@ int sfx_get_sizes(const sfx_engine *engine, int64_t *sizes7);
  * or 9 control nodes (2-D gather path; the same bits as the per-point
  * arrays); [1] 1 if the 2-D gather path reads kappa and mu once per element
  * (both the same at all points of every element), else 0; [2] the scatter
- * mode; [3] 1 if the device numbers the points in coordinate row order (2-D
- * gather path), else 0. */
+ * mode; [3] 1 if the device numbers the points by their place in the mesh
+ * (2-D gather path: patch by patch), else 0. */
 int sfx_get_layout(const sfx_engine *engine, int64_t *layout4);
 /* Per-medium sizes of a 2-D mesh (specfem::compute::simulation_field's
  * per-medium fields, field_impl.tpp:23-103): elastic elements, acoustic

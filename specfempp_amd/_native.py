@@ -17,7 +17,7 @@ LIB_PATH = os.path.join(LIB_DIR, "libspecfempp_amd.so")
 HEADER = os.path.join(os.path.dirname(HERE), "include", "specfempp_amd.h")
 
 SOURCES = ["engine.hip", "kernels.hip", "acoustic.hip", "general3d.hip", "block3d.hip", "batch.hip",
-           "assembly.cpp"]
+           "patch2d.hip", "patch2d.cpp", "assembly.cpp"]
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
     # packed FP32 instructions stay off: some of their forms have given wrong

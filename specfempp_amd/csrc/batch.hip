@@ -11,9 +11,10 @@
 //     constants (dt differs per simulation) once;
 //   - Stacey entries, sources and receivers are concatenated in the same order.
 // Three scatters, chosen by the autotuner or the caller:
-//   - SFX_SCATTER_GATHER: one launch per time step (batch_step_kernel) over
-//     the elements in simulation-major, element order; the state is
-//     double-buffered so that no grid-wide synchronisation is needed;
+//   - SFX_SCATTER_GATHER: one launch per time step over the patches of every
+//     running simulation (patch2d.hpp), the kernel and the operations of a
+//     single engine's gather scatter, so a simulation in the batch gives its
+//     engine's results bit for bit;
 //   - SFX_SCATTER_COLORED / _ATOMIC: a step is sources, stiffness per color
 //     (elements color-major, then by simulation, so each color's running
 //     elements are a prefix of the color's range), Stacey, seismograms, fused
@@ -35,7 +36,7 @@
 #include "../../include/specfempp_amd.h"
 #include "assembly.hpp"
 #include "kernels.hpp"
-#include "lattice.hpp"
+#include "patch2d.hpp"
 #include "runtime.hpp"
 
 namespace sfx {
@@ -137,293 +138,6 @@ __global__ void batch_tick_kernel(int *step) {
   if (threadIdx.x == 0) *step = *step + 1;
 }
 
-// ---------------------------------------------------------------------------
-// One launch per time step (scatter SFX_SCATTER_GATHER).
-//
-// Launch n carries every simulation from the unassembled forces of step n - 1
-// to those of step n with no grid-wide synchronisation: the state is
-// double-buffered by the parity of n.  Buffers A (read) hold u, v predicted
-// for step n - 1 and the element forces of step n - 1 (stiffness, Stacey,
-// sources; RE2_ELEM floats per element); buffers B (written) receive the same
-// for step n.  Each element point
-//   1. sums the step n - 1 contributions of its global point from A in a fixed
-//      order (by element, then point), divides by the mass and applies
-//      corrector n - 1 and predictor n to A's u, v; every element point of a
-//      global point does this with the same operands, so all hold the same
-//      values, and one of them (the point's first contribution) writes u, v
-//      to B;
-//   2. samples the step n - 1 seismograms of receivers in its element (u from
-//      A, v corrected, a) when that step is a sampling step;
-//   3. computes the element's weak-form force of step n from the predicted u
-//      (as elemforce_2d_kernel), adds the Stacey traction of its boundary
-//      entries with the predicted v (as stacey_re2_kernel) and the sources of
-//      its element in application order (as sources_re2_kernel), and stores
-//      the element's forces to B with coalesced 16-byte writes.
-// The step index lives in two device counters: launch n reads ctr[n % 2] and
-// its first workgroup writes ctr[(n + 1) % 2] = n + 1, so a captured pair of
-// launches replays for any even n.  Launch nstep_max only samples.
-// Each stage performs the operations of the single-engine gather path in the
-// same order (elemforce_2d_kernel, stacey_re2_kernel, sources_re2_kernel,
-// assemble_update_2d_kernel, seismogram_kernel's 64-lane reduction), with no
-// contraction into fused multiply-adds in either, so a simulation in the
-// batch gives its engine's gather-path results bit for bit.
-// ---------------------------------------------------------------------------
-struct StepTables {
-  const int *gather;        // (nel, 25) arena point of each element point
-  const float *geo;         // (nel, 8) affine geometry record, or null
-  const float *xix, *xiz, *gammax, *gammaz, *jac;  // (nel, 25) when geo is null
-  const float *kappa, *mu;  // (nel, 25)
-  const int *elem_sim;      // (nel) simulation of each element
-  const int *off;           // (npts + 1) contributions of each point: [off[g], off[g+1])
-  const int *ent;           // element * RE2_ELEM + 2 p of each contribution
-  const int *seg_elem;      // (nel + 1) boundary segments of each element
-  const int *seg_pt;        // element point of each segment
-  const int *seg_off;       // (nseg + 1) Stacey entries of each segment
-  const float *bnormal, *bweight, *brvp, *brvs;
-  const int *src_elem;      // (nel + 1) sources of each element, application order
-  const int *src_id;
-  const float *src_array;   // (nsrc, 2, 25)
-  const float *stf;         // (nsrc, nstep_max)
-  const int *rec_elem;      // (nel + 1) receivers of each element
-  const int *rec_id;
-  const float *rec_h;       // (nrec, 25)
-  const int *rec_local;     // receiver index within its simulation
-  const int *nstep, *nsb, *nrec_sim;
-  const long long *seis_off;
-  const float *ncs;         // (nsim, 3) dt, dt/2, dt^2/2
-  const int *types;
-  const float *minv;        // (2, npts)
-  float *seismo;
-  int ntypes, nstep_max, npts;
-};
-
-struct StepState {
-  float *u[2], *v[2], *re[2];
-  int *ctr;  // (2)
-};
-
-template <int E> constexpr int step_threads() { return (E * 25 + 63) / 64 * 64; }
-// contributions of a point loaded together before the sum (the rest one by one)
-constexpr int STEP_BATCH = 4;
-
-template <int E>
-__global__ __launch_bounds__(step_threads<E>()) void batch_step_kernel(int par, int nel, StepTables T, StepState S,
-                                                                      GllConst q) {
-  // every product and sum rounded on its own, as in the engine's gather-path
-  // kernels, so both give the same bits
-#pragma clang fp contract(off)
-  __shared__ float su[E][2][25];
-  __shared__ float sF[E][4][25];  // F(c, d) as [2c + d]
-  __shared__ __align__(16) float st[E * RE2_ELEM];
-  __shared__ float ss[E][3][2][25];  // samples: u, corrected v, a
-
-  const int n = S.ctr[par];
-  if (blockIdx.x == 0 && threadIdx.x == 0) S.ctr[par ^ 1] = n + 1;
-  const int t = threadIdx.x;
-  const int el = t / 25;
-  const int p = t - el * 25;
-  const int iz = p / 5, ix = p - (p / 5) * 5;
-  const int first = xcd_block(blockIdx.x, gridDim.x) * E;
-  const int e = first + el;
-  const bool inside = (el < E) && (e < nel);
-  const int np = T.npts;
-  const float *UA = S.u[par], *VA = S.v[par], *reA = S.re[par];
-  float *UB = S.u[par ^ 1], *VB = S.v[par ^ 1], *reB = S.re[par ^ 1];
-
-  // Every lane issues all of its loads here, before the first barrier and
-  // without branches around them (lanes past the last element re-read it; all
-  // addresses are valid): the element's simulation and the point's gather
-  // index, then the point's contribution bounds, state and M^-1, the
-  // simulation's constants, the first STEP_BATCH contributions and the
-  // element's properties and geometry, so their latencies overlap.
-  const int ec = e < nel ? e : nel - 1;
-  const size_t idx = static_cast<size_t>(ec) * 25 + p;
-  const int sim_l = T.elem_sim[ec];
-  const int g = T.gather[idx];
-  const int ns = T.nstep[sim_l], nsb = T.nsb[sim_l];
-  const float dt = T.ncs[3 * sim_l], dto2 = T.ncs[3 * sim_l + 1], dt2o2 = T.ncs[3 * sim_l + 2];
-  const int k0 = T.off[g], k1 = T.off[g + 1];
-  float minv[2], ua[2], va[2];
-#pragma unroll
-  for (int c = 0; c < 2; c++) {
-    const size_t o = static_cast<size_t>(c) * np + g;
-    minv[c] = T.minv[o];
-    ua[c] = UA[o];
-    va[c] = VA[o];
-  }
-  int en[STEP_BATCH];
-#pragma unroll
-  for (int j = 0; j < STEP_BATCH; j++) en[j] = T.ent[k0 + j < k1 ? k0 + j : k1 - 1];
-  float2 rj[STEP_BATCH];
-#pragma unroll
-  for (int j = 0; j < STEP_BATCH; j++) rj[j] = *reinterpret_cast<const float2 *>(reA + en[j]);
-  const float kappa = T.kappa[idx], mu = T.mu[idx];
-  const size_t gr = static_cast<size_t>(ec) * 8;
-  const float xix = T.geo ? T.geo[gr] : T.xix[idx];
-  const float xiz = T.geo ? T.geo[gr + 1] : T.xiz[idx];
-  const float gammax = T.geo ? T.geo[gr + 2] : T.gammax[idx];
-  const float gammaz = T.geo ? T.geo[gr + 3] : T.gammaz[idx];
-  const float J = T.geo ? T.geo[gr + 4] : T.jac[idx];
-  float hpx[5], hpz[5], hwx[5], hwz[5];
-#pragma unroll
-  for (int l = 0; l < 5; l++) {
-    hpx[l] = q.hp[ix][l];
-    hpz[l] = q.hp[iz][l];
-    hwx[l] = q.hpw[ix][l];
-    hwz[l] = q.hpw[iz][l];
-  }
-  const float wx = q.w[ix], wz = q.w[iz];
-
-  int sim = 0;
-  bool forces = false, sample = false;
-  if (inside) {
-    sim = sim_l;
-    forces = n < ns;
-    sample = n >= 1 && n - 1 < ns && (n - 1) % nsb == 0;
-  }
-  float un[2] = {0.0f, 0.0f}, vn[2] = {0.0f, 0.0f};
-  if (forces || sample) {
-    float sum[2] = {0.0f, 0.0f};
-#pragma unroll
-    for (int j = 0; j < STEP_BATCH; j++)
-      if (k0 + j < k1) {
-        sum[0] += rj[j].x;
-        sum[1] += rj[j].y;
-      }
-    for (int k = k0 + STEP_BATCH; k < k1; k++) {
-      const float2 r = *reinterpret_cast<const float2 *>(reA + T.ent[k]);
-      sum[0] += r.x;
-      sum[1] += r.y;
-    }
-    const bool owner = forces && en[0] == e * RE2_ELEM + 2 * p;
-#pragma unroll
-    for (int c = 0; c < 2; c++) {
-      const size_t o = static_cast<size_t>(c) * np + g;
-      const float a = sum[c] * minv[c];
-      const float u0 = ua[c];
-      const float v1 = va[c] + dto2 * a;
-      un[c] = u0 + (dt * v1 + dt2o2 * a);
-      vn[c] = v1 + dto2 * a;
-      if (sample) {
-        ss[el][0][c][p] = u0;
-        ss[el][1][c][p] = v1;
-        ss[el][2][c][p] = a;
-      }
-      if (owner) {
-        UB[o] = un[c];
-        VB[o] = vn[c];
-      }
-    }
-  }
-  if (inside) {
-    su[el][0][p] = un[0];
-    su[el][1][p] = un[1];
-  }
-  __syncthreads();
-
-  // step n - 1 samples: one thread per receiver; the reduction is the 64-lane
-  // shuffle tree of seismogram_kernel (values in lanes 0-24, zeros above)
-  if (sample && p == 0) {
-    const int isig = (n - 1) / T.nsb[sim];
-    for (int k = T.rec_elem[e]; k < T.rec_elem[e + 1]; k++) {
-      const int r = T.rec_id[k];
-      const float *hw = T.rec_h + static_cast<size_t>(r) * 25;
-      for (int it = 0; it < T.ntypes; it++) {
-        const int type = T.types[it];
-#pragma unroll
-        for (int c = 0; c < 2; c++) {
-          float s32[32];
-#pragma unroll
-          for (int i = 0; i < 32; i++) s32[i] = (i < 25 ? hw[i] * ss[el][type][c][i] : 0.0f) + 0.0f;
-#pragma unroll
-          for (int w = 16; w > 0; w >>= 1)
-#pragma unroll
-            for (int i = 0; i < w; i++) s32[i] = s32[i] + s32[i + w];
-          T.seismo[T.seis_off[sim] + ((static_cast<long long>(isig) * T.ntypes + it) * T.nrec_sim[sim] +
-                                      T.rec_local[r]) * 2 + c] = s32[0] + 0.0f;
-        }
-      }
-    }
-  }
-
-  if (forces) {
-    float dxi[2] = {0.0f, 0.0f}, dga[2] = {0.0f, 0.0f};
-#pragma unroll
-    for (int l = 0; l < 5; l++) {
-#pragma unroll
-      for (int c = 0; c < 2; c++) {
-        dxi[c] += hpx[l] * su[el][c][iz * 5 + l];
-        dga[c] += hpz[l] * su[el][c][l * 5 + ix];
-      }
-    }
-    float du[2][2];
-#pragma unroll
-    for (int c = 0; c < 2; c++) {
-      du[c][0] = xix * dxi[c] + gammax * dga[c];
-      du[c][1] = xiz * dxi[c] + gammaz * dga[c];
-    }
-    const float lp2m = kappa + (4.0f / 3.0f) * mu;
-    const float lambda = lp2m - 2.0f * mu;
-    const float sxx = lp2m * du[0][0] + lambda * du[1][1];
-    const float szz = lp2m * du[1][1] + lambda * du[0][0];
-    const float sxz = mu * (du[0][1] + du[1][0]);
-    sF[el][0][p] = J * (sxx * xix + sxz * xiz);
-    sF[el][1][p] = J * (sxx * gammax + sxz * gammaz);
-    sF[el][2][p] = J * (sxz * xix + szz * xiz);
-    sF[el][3][p] = J * (sxz * gammax + szz * gammaz);
-  }
-  __syncthreads();
-  if (inside) {
-    float r[2] = {0.0f, 0.0f};
-    if (forces) {
-      float t1[2] = {0.0f, 0.0f}, t2[2] = {0.0f, 0.0f};
-#pragma unroll
-      for (int l = 0; l < 5; l++) {
-#pragma unroll
-        for (int c = 0; c < 2; c++) {
-          t1[c] += sF[el][2 * c][iz * 5 + l] * hwx[l];
-          t2[c] += sF[el][2 * c + 1][l * 5 + ix] * hwz[l];
-        }
-      }
-#pragma unroll
-      for (int c = 0; c < 2; c++) r[c] = -(wz * t1[c] + wx * t2[c]);
-      // Stacey traction with the predicted velocity (the entries of this
-      // element point, summed in order, then added once)
-      for (int sg = T.seg_elem[e]; sg < T.seg_elem[e + 1]; sg++) {
-        if (T.seg_pt[sg] != p) continue;
-        float sum[2] = {0.0f, 0.0f};
-        for (int qq = T.seg_off[sg]; qq < T.seg_off[sg + 1]; qq++) {
-          const float nv[2] = {T.bnormal[2 * qq], T.bnormal[2 * qq + 1]};
-          const float vnn = vn[0] * nv[0] + vn[1] * nv[1];
-          const float nn = nv[0] * nv[0] + nv[1] * nv[1];
-          const float j1 = sqrtf(nn);
-          const float w = T.bweight[qq], rvp = T.brvp[qq], rvs = T.brvs[qq];
-#pragma unroll
-          for (int d = 0; d < 2; d++) {
-            const float fac = ((vnn * nv[d] / (j1 * j1)) * (rvp - rvs)) + vn[d] * rvs;
-            sum[d] += -1.0f * fac * j1 * w;
-          }
-        }
-        r[0] += sum[0];
-        r[1] += sum[1];
-      }
-      for (int k = T.src_elem[e]; k < T.src_elem[e + 1]; k++) {
-        const int s = T.src_id[k];
-        const float sv = T.stf[static_cast<size_t>(s) * T.nstep_max + n];
-#pragma unroll
-        for (int c = 0; c < 2; c++) r[c] += sv * T.src_array[(static_cast<size_t>(s) * 2 + c) * 25 + p];
-      }
-    }
-    st[el * RE2_ELEM + 2 * p] = r[0];
-    st[el * RE2_ELEM + 2 * p + 1] = r[1];
-  }
-  __syncthreads();
-  const int nb = nel - first < E ? nel - first : E;
-  float4 *dst = reinterpret_cast<float4 *>(reB + static_cast<size_t>(first) * RE2_ELEM);
-  const float4 *from = reinterpret_cast<const float4 *>(st);
-  for (int qv = t; qv < nb * (RE2_ELEM / 4); qv += step_threads<E>()) dst[qv] = from[qv];
-}
-
 }  // namespace
 }  // namespace sfx
 
@@ -454,14 +168,13 @@ struct sfx_batch {
   DevBuf<float> xix, xiz, gammax, gammaz, jac, kappa, mu, bnd_normal, bnd_weight, bnd_rvp, bnd_rvs, src_array, stf,
       rec_h, seismo, fields, ncs;
   int nsrc = 0, nrec_total = 0;
-  // one-launch-per-step layout (SFX_SCATTER_GATHER): elements in simulation-
-  // major, element order; elem_cnt_f[k] elements belong to the first k
-  // simulations
-  int nel_f = 0;
-  std::vector<int> elem_cnt_f;
-  DevBuf<int> f_gather, f_elem_sim, f_off, f_ent, f_seg_elem, f_seg_pt, f_seg_off, f_src_elem, f_src_id, f_rec_elem,
-      f_rec_id, ctr;
-  DevBuf<float> f_geo, f_xix, f_xiz, f_gx, f_gz, f_jac, f_kappa, f_mu, f_bn, f_bw, f_bp, f_bs, re;
+  // one launch per step (SFX_SCATTER_GATHER): the patches of all simulations,
+  // their state u, v (2 points each) and M^-1; ctr: step of the next even and
+  // odd launch
+  PatchDevice patch;
+  DevBuf<float> pfields;
+  DevBuf<int> ctr;
+  size_t pts = 0;
   // tuning
   int scatter = SFX_SCATTER_GATHER;
   int elems_per_block = 5;
@@ -469,61 +182,22 @@ struct sfx_batch {
   double last_run_ms = 0.0;
   std::vector<hipGraphExec_t> graph_cache;  // per k (nullptr until captured)
 
-  // fields: u, v, a, M^-1 (2 npts each), then the second u, v of the
-  // double-buffered one-launch-per-step state
   Fields f() const {
     const size_t stride = 2 * npts;
     return Fields{fields.p, fields.p + stride, fields.p + 2 * stride, fields.p + 3 * stride, static_cast<int>(npts)};
   }
-  StepState step_state() const {
-    const size_t stride = 2 * npts;
-    const size_t nre = static_cast<size_t>(nel_f) * RE2_ELEM;
-    return StepState{{fields.p, fields.p + 4 * stride},
-                     {fields.p + stride, fields.p + 5 * stride},
-                     {re.p, re.p + nre},
-                     ctr.p};
-  }
-  StepTables step_tables() const {
-    StepTables T{};
-    T.gather = f_gather.p;
-    T.geo = f_geo.p;
-    T.xix = f_xix.p;
-    T.xiz = f_xiz.p;
-    T.gammax = f_gx.p;
-    T.gammaz = f_gz.p;
-    T.jac = f_jac.p;
-    T.kappa = f_kappa.p;
-    T.mu = f_mu.p;
-    T.elem_sim = f_elem_sim.p;
-    T.off = f_off.p;
-    T.ent = f_ent.p;
-    T.seg_elem = f_seg_elem.p;
-    T.seg_pt = f_seg_pt.p;
-    T.seg_off = f_seg_off.p;
-    T.bnormal = f_bn.p;
-    T.bweight = f_bw.p;
-    T.brvp = f_bp.p;
-    T.brvs = f_bs.p;
-    T.src_elem = f_src_elem.p;
-    T.src_id = f_src_id.p;
-    T.src_array = src_array.p;
-    T.stf = stf.p;
-    T.rec_elem = f_rec_elem.p;
-    T.rec_id = f_rec_id.p;
-    T.rec_h = rec_h.p;
-    T.rec_local = rec_local.p;
-    T.nstep = d_nstep.p;
-    T.nsb = d_nsb.p;
-    T.nrec_sim = d_nrec.p;
-    T.seis_off = d_seis_off.p;
-    T.ncs = ncs.p;
-    T.types = d_types.p;
-    T.minv = fields.p + 6 * npts;
-    T.seismo = seismo.p;
-    T.ntypes = ntypes;
-    T.nstep_max = nstep_max;
-    T.npts = static_cast<int>(npts);
-    return T;
+  PatchTables patch_tables() const {
+    PatchTables t = patch.t;
+    t.src_array = src_array.p;
+    t.stf = stf.p;
+    t.stf_step = 1;
+    t.stf_src = nstep_max;
+    t.types = d_types.p;
+    t.ntypes = ntypes;
+    t.minv = pfields.p + 4 * pts;
+    t.seismo = seismo.p;
+    t.np = static_cast<int>(pts);
+    return t;
   }
 
   ~sfx_batch() {
@@ -698,95 +372,30 @@ struct sfx_batch {
     }
     nsrc = static_cast<int>(ssim_h.size());
     nrec_total = static_cast<int>(rsim_h.size());
-    // one-launch-per-step layout: simulation k's element ce is element
-    // ebase[k] + ce; a point's contributions are listed by element, then by
-    // point, the order in which an engine's gather path sums them
-    std::vector<int> ebase(nsim + 1, 0);
-    for (int k = 0; k < nsim; k++) ebase[k + 1] = ebase[k] + H[k]->nspec;
-    nel_f = ebase[nsim];
-    if (static_cast<long long>(nel_f) * RE2_ELEM > INT_MAX) throw std::invalid_argument("batch too large");
-    elem_cnt_f = ebase;
-    bool affine = true;
-    for (int k = 0; k < nsim; k++) affine = affine && !H[k]->geo2d.empty();
-    std::vector<int> fg_h(static_cast<size_t>(nel_f) * 25), fsim_h(nel_f);
-    std::vector<float> fk_h(fg_h.size()), fm_h(fg_h.size()), fgeo_h, fx_h, fxz_h, fgx_h, fgz_h, fj_h;
-    if (affine)
-      fgeo_h.resize(static_cast<size_t>(nel_f) * 8);
-    else
-      for (auto *v : {&fx_h, &fxz_h, &fgx_h, &fgz_h, &fj_h}) v->resize(fg_h.size());
-    std::vector<int> off_h(npts + 1, 0), ent_h;
-    std::vector<int> sege_h(nel_f + 1, 0), segp_h, sego_h(1, 0);
-    std::vector<float> fbn_h, fbw_h, fbp_h, fbs_h;
-    std::vector<int> srce_h(nel_f + 1, 0), srcid_h, rece_h(nel_f + 1, 0), recid_h;
+    // one launch per step: a point's contributions are summed by element, the
+    // order of an engine's gather scatter
+    PatchPlan plan;
     {
-      int src_base = 0, rec_base = 0;
-      std::vector<std::vector<int>> src_of(nel_f), rec_of(nel_f);
+      int64_t nspec = 0;
+      for (int k = 0; k < nsim; k++) nspec += H[k]->nspec;
+      plan.pe = patch_elements(nspec);
+      std::vector<int32_t> key;
       for (int k = 0; k < nsim; k++) {
-        const HostAssembly &h = *H[k];
-        for (int ce = 0; ce < h.nspec; ce++) {
-          const int e = ebase[k] + ce;
-          fsim_h[e] = k;
-          for (int p = 0; p < 25; p++) {
-            const size_t d = static_cast<size_t>(e) * 25 + p, src = static_cast<size_t>(ce) * 25 + p;
-            fg_h[d] = h.gather[src] + pt_off[k];
-            fk_h[d] = h.kappa[src];
-            fm_h[d] = h.mu[src];
-            if (!affine) {
-              fx_h[d] = h.xix[src];
-              fxz_h[d] = h.xiz[src];
-              fgx_h[d] = h.gammax[src];
-              fgz_h[d] = h.gammaz[src];
-              fj_h[d] = h.jac[src];
-            }
-          }
-          if (affine) std::memcpy(&fgeo_h[static_cast<size_t>(e) * 8], &h.geo2d[static_cast<size_t>(ce) * 8], 32);
-        }
-        for (size_t i = 0; i < static_cast<size_t>(h.nspec) * 25; i++) off_h[pt_off[k] + h.gather[i] + 1]++;
-        // Stacey entries grouped by element point (stable: edge order kept)
-        std::vector<size_t> ord(h.bnd_gather.size());
-        std::iota(ord.begin(), ord.end(), 0);
-        std::stable_sort(ord.begin(), ord.end(), [&](size_t a, size_t b) { return h.bnd_slot[a] < h.bnd_slot[b]; });
-        for (size_t i = 0; i < ord.size(); i++) {
-          const size_t qq = ord[i];
-          if (i == 0 || h.bnd_slot[qq] != h.bnd_slot[ord[i - 1]]) {
-            if (i > 0) sego_h.push_back(static_cast<int>(fbw_h.size()));
-            segp_h.push_back(h.bnd_slot[qq] % 25);
-            sege_h[ebase[k] + h.bnd_slot[qq] / 25 + 1]++;
-          }
-          fbn_h.push_back(h.bnd_normal[2 * qq]);
-          fbn_h.push_back(h.bnd_normal[2 * qq + 1]);
-          fbw_h.push_back(h.bnd_weight[qq]);
-          fbp_h.push_back(h.bnd_rho_vp[qq]);
-          fbs_h.push_back(h.bnd_rho_vs[qq]);
-        }
-        if (!ord.empty()) sego_h.push_back(static_cast<int>(fbw_h.size()));
-        for (size_t i = 0; i < h.src_order.size(); i++)
-          src_of[ebase[k] + h.src_ispec[h.src_order[i]]].push_back(src_base + static_cast<int>(i));
-        src_base += static_cast<int>(h.src_order.size());
-        for (int r = 0; r < h.nrec; r++) rec_of[ebase[k] + h.rec_ispec[r]].push_back(rec_base + r);
-        rec_base += h.nrec;
+        key.resize(H[k]->nspec);
+        std::iota(key.begin(), key.end(), 0);
+        add_patches(plan, *H[k], key, false);
       }
-      for (size_t g = 0; g < npts; g++) off_h[g + 1] += off_h[g];
-      ent_h.resize(off_h[npts]);
-      std::vector<int> fill(off_h.begin(), off_h.end() - 1);
-      for (int k = 0; k < nsim; k++) {
-        const HostAssembly &h = *H[k];
-        for (int ce = 0; ce < h.nspec; ce++) {
-          for (int p = 0; p < 25; p++) {
-            const int g = pt_off[k] + h.gather[static_cast<size_t>(ce) * 25 + p];
-            ent_h[fill[g]++] = (ebase[k] + ce) * RE2_ELEM + 2 * p;
-          }
-        }
-      }
-      for (int e = 0; e < nel_f; e++) {
-        sege_h[e + 1] += sege_h[e];
-        srce_h[e + 1] = srce_h[e] + static_cast<int>(src_of[e].size());
-        rece_h[e + 1] = rece_h[e] + static_cast<int>(rec_of[e].size());
-        srcid_h.insert(srcid_h.end(), src_of[e].begin(), src_of[e].end());
-        recid_h.insert(recid_h.end(), rec_of[e].begin(), rec_of[e].end());
-      }
-      if (sege_h[nel_f] != static_cast<int>(segp_h.size()) || sego_h.size() != segp_h.size() + 1)
-        throw std::logic_error("batch: Stacey segments are inconsistent");
+      finish_patches(plan);
+    }
+    pts = (static_cast<size_t>(plan.nint) + plan.nbnd + 63) / 64 * 64;
+    std::vector<float> pminv_h(2 * pts, 0.0f);
+    std::vector<PatchSim> sims(nsim);
+    for (int k = 0; k < nsim; k++) {
+      const HostAssembly &h = *H[k];
+      for (int c = 0; c < 2; c++)
+        for (int g = 0; g < h.nglob; g++)
+          pminv_h[c * pts + plan.device_of[k][g]] = h.mass_inverse[static_cast<size_t>(c) * h.nglob_pad + g];
+      sims[k] = PatchSim{ncs_h[3 * k], ncs_h[3 * k + 1], ncs_h[3 * k + 2], nstep[k], nsb[k], nrec[k], seis_off[k]};
     }
     // upload
     SFX_HIP(hipStreamCreate(&stream));
@@ -819,36 +428,12 @@ struct sfx_batch {
     d_nrec.upload(nrec, s);
     d_seis_off.upload(seis_off, s);
     ncs.upload(ncs_h, s);
-    f_gather.upload(fg_h, s);
-    f_elem_sim.upload(fsim_h, s);
-    f_kappa.upload(fk_h, s);
-    f_mu.upload(fm_h, s);
-    if (affine) {
-      f_geo.upload(fgeo_h, s);
-    } else {
-      f_xix.upload(fx_h, s);
-      f_xiz.upload(fxz_h, s);
-      f_gx.upload(fgx_h, s);
-      f_gz.upload(fgz_h, s);
-      f_jac.upload(fj_h, s);
-    }
-    f_off.upload(off_h, s);
-    f_ent.upload(ent_h, s);
-    f_seg_elem.upload(sege_h, s);
-    f_seg_pt.upload(segp_h, s);
-    f_seg_off.upload(sego_h, s);
-    f_bn.upload(fbn_h, s);
-    f_bw.upload(fbw_h, s);
-    f_bp.upload(fbp_h, s);
-    f_bs.upload(fbs_h, s);
-    f_src_elem.upload(srce_h, s);
-    f_src_id.upload(srcid_h, s);
-    f_rec_elem.upload(rece_h, s);
-    f_rec_id.upload(recid_h, s);
-    re.alloc(2 * static_cast<size_t>(nel_f) * RE2_ELEM);
+    patch.upload(plan, H, true, sims, s);
+    pfields.alloc(6 * pts);
+    SFX_HIP(hipMemcpyAsync(pfields.p + 4 * pts, pminv_h.data(), 2 * pts * sizeof(float), hipMemcpyHostToDevice, s));
     ctr.alloc(2);
     seismo.alloc(std::max<long long>(seis_off[nsim], 1));
-    fields.alloc(12 * npts);
+    fields.alloc(8 * npts);
     SFX_HIP(hipMemcpyAsync(fields.p + 6 * npts, minv_h.data(), 2 * npts * sizeof(float), hipMemcpyHostToDevice, s));
     step.alloc(1);
     SFX_HIP(hipStreamSynchronize(s));
@@ -890,30 +475,20 @@ struct sfx_batch {
     hipLaunchKernelGGL(batch_tick_kernel, dim3(1), dim3(64), 0, s, step.p);
   }
 
-  // Launch n (n % 2 == par) of the one-launch-per-step scatter over the
-  // elements of the first k simulations.
+  // Launch n (n % 2 == par) of the one-launch-per-step scatter over the first
+  // k simulations.  It reads its step from ctr[par] and leaves n + 1 in
+  // ctr[par ^ 1], so a captured pair replays for every even n.
   void enqueue_launch(int par, int k) {
-    const int nel = elem_cnt_f[k];
-    if (nel <= 0) return;
-    const StepTables T = step_tables();
-    const StepState S = step_state();
-    const unsigned nb = static_cast<unsigned>((nel + elems_per_block - 1) / elems_per_block);
-    switch (elems_per_block) {
-      case 2:
-        hipLaunchKernelGGL(batch_step_kernel<2>, dim3(nb), dim3(step_threads<2>()), 0, stream, par, nel, T, S, q);
-        break;
-      case 10:
-        hipLaunchKernelGGL(batch_step_kernel<10>, dim3(nb), dim3(step_threads<10>()), 0, stream, par, nel, T, S, q);
-        break;
-      default:
-        hipLaunchKernelGGL(batch_step_kernel<5>, dim3(nb), dim3(step_threads<5>()), 0, stream, par, nel, T, S, q);
-    }
+    if (k <= 0) return;
+    const PatchState st = patch.state(pfields.p, pfields.p + 2 * pts, nullptr);
+    launch_patch_step(stream, patch.pe, patch.patch_end[k - 1], patch.rec_end[k - 1], true, patch_tables(), st, q,
+                      PatchLaunch{ctr.p + par, ctr.p + (par ^ 1), 0, par, 1, 1, 0});
   }
 
   void reset() {
     launch_fill(stream, fields.p, 6 * npts, 0.0f);
-    launch_fill(stream, fields.p + 8 * npts, 4 * npts, 0.0f);
-    launch_fill(stream, re.p, re.n, 0.0f);
+    launch_fill(stream, pfields.p, 4 * pts, 0.0f);
+    launch_fill(stream, patch.work.p, patch.work.n, 0.0f);
     launch_fill(stream, seismo.p, seismo.n, 0.0f);
     const int zero[2] = {0, 0};
     SFX_HIP(hipMemcpyAsync(step.p, zero, sizeof(int), hipMemcpyHostToDevice, stream));
@@ -1049,6 +624,7 @@ int sfx_batch_tune(sfx_batch *b, int steps_per_candidate, int *choice4) {
     for (int sc : {SFX_SCATTER_GATHER, SFX_SCATTER_COLORED, SFX_SCATTER_ATOMIC})
       for (int e : {2, 5, 10})
         for (bool g : {false, true}) {
+          if (sc == SFX_SCATTER_GATHER && e != 5) continue;  // its patches do not depend on it
           b->scatter = sc;
           b->elems_per_block = e;
           b->use_graph = g;

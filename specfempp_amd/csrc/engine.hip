@@ -19,6 +19,7 @@
 #include "assembly.hpp"
 #include "kernels.hpp"
 #include "lattice.hpp"
+#include "patch2d.hpp"
 #include "runtime.hpp"
 
 namespace sfx {
@@ -78,18 +79,17 @@ struct sfx_engine {
   DevBuf<float> xix, xiz, gammax, gammaz, jac, kappa, mu;
   DevBuf<float> geo;     // 2-D affine meshes: one geometry record per element (the forward stiffness reads it)
   DevBuf<float> geo3;    // 3-D database meshes: per-point derivatives and jacobian (nspec, 10, 125)
-  // 2-D gather path: element forces, the per-point inverse index, Stacey
-  // entries sorted by element point with their segments
-  DevBuf<float> re2;
-  // 2-D gather path on meshes without constant element geometry: the control
-  // nodes per element and the shape derivatives at the GLL points, from which
-  // the element forces recompute each point's geometry; and (2-D and 3-D
-  // gather paths) (kappa, mu) per element when both are the same at all
+  // 2-D elastic engines (COLORED and GATHER): the patches that carry the
+  // forward steps
+  PatchPlan plan;
+  PatchDevice patch;
+  // 3-D gather path: (kappa, mu) per element when both are the same at all
   // points of every element
-  DevBuf<float> ctrl, dsh, kmu_e;
-  DevBuf<int> inv_off, inv_ent, g2_seg, g2_gather, g2_slot;
-  DevBuf<float> g2_normal, g2_weight, g2_rvp, g2_rvs;
-  int g2_nseg = 0;
+  DevBuf<float> kmu_e;
+  // API point order -> device order (lattice_of on the device) and a
+  // component's staging copy, at first use
+  DevBuf<int> d_lattice;
+  DevBuf<float> stage;
   DevBuf<float> bnd_normal, bnd_weight, bnd_rvp, bnd_rvs;
   DevBuf<float> src_array, stf, rec_h, seismo;
   DevBuf<float> fields;  // u, v, a, minv: 4 * ncomp * nglob_pad
@@ -128,7 +128,8 @@ struct sfx_engine {
   bool use_graphs = true;
   float *rec_step = nullptr;
   bool initialized = false;
-  bool a_stale = false;  // fused gather steps leave the stored acceleration behind
+  bool a_stale = false;  // fused 3-D gather steps leave the stored acceleration behind
+  bool a_kept = false;   // 2-D patches: the stored acceleration may be nonzero (the colored kernels add to it)
   int nbseg = 0;         // Stacey segments (3-D)
   bool sources_off_boundary = false;  // 3-D gather: no source element has an absorbing face
   DevBuf<float> minv1;                // 3-D gather: M^-1 of one component (nglob_pad)
@@ -192,15 +193,6 @@ struct sfx_engine {
   // device counter; recording adds the Stacey-element record.
   void enqueue_forward_2d(bool record_on) {
     Fields ff = f();
-    if (gather2d()) {
-      forces_2d(ff, 0, d_step.p);
-      launch_seismograms(stream, 2, h.npe, h.nrec, run.nseismo_types, types.p, 0, rec_ispec.p, gather.p, rec_h.p, ff,
-                         nc.dto2, 1, seismo.p, PointGeom2D{xix.p, xiz.p, gammax.p, gammaz.p, kappa.p, mu.p}, q,
-                         d_step.p, run.nstep_between_samples, -1, fs2());
-      launch_assemble_update_2d(stream, h.nglob, fs2(), ff, nc, 0);
-      launch_step_tick(stream, d_step.p, 1);
-      return;
-    }
     const long long rstride = static_cast<long long>(nstacey) * h.npe * h.ncomp;
     launch_sources(stream, 2, h.npe, h.nsrc, 0, src_order.p, src_ispec.p, gather.p, src_array.p, stf.p, ff, d_step.p);
     const bool atomic = run.scatter == SFX_SCATTER_ATOMIC;
@@ -235,26 +227,84 @@ struct sfx_engine {
 
   bool gather_path() const { return h.dim == 3 && run.scatter == SFX_SCATTER_GATHER; }
   bool gather2d() const { return h.dim == 2 && run.scatter == SFX_SCATTER_GATHER; }
-  ForceSum2D fs2() const { return ForceSum2D{inv_off.p, inv_ent.p, re2.p}; }
-  // where the 2-D gather path's element forces take each point's geometry from
+  // 2-D elastic meshes: forward steps run patch by patch
+  bool patches() const {
+    return h.dim == 2 && !h.coupled() && !host_only &&
+           (run.scatter == SFX_SCATTER_GATHER || run.scatter == SFX_SCATTER_COLORED);
+  }
+  PatchTables patch_tables() const {
+    PatchTables t = patch.t;
+    t.src_array = src_array.p;
+    t.stf = stf.p;
+    t.stf_step = h.nsrc;
+    t.stf_src = 1;
+    t.types = types.p;
+    t.ntypes = run.nseismo_types;
+    t.minv = f().minv;
+    t.seismo = seismo.p;
+    t.np = h.nglob_pad;
+    return t;
+  }
+  int npatch() const { return patch.patch_end.back(); }
+  // Steps [first, first + count), one launch each; then the boundary points,
+  // whose last contributions are still open, and the last step's samples.
+  // The gather scatter rounds every product and sum on its own, as the oracle
+  // does, and keeps the last acceleration; the colored one contracts them and
+  // leaves the acceleration zero, where its other kernels accumulate.
+  void patch_steps(int first, int count, hipEvent_t *evs = nullptr) {
+    if (count <= 0) return;
+    const bool exact = gather2d();
+    if (!exact && a_kept) {
+      const size_t stride = static_cast<size_t>(h.ncomp) * h.nglob_pad;
+      launch_fill(stream, fields.p + 2 * stride, stride, 0.0f);
+      a_kept = false;
+    }
+    const Fields ff = f();
+    const PatchTables t = patch_tables();
+    const PatchState st = patch.state(ff.u, ff.v, ff.a);
+    if (evs) SFX_HIP(hipEventRecord(evs[0], stream));
+    if (evs) SFX_HIP(hipEventRecord(evs[1], stream));
+    Throttle throttle(stream);
+    for (int j = 0; j < count; j++) {
+      const bool last = j == count - 1;
+      launch_patch_step(stream, patch.pe, npatch(), h.nrec, exact, t, st, q,
+                        PatchLaunch{nullptr, nullptr, first + j, j & 1, j > 0, 1, exact && last});
+      throttle.tick();
+    }
+    if (evs) SFX_HIP(hipEventRecord(evs[2], stream));
+    const int rd = count & 1;
+    if ((first + count - 1) % run.nstep_between_samples == 0)
+      launch_patch_step(stream, patch.pe, 0, h.nrec, exact, t, st, q, PatchLaunch{nullptr, nullptr, first + count, rd, 1, 1, 0});
+    if (evs) SFX_HIP(hipEventRecord(evs[3], stream));
+    launch_patch_boundary(stream, exact, t, st, nc, rd, 1, exact);
+    if (evs) SFX_HIP(hipEventRecord(evs[4], stream));
+    if (exact) a_kept = true;
+  }
+  // update_wavefields of the forward field: a = M^-1 f of step istep
+  void patch_force(int istep) {
+    const bool exact = gather2d();
+    const Fields ff = f();
+    const PatchTables t = patch_tables();
+    const PatchState st = patch.state(ff.u, ff.v, ff.a);
+    launch_patch_step(stream, patch.pe, npatch(), 0, exact, t, st, q, PatchLaunch{nullptr, nullptr, istep, 0, 0, 0, 0});
+    launch_patch_boundary(stream, exact, t, st, nc, 1, 0, 0);
+    a_kept = true;
+  }
+  const int *device_order() {
+    if (h.lattice_of.empty()) return nullptr;
+    if (!d_lattice.p) {
+      d_lattice.upload(h.lattice_of, stream);
+      stage.alloc(h.lattice_of.size());
+      SFX_HIP(hipStreamSynchronize(stream));
+    }
+    return d_lattice.p;
+  }
+  // where the 2-D gather scatter takes each point's geometry from
   int geom2d_form() const {
     if (h.dim != 2) return GEOM2D_POINT;
     if (!h.geo2d.empty()) return GEOM2D_RECORD;
     if (gather2d() && (h.ngnod2d == 4 || h.ngnod2d == 9)) return h.ngnod2d;
     return GEOM2D_POINT;
-  }
-  Geom2D geom2d() const {
-    Geom2D gm;
-    gm.xix = xix.p;
-    gm.xiz = xiz.p;
-    gm.gammax = gammax.p;
-    gm.gammaz = gammaz.p;
-    gm.jac = jac.p;
-    gm.mode = geom2d_form();
-    gm.record = geo.p;
-    gm.ctrl = ctrl.p;
-    gm.dsh = dsh.p;
-    return gm;
   }
   // (kappa, mu) per element slot for the 2-D and 3-D gather paths when every
   // element holds one value of each at all of its points (bit for bit); empty
@@ -274,6 +324,7 @@ struct sfx_engine {
     return kmu;
   }
   void upload_element_properties(hipStream_t s) {
+    if (!gather_path()) return;
     const std::vector<float> kmu = element_properties();
     if (kmu.empty())
       kmu_e.alloc(0);
@@ -281,63 +332,6 @@ struct sfx_engine {
       kmu_e.upload(kmu, s);
   }
 
-  // 2-D gather path: per field point the re2 offsets of its element
-  // contributions (ascending element slot, then point), and the Stacey entries
-  // sorted by element point, one segment per point
-  void upload_gather_2d(hipStream_t s) {
-    const int npe = h.npe;
-    std::vector<int> off(static_cast<size_t>(h.nglob) + 1, 0);
-    for (int slot = 0; slot < h.nspec; slot++)
-      for (int p = 0; p < npe; p++) off[h.gather[static_cast<size_t>(h.perm[slot]) * npe + p] + 1]++;
-    for (int g = 0; g < h.nglob; g++) off[g + 1] += off[g];
-    std::vector<int> ent(off.back()), fill(off.begin(), off.end() - 1);
-    for (int slot = 0; slot < h.nspec; slot++)
-      for (int p = 0; p < npe; p++) {
-        const int g = h.gather[static_cast<size_t>(h.perm[slot]) * npe + p];
-        ent[fill[g]++] = slot * RE2_ELEM + 2 * p;
-      }
-    inv_off.upload(off, s);
-    inv_ent.upload(ent, s);
-    re2.alloc(static_cast<size_t>(h.nspec) * RE2_ELEM);
-    launch_fill(s, re2.p, re2.n, 0.0f);
-    const size_t nb = h.bnd_gather.size();
-    std::vector<size_t> order(nb);
-    std::iota(order.begin(), order.end(), 0);
-    auto dev_slot = [&](size_t q) {
-      const int c = h.bnd_slot[q] / npe, p = h.bnd_slot[q] - (h.bnd_slot[q] / npe) * npe;
-      return h.inv_perm[c] * npe + p;
-    };
-    std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return dev_slot(a) < dev_slot(b); });
-    std::vector<int> sg, gg(nb), sl(nb);
-    std::vector<float> nrm(2 * nb), wt(nb), rvp(nb), rvs(nb);
-    for (size_t k = 0; k < nb; k++) {
-      const size_t q = order[k];
-      gg[k] = h.bnd_gather[q];
-      sl[k] = dev_slot(q);
-      nrm[2 * k] = h.bnd_normal[2 * q];
-      nrm[2 * k + 1] = h.bnd_normal[2 * q + 1];
-      wt[k] = h.bnd_weight[q];
-      rvp[k] = h.bnd_rho_vp[q];
-      rvs[k] = h.bnd_rho_vs[q];
-      if (k == 0 || sl[k] != sl[k - 1]) sg.push_back(static_cast<int>(k));
-    }
-    sg.push_back(static_cast<int>(nb));
-    g2_nseg = static_cast<int>(sg.size()) - 1;
-    g2_seg.upload(sg, s);
-    g2_gather.upload(gg, s);
-    g2_slot.upload(sl, s);
-    g2_normal.upload(nrm, s);
-    g2_weight.upload(wt, s);
-    g2_rvp.upload(rvp, s);
-    g2_rvs.upload(rvs, s);
-  }
-  // element forces, Stacey and sources into re2 (the step's force, unassembled)
-  void forces_2d(Fields ff, int istep, const int *step) {
-    launch_elemforce_2d(stream, h.nspec, gather.p, geom2d(), kappa.p, mu.p, kmu_e.p, q, ff.u, h.nglob_pad, re2.p);
-    launch_stacey_re2(stream, g2_nseg, g2_seg.p, g2_gather.p, g2_slot.p, g2_normal.p, g2_weight.p, g2_rvp.p, g2_rvs.p,
-                      ff, re2.p);
-    launch_sources_re2(stream, h.nsrc, istep, src_order.p, src_ispec.p, src_array.p, stf.p, re2.p, step);
-  }
   bool block_path() const { return h.dim == 3 && run.scatter == SFX_SCATTER_BLOCK; }
 
   // Stacey entries regrouped for the block path: entry slot = owner * 386 +
@@ -408,10 +402,6 @@ struct sfx_engine {
       gammaz.upload(permuted(h.gammaz), s);
       jac.upload(permuted(h.jac), s);
       if (!h.geo2d.empty()) geo.upload(permuted(h.geo2d, 8), s);
-      if (geom2d_form() == GEOM2D_CTRL4 || geom2d_form() == GEOM2D_CTRL9) {
-        ctrl.upload(permuted(h.ctrl2d, 2 * static_cast<size_t>(h.ngnod2d)), s);
-        dsh.upload(h.dsh2d, s);
-      }
       rho.upload(permuted(h.rho), s);
       // Stacey elements are the last ones in compute order
       nstacey = h.nspec - h.nspec_none;
@@ -424,7 +414,12 @@ struct sfx_engine {
       }
       rec_index.upload(ri, s);
       bnd_rec.upload(br, s);
-      if (gather2d()) upload_gather_2d(s);
+      if (patches()) {
+        const float dt = static_cast<float>(run.dt);
+        const PatchSim sim{dt, static_cast<float>(dt / 2.0), static_cast<float>(dt * dt / 2.0), run.nstep,
+                           run.nstep_between_samples, h.nrec, 0};
+        patch.upload(plan, {&h}, false, {sim}, s);
+      }
     }
     bnd_gather.upload(h.bnd_gather, s);
     bnd_slot.upload(h.bnd_slot, s);
@@ -565,10 +560,6 @@ struct sfx_engine {
       launch_assemble_3d(stream, lat, re_p, f(), 1);
       a_stale = false;
     }
-    if (gather2d() && a_stale) {  // re2 still holds the last step's forces
-      launch_assemble_update_2d(stream, h.nglob, fs2(), f(), nc, 1);
-      a_stale = false;
-    }
   }
 
   // One launch per color (plain read-modify-write), or one atomic launch.
@@ -604,7 +595,7 @@ struct sfx_engine {
     const bool cpl = h.coupled();
     launch_seismograms(stream, h.dim, h.npe, h.nrec, run.nseismo_types, types.p, isig, rec_ispec.p, gather.p, rec_h.p,
                        ff, dto2, corrected, seismo.p, PointGeom2D{xix.p, xiz.p, gammax.p, gammaz.p, kappa.p, mu.p},
-                       q, nullptr, 1, -1, ForceSum2D{}, cpl ? rec_el.p : nullptr,
+                       q, nullptr, 1, -1, cpl ? rec_el.p : nullptr,
                        cpl ? static_cast<int>(h.rec_el.size()) : -1);
     if (cpl)
       launch_acoustic_seismograms(stream, static_cast<int>(h.rec_ac.size()), rec_ac.p, h.nrec, run.nseismo_types,
@@ -666,24 +657,9 @@ struct sfx_engine {
       if (evs) SFX_HIP(hipEventRecord(evs[4], stream));
       return;
     }
-    if (gather2d()) {
+    if (patches() && !recording) {
       if (istep < 0 || istep >= run.nstep) throw std::invalid_argument("istep out of range");
-      if (recording) throw std::invalid_argument("adjoint runs need SFX_SCATTER_COLORED or _ATOMIC");
-      if (evs) SFX_HIP(hipEventRecord(evs[0], stream));
-      if (evs) SFX_HIP(hipEventRecord(evs[1], stream));
-      forces_2d(ff, istep, nullptr);
-      if (evs) SFX_HIP(hipEventRecord(evs[2], stream));
-      if (istep % run.nstep_between_samples == 0) {
-        const int isig = istep / run.nstep_between_samples;
-        if (isig >= nsig) throw std::invalid_argument("seismogram step out of range");
-        launch_seismograms(stream, 2, h.npe, h.nrec, run.nseismo_types, types.p, isig, rec_ispec.p, gather.p,
-                           rec_h.p, ff, nc.dto2, 1, seismo.p,
-                           PointGeom2D{xix.p, xiz.p, gammax.p, gammaz.p, kappa.p, mu.p}, q, nullptr, 1, -1, fs2());
-      }
-      if (evs) SFX_HIP(hipEventRecord(evs[3], stream));
-      launch_assemble_update_2d(stream, h.nglob, fs2(), ff, nc, 0);
-      if (evs) SFX_HIP(hipEventRecord(evs[4], stream));
-      a_stale = true;
+      patch_steps(istep, 1, evs);
       return;
     }
     if (gather_path()) {
@@ -838,11 +814,9 @@ struct sfx_engine {
       element_boundary_sources(ff, istep);
       launch_assemble_3d(stream, lat, re_p, ff, 1);
       a_stale = false;
-    } else if (gather2d()) {
+    } else if (patches()) {
       if (istep < 0 || istep >= run.nstep) throw std::invalid_argument("istep out of range");
-      forces_2d(ff, istep, nullptr);
-      launch_assemble_update_2d(stream, h.nglob, fs2(), ff, nc, 1);
-      a_stale = false;
+      patch_force(istep);
     } else {
       if (h.coupled()) couple_into_elastic(ff);
       sources(ff, istep);
@@ -1048,8 +1022,20 @@ template <class Build> int create(Build &&build, const sfx_run_desc *run, sfx_en
     // the element coloring and the sample count are host data: host-only
     // engines carry them too
     color_elements(e->h, run->scatter);
-    e->nsig = (run->nstep + run->nstep_between_samples - 1) / run->nstep_between_samples;
     e->host_only = host_only;
+    if (e->patches()) {
+      // a point's contributions are summed by element in compute order
+      // (gather) or in color order
+      e->plan.pe = patch_elements(e->h.nspec);
+      std::vector<int32_t> key(e->h.nspec);
+      std::iota(key.begin(), key.end(), 0);
+      const bool colored = run->scatter == SFX_SCATTER_COLORED;
+      add_patches(e->plan, e->h, colored ? e->h.inv_perm : key, colored);
+      finish_patches(e->plan);
+      renumber_points(e->h, e->plan);
+      e->plan.device_of.clear();
+    }
+    e->nsig = (run->nstep + run->nstep_between_samples - 1) / run->nstep_between_samples;
     if (!host_only) e->upload();
     *out = e.release();
   });
@@ -1212,6 +1198,7 @@ int sfx_initialize(sfx_engine *e) {
     if (e->h.coupled()) launch_fill(e->stream, e->ac_fields.p, 3 * static_cast<size_t>(e->h.nglob_ac_pad), 0.0f);
     if (e->seismo.n) launch_fill(e->stream, e->seismo.p, e->seismo.n, 0.0f);
     e->a_stale = false;
+    e->a_kept = false;
     SFX_HIP(hipGetLastError());
     e->initialized = true;
   }, stream_of(e));
@@ -1224,6 +1211,7 @@ int sfx_predictor(sfx_engine *e) {
     e->require_init();
     e->refresh_acceleration();
     launch_predictor(e->stream, e->h.ncomp, e->f(), e->nc, e->gather2d());
+    e->a_kept = false;
     SFX_HIP(hipGetLastError());
     dofs = e->h.nglob_el * e->h.ncomp;
   }, stream_of(e));
@@ -1296,6 +1284,7 @@ int sfx_predictor_phase(sfx_engine *e, int medium, int wavefield, int direction)
     Fields F = e->medium_wavefield(medium, wavefield, ncomp);
     if (wavefield == SFX_WAVEFIELD_FORWARD) e->refresh_acceleration();
     launch_predictor(e->stream, ncomp, F, k, e->gather2d());
+    if (medium == SFX_MEDIUM_ELASTIC_PSV && wavefield == SFX_WAVEFIELD_FORWARD) e->a_kept = false;
     SFX_HIP(hipGetLastError());
   }, stream_of(e));
   return rc == SFX_OK ? dofs : rc;
@@ -1361,7 +1350,7 @@ int sfx_copy_wavefield(sfx_engine *e, int dst, int src) {
     Fields from = e->wavefield(src), to = e->wavefield(dst);
     const size_t n3 = 3 * static_cast<size_t>(e->h.ncomp) * e->h.nglob_pad;
     SFX_HIP(hipMemcpyAsync(to.u, from.u, n3 * sizeof(float), hipMemcpyDeviceToDevice, e->stream));
-    if (dst == SFX_WAVEFIELD_FORWARD) e->a_stale = false;
+    if (dst == SFX_WAVEFIELD_FORWARD) e->a_stale = false, e->a_kept = true;
   }, stream_of(e));
 }
 
@@ -1397,6 +1386,23 @@ int sfx_run(sfx_engine *e, int first, int count) {
     e->require_init();
     if (first < 0 || count < 0 || first + count > e->run.nstep) throw std::invalid_argument("step range out of bounds");
     e->own_forces();
+    if (e->patches() && count > 1) {
+      while (e->ev.size() < 2) {
+        hipEvent_t ev;
+        SFX_HIP(hipEventCreate(&ev));
+        e->ev.push_back(ev);
+      }
+      SFX_HIP(hipEventRecord(e->ev[0], e->stream));
+      e->patch_steps(first, count);
+      SFX_HIP(hipEventRecord(e->ev[1], e->stream));
+      SFX_HIP(hipGetLastError());
+      SFX_HIP(hipStreamSynchronize(e->stream));
+      float all = 0.0f;
+      SFX_HIP(hipEventElapsedTime(&all, e->ev[0], e->ev[1]));
+      e->timings[0] = e->timings[1] = e->timings[2] = 0.0;
+      e->timings[3] = all / count;
+      return;
+    }
     if (e->graph_2d() && count > 1) {
       // 2-D: one captured graph per step; only the whole-step time is taken
       e->set_step(first);
@@ -1413,7 +1419,6 @@ int sfx_run(sfx_engine *e, int first, int count) {
         throttle.tick();
       }
       SFX_HIP(hipEventRecord(e->ev[1], e->stream));
-      if (e->gather2d()) e->a_stale = true;
       SFX_HIP(hipStreamSynchronize(e->stream));
       float all = 0.0f;
       SFX_HIP(hipEventElapsedTime(&all, e->ev[0], e->ev[1]));
@@ -1519,17 +1524,15 @@ int sfx_get_wavefield(const sfx_engine *ce, int wavefield, int which, float *out
     if (wavefield == SFX_WAVEFIELD_FORWARD && which == 2) e->refresh_acceleration();
     Fields F = e->wavefield(wavefield);
     const float *arrays[4] = {F.u, F.v, F.a, F.minv};
-    SFX_HIP(hipStreamSynchronize(e->stream));
-    const size_t ng = e->h.nglob_el;
-    std::vector<float> buf(e->h.nglob_pad);
+    // the device permutes to the reference's point order; one copy per component
+    const int ng = e->h.nglob_el;
+    const int *order = e->device_order();
     for (int c = 0; c < e->h.ncomp; c++) {
-      SFX_HIP(hipMemcpy(buf.data(), arrays[which] + static_cast<size_t>(c) * e->h.nglob_pad,
-                        e->h.nglob_pad * sizeof(float), hipMemcpyDeviceToHost));
-      float *o = out + static_cast<size_t>(c) * ng;
-      if (e->h.lattice_of.empty())
-        std::memcpy(o, buf.data(), ng * sizeof(float));
-      else
-        for (size_t g = 0; g < ng; g++) o[g] = buf[e->h.lattice_of[g]];
+      const float *src = arrays[which] + static_cast<size_t>(c) * e->h.nglob_pad;
+      if (order) launch_take(e->stream, ng, order, src, e->stage.p);
+      SFX_HIP(hipStreamSynchronize(e->stream));
+      SFX_HIP(hipMemcpy(out + static_cast<size_t>(c) * ng, order ? e->stage.p : src, ng * sizeof(float),
+                        hipMemcpyDeviceToHost));
     }
   }, stream_of(ce));
 }
@@ -1545,19 +1548,17 @@ int sfx_set_wavefield(sfx_engine *e, int wavefield, int which, const float *in) 
     if (!in) throw std::invalid_argument("null input");
     Fields F = e->wavefield(wavefield);
     float *arrays[3] = {F.u, F.v, F.a};
-    SFX_HIP(hipStreamSynchronize(e->stream));
-    const size_t ng = e->h.nglob_el;
-    std::vector<float> buf(e->h.nglob_pad, 0.0f);
+    const int ng = e->h.nglob_el;
+    const int *order = e->device_order();
     for (int c = 0; c < e->h.ncomp; c++) {
-      const float *src = in + static_cast<size_t>(c) * ng;
-      if (e->h.lattice_of.empty())
-        std::memcpy(buf.data(), src, ng * sizeof(float));
-      else
-        for (size_t g = 0; g < ng; g++) buf[e->h.lattice_of[g]] = src[g];
-      SFX_HIP(hipMemcpy(arrays[which] + static_cast<size_t>(c) * e->h.nglob_pad, buf.data(),
-                        e->h.nglob_pad * sizeof(float), hipMemcpyHostToDevice));
+      float *dst = arrays[which] + static_cast<size_t>(c) * e->h.nglob_pad;
+      SFX_HIP(hipStreamSynchronize(e->stream));
+      SFX_HIP(hipMemcpy(order ? e->stage.p : dst, in + static_cast<size_t>(c) * ng, ng * sizeof(float),
+                        hipMemcpyHostToDevice));
+      if (order) launch_put(e->stream, ng, order, e->stage.p, dst);
     }
-    if (wavefield == SFX_WAVEFIELD_FORWARD && which == 2) e->a_stale = false;
+    SFX_HIP(hipStreamSynchronize(e->stream));
+    if (wavefield == SFX_WAVEFIELD_FORWARD && which == 2) e->a_stale = false, e->a_kept = true;
   }, stream_of(e));
 }
 
@@ -1610,7 +1611,7 @@ int sfx_set_properties(sfx_engine *e, const float *rho, const float *kappa, cons
     const size_t stride = static_cast<size_t>(e->h.ncomp) * e->h.nglob_pad;
     SFX_HIP(hipMemcpyAsync(e->fields.p + 3 * stride, e->h.mass_inverse.data(), stride * sizeof(float),
                            hipMemcpyHostToDevice, s));
-    if (e->gather2d()) e->upload_gather_2d(s);  // the sorted Stacey entries carry the impedances
+    if (e->patches()) e->patch.upload_properties(e->plan, {&e->h}, s);
     SFX_HIP(hipStreamSynchronize(s));
     e->recorded = false;
     e->invalidate_graphs();

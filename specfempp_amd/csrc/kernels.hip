@@ -156,307 +156,6 @@ __global__ __launch_bounds__(threads_for(E)) void stiffness_2d_kernel(
   for (int c = 0; c < 2; c++) scatter_add<ATOMIC>(&f.a[c * f.nglob_pad + g], r[c]);
 }
 
-// ---------------------------------------------------------------------------
-// 2-D gather path (forward runs): the element forces of 5 elements per
-// workgroup are staged in LDS and stored with coalesced 16-byte writes
-// (RE2_ELEM floats per element); Stacey tractions and sources are added to
-// them; one update per field point then sums its contributions in a fixed
-// order (ascending element, then point) and applies the Newmark update, with
-// no scattered read-modify-write of the acceleration.
-// ---------------------------------------------------------------------------
-// Geometry of local point p (index idx) of element e from the source GEOM
-// names.  The control-node forms sum the shape derivatives times the nodes in
-// node order, then form J and the four quotients exactly as the host does.
-template <int GEOM>
-__device__ __forceinline__ void point_geometry_2d(const Geom2D &gm, int e, int p, size_t idx, float &xix,
-                                                  float &xiz, float &gammax, float &gammaz, float &J) {
-#pragma clang fp contract(off)
-  if constexpr (GEOM == GEOM2D_POINT) {
-    xix = gm.xix[idx];
-    xiz = gm.xiz[idx];
-    gammax = gm.gammax[idx];
-    gammaz = gm.gammaz[idx];
-    J = gm.jac[idx];
-  } else if constexpr (GEOM == GEOM2D_RECORD) {
-    const float *ge = gm.record + static_cast<size_t>(e) * 8;
-    xix = ge[0];
-    xiz = ge[1];
-    gammax = ge[2];
-    gammaz = ge[3];
-    J = ge[4];
-  } else {
-    constexpr int NG = GEOM;
-    const float *c = gm.ctrl + static_cast<size_t>(e) * (2 * NG);
-    const float *d = gm.dsh + p * (2 * NG);
-    float xxi = 0.0f, zxi = 0.0f, xgamma = 0.0f, zgamma = 0.0f;
-#pragma unroll
-    for (int n = 0; n < NG; n++) {
-      const float cx = c[2 * n], cz = c[2 * n + 1];
-      xxi += d[n] * cx;
-      zxi += d[n] * cz;
-      xgamma += d[NG + n] * cx;
-      zgamma += d[NG + n] * cz;
-    }
-    J = xxi * zgamma - xgamma * zxi;
-    xix = zgamma / J;
-    gammax = -zxi / J;
-    xiz = -xgamma / J;
-    gammaz = xxi / J;
-  }
-}
-
-// A workgroup of 128 threads computes G groups of E2 elements: thread t holds
-// local point t % 25 of element t / 25 of every group, and the loads of all
-// groups are issued before the first is used, so a wave keeps G times the
-// bytes in flight (the kernel is bound by the latency of its two dependent
-// loads, the gather index and the displacement it names).
-template <int GEOM, bool EPROP, int G>
-__global__ __launch_bounds__(128) void elemforce_2d_kernel(int nspec, const int *__restrict__ gather, Geom2D gm,
-                                                           const float *__restrict__ kappa_,
-                                                           const float *__restrict__ mu_,
-                                                           const float *__restrict__ kmu, GllConst q,
-                                                           const float *__restrict__ uf, int np,
-                                                           float *__restrict__ re2) {
-  // every product and sum rounded on its own: the one-launch batch step
-  // performs the same operations and must round them the same way
-#pragma clang fp contract(off)
-  constexpr int NE = G * E2;  // elements per workgroup
-  __shared__ float su[NE][2][25];
-  __shared__ float sF[NE][4][25];  // F(c, d) as [2c + d]
-  __shared__ __align__(16) float st[NE * RE2_ELEM];
-
-  const int t = threadIdx.x;
-  const int el = t / 25;
-  const int p = t - el * 25;
-  const int iz = p / 5, ix = p - (p / 5) * 5;
-  const int first = blockIdx.x * NE;
-  // Loads are issued for every lane, inactive ones re-reading the last
-  // element (all addresses stay in bounds): with no branch around them the
-  // loads of all groups are in flight together instead of one after another.
-  int e[G];
-  bool active[G];
-  size_t idx[G];
-#pragma unroll
-  for (int g = 0; g < G; g++) {
-    const int eg = first + g * E2 + el;
-    active[g] = (el < E2) && (eg < nspec);
-    e[g] = eg < nspec ? eg : nspec - 1;
-    idx[g] = static_cast<size_t>(e[g]) * 25 + p;
-  }
-
-  // the gather indices, then the displacement they name, of every group
-  int gi[G];
-#pragma unroll
-  for (int g = 0; g < G; g++) gi[g] = gather[idx[g]];
-  float ux[G], uz[G];
-#pragma unroll
-  for (int g = 0; g < G; g++) {
-    ux[g] = uf[gi[g]];
-    uz[g] = uf[np + gi[g]];
-  }
-  float kappa[G], mu[G], xix[G], xiz[G], gammax[G], gammaz[G], J[G];
-#pragma unroll
-  for (int g = 0; g < G; g++) {
-    if constexpr (EPROP) {
-      kappa[g] = kmu[2 * static_cast<size_t>(e[g])];
-      mu[g] = kmu[2 * static_cast<size_t>(e[g]) + 1];
-    } else {
-      kappa[g] = kappa_[idx[g]];
-      mu[g] = mu_[idx[g]];
-    }
-    point_geometry_2d<GEOM>(gm, e[g], p, idx[g], xix[g], xiz[g], gammax[g], gammaz[g], J[g]);
-  }
-  // the derivative rows of this point (lane-indexed, so vector loads; before
-  // the barrier, where their latency overlaps the loads above)
-  float hpx[5], hpz[5], hwx[5], hwz[5];
-#pragma unroll
-  for (int l = 0; l < 5; l++) {
-    hpx[l] = q.hp[ix][l];
-    hpz[l] = q.hp[iz][l];
-    hwx[l] = q.hpw[ix][l];
-    hwz[l] = q.hpw[iz][l];
-  }
-  const float wx = q.w[ix], wz = q.w[iz];
-#pragma unroll
-  for (int g = 0; g < G; g++)
-    if (active[g]) {
-      su[g * E2 + el][0][p] = ux[g];
-      su[g * E2 + el][1][p] = uz[g];
-    }
-  __syncthreads();
-#pragma unroll
-  for (int g = 0; g < G; g++) {
-    if (!active[g]) continue;
-    const int le = g * E2 + el;
-    // the gradient, stress and stress integrand of stiffness_2d_kernel
-    float dxi[2] = {0.0f, 0.0f}, dga[2] = {0.0f, 0.0f};
-#pragma unroll
-    for (int l = 0; l < 5; l++) {
-#pragma unroll
-      for (int c = 0; c < 2; c++) {
-        dxi[c] += hpx[l] * su[le][c][iz * 5 + l];
-        dga[c] += hpz[l] * su[le][c][l * 5 + ix];
-      }
-    }
-    float du[2][2];
-#pragma unroll
-    for (int c = 0; c < 2; c++) {
-      du[c][0] = xix[g] * dxi[c] + gammax[g] * dga[c];
-      du[c][1] = xiz[g] * dxi[c] + gammaz[g] * dga[c];
-    }
-    const float lp2m = kappa[g] + (4.0f / 3.0f) * mu[g];
-    const float lambda = lp2m - 2.0f * mu[g];
-    const float sxx = lp2m * du[0][0] + lambda * du[1][1];
-    const float szz = lp2m * du[1][1] + lambda * du[0][0];
-    const float sxz = mu[g] * (du[0][1] + du[1][0]);
-    sF[le][0][p] = J[g] * (sxx * xix[g] + sxz * xiz[g]);
-    sF[le][1][p] = J[g] * (sxx * gammax[g] + sxz * gammaz[g]);
-    sF[le][2][p] = J[g] * (sxz * xix[g] + szz * xiz[g]);
-    sF[le][3][p] = J[g] * (sxz * gammax[g] + szz * gammaz[g]);
-  }
-  __syncthreads();
-#pragma unroll
-  for (int g = 0; g < G; g++) {
-    if (!active[g]) continue;
-    const int le = g * E2 + el;
-    float t1[2] = {0.0f, 0.0f}, t2[2] = {0.0f, 0.0f};
-#pragma unroll
-    for (int l = 0; l < 5; l++) {
-#pragma unroll
-      for (int c = 0; c < 2; c++) {
-        t1[c] += sF[le][2 * c][iz * 5 + l] * hwx[l];
-        t2[c] += sF[le][2 * c + 1][l * 5 + ix] * hwz[l];
-      }
-    }
-#pragma unroll
-    for (int c = 0; c < 2; c++) st[le * RE2_ELEM + 2 * p + c] = -(wz * t1[c] + wx * t2[c]);
-  }
-  __syncthreads();
-  const int nel = nspec - first < NE ? nspec - first : NE;
-  float4 *dst = reinterpret_cast<float4 *>(re2 + static_cast<size_t>(first) * RE2_ELEM);
-  const float4 *from = reinterpret_cast<const float4 *>(st);
-  for (int qv = t; qv < nel * (RE2_ELEM / 4); qv += 128) dst[qv] = from[qv];
-}
-
-// One thread per element point on the absorbing boundary (entries sorted by
-// element point); its edge entries (two at a corner) are summed in order and
-// added to the point's element force once.
-__global__ __launch_bounds__(256) void stacey_re2_kernel(int nseg, const int *__restrict__ seg,
-                                                         const int *__restrict__ gather, const int *__restrict__ slot,
-                                                         const float *__restrict__ normal,
-                                                         const float *__restrict__ weight,
-                                                         const float *__restrict__ rho_vp,
-                                                         const float *__restrict__ rho_vs, Fields f,
-                                                         float *__restrict__ re2) {
-#pragma clang fp contract(off)
-  const int sidx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (sidx >= nseg) return;
-  const int q0 = seg[sidx], q1 = seg[sidx + 1];
-  const int g = gather[q0];
-  const int sl = slot[q0];
-  const int e = sl / 25, p = sl - (sl / 25) * 25;
-  const int np = f.nglob_pad;
-  const float v[2] = {f.v[g], f.v[np + g]};
-  float sum[2] = {0.0f, 0.0f};
-  for (int qq = q0; qq < q1; qq++) {
-    const float n[2] = {normal[2 * qq], normal[2 * qq + 1]};
-    const float vn = v[0] * n[0] + v[1] * n[1];
-    const float nn = n[0] * n[0] + n[1] * n[1];
-    const float j1 = sqrtf(nn);
-    const float w = weight[qq], rvp = rho_vp[qq], rvs = rho_vs[qq];
-#pragma unroll
-    for (int d = 0; d < 2; d++) {
-      const float fac = ((vn * n[d] / (j1 * j1)) * (rvp - rvs)) + v[d] * rvs;
-      sum[d] += -1.0f * fac * j1 * w;
-    }
-  }
-  float *o = re2 + static_cast<size_t>(e) * RE2_ELEM + 2 * p;
-  o[0] += sum[0];
-  o[1] += sum[1];
-}
-
-// Sources in application order, one thread per element point.
-__global__ __launch_bounds__(64) void sources_re2_kernel(int nsrc, int istep_arg, const int *__restrict__ order,
-                                                         const int *__restrict__ ispec,
-                                                         const float *__restrict__ array,
-                                                         const float *__restrict__ stf, float *__restrict__ re2,
-                                                         const int *__restrict__ step) {
-#pragma clang fp contract(off)
-  const int p = threadIdx.x;
-  if (p >= 25) return;
-  const int istep = step ? *step : istep_arg;
-  for (int k = 0; k < nsrc; k++) {
-    const int s = order[k];
-    const float sv = stf[static_cast<size_t>(istep) * nsrc + s];
-    float *o = re2 + static_cast<size_t>(ispec[s]) * RE2_ELEM + 2 * p;
-#pragma unroll
-    for (int c = 0; c < 2; c++) o[c] += sv * array[(static_cast<size_t>(s) * 2 + c) * 25 + p];
-  }
-}
-
-// One thread per field point: the assembled force (its element contributions
-// in a fixed order), a = M^-1 f; divide_only stores a, otherwise corrector and
-// predictor follow: v += dt/2 a; u += dt v + dt^2/2 a; v += dt/2 a, and a is
-// not stored (nothing in the fused loop reads it; the engine recomputes it
-// from re2 with divide_only when a caller asks for it).
-// The first AU2_BATCH contributions of a point are loaded together (entry
-// indices clamped to the point's last one, so every address is valid) and
-// summed in ascending order, then any further ones one by one: the same sum
-// as a plain loop, with two dependent round trips instead of one per entry.
-// M^-1, u and v do not depend on the sum and are loaded first.
-constexpr int AU2_BATCH = 4;
-
-__global__ __launch_bounds__(256) void assemble_update_2d_kernel(int nglob, ForceSum2D fs, Fields f,
-                                                                 NewmarkConst nc, int divide_only) {
-#pragma clang fp contract(off)
-  const int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= nglob) return;
-  const int np = f.nglob_pad;
-  float minv[2], u[2] = {0.0f, 0.0f}, v[2] = {0.0f, 0.0f};
-#pragma unroll
-  for (int c = 0; c < 2; c++) {
-    const size_t o = static_cast<size_t>(c) * np + g;
-    minv[c] = f.minv[o];
-    if (!divide_only) {
-      u[c] = f.u[o];
-      v[c] = f.v[o];
-    }
-  }
-  const int k0 = fs.off[g], k1 = fs.off[g + 1];
-  float sum[2] = {0.0f, 0.0f};
-  if (k1 > k0) {
-    int en[AU2_BATCH];
-#pragma unroll
-    for (int j = 0; j < AU2_BATCH; j++) en[j] = fs.ent[k0 + j < k1 ? k0 + j : k1 - 1];
-    float2 r[AU2_BATCH];
-#pragma unroll
-    for (int j = 0; j < AU2_BATCH; j++) r[j] = *reinterpret_cast<const float2 *>(fs.re2 + en[j]);
-#pragma unroll
-    for (int j = 0; j < AU2_BATCH; j++)
-      if (k0 + j < k1) {
-        sum[0] += r[j].x;
-        sum[1] += r[j].y;
-      }
-    for (int k = k0 + AU2_BATCH; k < k1; k++) {
-      const float2 rr = *reinterpret_cast<const float2 *>(fs.re2 + fs.ent[k]);
-      sum[0] += rr.x;
-      sum[1] += rr.y;
-    }
-  }
-#pragma unroll
-  for (int c = 0; c < 2; c++) {
-    const size_t o = static_cast<size_t>(c) * np + g;
-    const float a = sum[c] * minv[c];
-    if (divide_only) {
-      f.a[o] = a;
-      continue;
-    }
-    const float v1 = v[c] + nc.dto2 * a;
-    f.u[o] = u[c] + (nc.dt * v1 + nc.dt2o2 * a);
-    f.v[o] = v1 + nc.dto2 * a;
-  }
-}
-
 // Adjoint and backward fields together (the combined loop's two
 // update_wavefields calls, time_marching.tpp:160-186): one pass over the
 // elements loads the geometry and properties once and computes both fields'
@@ -967,7 +666,7 @@ __global__ __launch_bounds__(128) void seismogram_kernel(int npe, int nrec, int 
                                                          Fields f, float dto2, int corrected,
                                                          float *__restrict__ seismo, PointGeom2D pg, GllConst q,
                                                          const int *__restrict__ step, int nsb, int sig_top,
-                                                         ForceSum2D fs, const int *__restrict__ rec_list) {
+                                                         const int *__restrict__ rec_list) {
   __shared__ float red[2][D][64];
   __shared__ float su[2][25];
   if (step) {  // sample only on steps istep % nsb == 0 (the same for the whole block)
@@ -1004,19 +703,11 @@ __global__ __launch_bounds__(128) void seismogram_kernel(int npe, int nrec, int 
         if (type == 0) {
           x = f.u[c * np + g];
         } else {
-          float acc;
-          if (D == 2 && fs.re2) {  // gather path: the assembled force, summed as the update sums it
-            acc = 0.0f;
-            for (int k = fs.off[g]; k < fs.off[g + 1]; k++) acc += fs.re2[fs.ent[k] + c];
-          } else {
-            acc = f.a[c * np + g];
-          }
+          float acc = f.a[c * np + g];
           if (corrected) acc = acc * f.minv[c * np + g];
           if (type == 1) {
             x = f.v[c * np + g];
-            // the gather path rounds v + dt/2 a as its update does (no fused
-            // multiply-add)
-            if (corrected) x = fs.re2 ? plus_product_rounded(x, dto2, acc) : x + dto2 * acc;
+            if (corrected) x = x + dto2 * acc;
           } else {
             x = acc;
           }
@@ -1720,7 +1411,7 @@ void launch_sources(hipStream_t s, int dim, int npe, int nsrc, int istep, const 
 void launch_seismograms(hipStream_t s, int dim, int npe, int nrec, int ntypes, const int *types, int isig,
                         const int *ispec, const int *gather, const float *h, Fields f, float dto2, int corrected,
                         float *seismo, const PointGeom2D &pg, const GllConst &q, const int *step, int nsb,
-                        int sig_top, ForceSum2D fs, const int *rec_list, int nlist) {
+                        int sig_top, const int *rec_list, int nlist) {
   // nlist >= 0: the receivers rec_list[0..nlist) only (an empty list launches
   // nothing, whatever rec_list holds); -1: every receiver
   if (nlist > 0 && !rec_list) throw std::invalid_argument("receiver list missing");
@@ -1728,68 +1419,10 @@ void launch_seismograms(hipStream_t s, int dim, int npe, int nrec, int ntypes, c
   if (nb <= 0 || ntypes <= 0) return;
   if (dim == 2)
     hipLaunchKernelGGL(seismogram_kernel<2>, dim3(nb), dim3(128), 0, s, npe, nrec, ntypes, types, isig, ispec,
-                       gather, h, f, dto2, corrected, seismo, pg, q, step, nsb, sig_top, fs, rec_list);
+                       gather, h, f, dto2, corrected, seismo, pg, q, step, nsb, sig_top, rec_list);
   else
     hipLaunchKernelGGL(seismogram_kernel<3>, dim3(nb), dim3(128), 0, s, npe, nrec, ntypes, types, isig, ispec,
-                       gather, h, f, dto2, corrected, seismo, pg, q, step, nsb, sig_top, ForceSum2D{}, rec_list);
-}
-
-// element groups per workgroup of elemforce_2d
-constexpr int EF2_GROUPS = 2;
-
-template <int GEOM>
-static void launch_elemforce_2d_geom(hipStream_t s, int nspec, const int *gather, const Geom2D &gm,
-                                     const float *kappa, const float *mu, const float *kmu, const GllConst &q,
-                                     const float *u, int nglob_pad, float *re2) {
-  const dim3 grid(blocks(nspec, EF2_GROUPS * E2));
-  if (kmu)
-    hipLaunchKernelGGL((elemforce_2d_kernel<GEOM, true, EF2_GROUPS>), grid, dim3(128), 0, s, nspec, gather, gm, kappa,
-                       mu, kmu, q, u, nglob_pad, re2);
-  else
-    hipLaunchKernelGGL((elemforce_2d_kernel<GEOM, false, EF2_GROUPS>), grid, dim3(128), 0, s, nspec, gather, gm,
-                       kappa, mu, kmu, q, u, nglob_pad, re2);
-}
-
-void launch_elemforce_2d(hipStream_t s, int nspec, const int *gather, const Geom2D &gm, const float *kappa,
-                         const float *mu, const float *kmu, const GllConst &q, const float *u, int nglob_pad,
-                         float *re2) {
-  if (nspec <= 0) return;
-  switch (gm.mode) {
-    case GEOM2D_POINT:
-      launch_elemforce_2d_geom<GEOM2D_POINT>(s, nspec, gather, gm, kappa, mu, kmu, q, u, nglob_pad, re2);
-      break;
-    case GEOM2D_RECORD:
-      launch_elemforce_2d_geom<GEOM2D_RECORD>(s, nspec, gather, gm, kappa, mu, kmu, q, u, nglob_pad, re2);
-      break;
-    case GEOM2D_CTRL4:
-      launch_elemforce_2d_geom<GEOM2D_CTRL4>(s, nspec, gather, gm, kappa, mu, kmu, q, u, nglob_pad, re2);
-      break;
-    case GEOM2D_CTRL9:
-      launch_elemforce_2d_geom<GEOM2D_CTRL9>(s, nspec, gather, gm, kappa, mu, kmu, q, u, nglob_pad, re2);
-      break;
-    default:
-      throw std::invalid_argument("elemforce_2d: unknown geometry form");
-  }
-}
-
-void launch_stacey_re2(hipStream_t s, int nseg, const int *seg, const int *gather, const int *slot,
-                       const float *normal, const float *weight, const float *rho_vp, const float *rho_vs, Fields f,
-                       float *re2) {
-  if (nseg <= 0) return;
-  hipLaunchKernelGGL(stacey_re2_kernel, dim3(blocks(nseg, 256)), dim3(256), 0, s, nseg, seg, gather, slot, normal,
-                     weight, rho_vp, rho_vs, f, re2);
-}
-
-void launch_sources_re2(hipStream_t s, int nsrc, int istep, const int *order, const int *ispec, const float *array,
-                        const float *stf, float *re2, const int *step) {
-  if (nsrc <= 0) return;
-  hipLaunchKernelGGL(sources_re2_kernel, dim3(1), dim3(64), 0, s, nsrc, istep, order, ispec, array, stf, re2, step);
-}
-
-void launch_assemble_update_2d(hipStream_t s, int nglob, ForceSum2D fs, Fields f, NewmarkConst nc, int divide_only) {
-  if (nglob <= 0) return;
-  hipLaunchKernelGGL(assemble_update_2d_kernel, dim3(blocks(nglob, 256)), dim3(256), 0, s, nglob, fs, f, nc,
-                     divide_only);
+                       gather, h, f, dto2, corrected, seismo, pg, q, step, nsb, sig_top, rec_list);
 }
 
 void launch_update_fused(hipStream_t s, int ncomp, Fields f, NewmarkConst nc) {

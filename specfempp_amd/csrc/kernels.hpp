@@ -28,13 +28,6 @@ struct Gll3 {
 };
 Gll3 scaled_gll3(const GllConst &q, float xix, float ety, float gaz, float jac);
 
-// x + s * y with the product rounded before the sum (never one fused
-// multiply-add, whatever contraction the caller's code allows).
-__device__ __forceinline__ float plus_product_rounded(float x, float s, float y) {
-#pragma clang fp contract(off)
-  return x + s * y;
-}
-
 struct Fields {
   float *u, *v, *a;
   const float *minv;
@@ -183,25 +176,16 @@ struct PointGeom2D {
 // corrected = 1: sample the state after the (not yet applied) mass division and
 // corrector of this step, i.e. u, v + dt/2 a M^-1, a M^-1.  Types 0..2
 // displacement, velocity, acceleration; 3 pressure (2-D).
-// 2-D gather path: element forces re2 (RE2_ELEM floats per element, point p
-// component c at 2 p + c) and, per field point g, the re2 offsets of its
-// element contributions in [off[g], off[g + 1]) of ent (summed in that order).
-constexpr int RE2_ELEM = 52;
-struct ForceSum2D {
-  const int *off = nullptr, *ent = nullptr;
-  const float *re2 = nullptr;
-};
-
 void launch_seismograms(hipStream_t s, int dim, int npe, int nrec, int ntypes, const int *types, int isig,
                         const int *ispec, const int *gather, const float *h, Fields f, float dto2, int corrected,
                         float *seismo, const PointGeom2D &pg, const GllConst &q, const int *step = nullptr,
-                        int nsb = 1, int sig_top = -1, ForceSum2D fs = ForceSum2D{}, const int *rec_list = nullptr,
+                        int nsb = 1, int sig_top = -1, const int *rec_list = nullptr,
                         int nlist = -1);
-// Where elemforce_2d takes an element point's geometry from.  Every form gives
-// the same bits: the control-node forms repeat the host's float operations in
-// the host's order (compute_partial_derivatives.cpp:46-91, no fused
-// multiply-add, correctly rounded division), so they trade 20 bytes per point
-// for 8 or 18 floats per element.
+// Where the 2-D patches take an element point's geometry from.  Every form
+// gives the same bits: the control-node forms repeat the host's float
+// operations in the host's order (compute_partial_derivatives.cpp:46-91, no
+// fused multiply-add, correctly rounded division), so they trade 20 bytes per
+// point for 8 or 18 floats per element.
 enum Geom2DMode : int { GEOM2D_POINT = 0, GEOM2D_RECORD = 1, GEOM2D_CTRL4 = 4, GEOM2D_CTRL9 = 9 };
 struct Geom2D {
   int mode = GEOM2D_POINT;
@@ -210,16 +194,6 @@ struct Geom2D {
   const float *ctrl = nullptr;    // per element: its ngnod control nodes (x, z)
   const float *dsh = nullptr;     // (25, 2, ngnod): shape derivatives in xi, then gamma, at each GLL point
 };
-// kappa and mu per local point, or (kmu given) one (kappa, mu) pair per element
-void launch_elemforce_2d(hipStream_t s, int nspec, const int *gather, const Geom2D &gm, const float *kappa,
-                         const float *mu, const float *kmu, const GllConst &q, const float *u, int nglob_pad,
-                         float *re2);
-void launch_stacey_re2(hipStream_t s, int nseg, const int *seg, const int *gather, const int *slot,
-                       const float *normal, const float *weight, const float *rho_vp, const float *rho_vs, Fields f,
-                       float *re2);
-void launch_sources_re2(hipStream_t s, int nsrc, int istep, const int *order, const int *ispec, const float *array,
-                        const float *stf, float *re2, const int *step = nullptr);
-void launch_assemble_update_2d(hipStream_t s, int nglob, ForceSum2D fs, Fields f, NewmarkConst nc, int divide_only);
 void launch_update_fused(hipStream_t s, int ncomp, Fields f, NewmarkConst nc);
 // rounded: every product and sum rounded on its own (no fused multiply-add),
 // as the 2-D gather path's fused update rounds them; its seams pass true.

@@ -276,7 +276,8 @@ class _EngineBase:
         "control_nodes_4" / "control_nodes_9" (recomputed per point from the
         element's control nodes, the same bits as the per-point arrays),
         ``element_properties`` (kappa and mu read once per element),
-        ``scatter`` and ``row_order`` (points in coordinate row order)."""
+        ``scatter`` and ``row_order`` (points ordered by their place in the
+        mesh)."""
         out = (C.c_int64 * 4)()
         self._check(self.lib.sfx_get_layout(self.h, out))
         geom = {0: "point", 1: "element", 4: "control_nodes_4", 9: "control_nodes_9"}[int(out[0])]

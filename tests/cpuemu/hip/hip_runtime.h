@@ -29,7 +29,10 @@
 struct float4 { float x, y, z, w; };
 struct float2 { float x, y; };
 inline float4 make_float4(float a, float b, float c, float d) { return float4{a, b, c, d}; }
+inline float2 make_float2(float a, float b) { return float2{a, b}; }
 struct int4 { int x, y, z, w; };
+inline int4 make_int4(int a, int b, int c, int d) { return int4{a, b, c, d}; }
+struct uint4 { unsigned x, y, z, w; };
 
 struct dim3 {
   unsigned x = 1, y = 1, z = 1;
@@ -57,6 +60,14 @@ inline float __shfl_down(float v, int off, int width = 64) {
   emu::sync();
   return r;
 }
+inline float __shfl(float v, int lane, int width = 64) {
+  const unsigned t = threadIdx.x;
+  emu::shfl_buf[t] = v;
+  emu::sync();
+  const float r = emu::shfl_buf[t / width * width + lane];
+  emu::sync();
+  return r;
+}
 inline float unsafeAtomicAdd(float *p, float v) {
   std::lock_guard<std::mutex> g(emu::atom_mu);
   const float old = *p;
@@ -64,6 +75,8 @@ inline float unsafeAtomicAdd(float *p, float v) {
   return old;
 }
 inline float atomicAdd(float *p, float v) { return unsafeAtomicAdd(p, v); }
+#define __builtin_amdgcn_sched_barrier(m) ((void)0)
+inline float __builtin_amdgcn_rcpf(float x) { return 1.0f / x; }
 inline float sqrtf_(float x) { return std::sqrt(x); }
 
 typedef int hipError_t;
