@@ -1643,6 +1643,9 @@ HostAssembly build_assembly_3d_db(const sfx_mesh3d_db &m, int nsrc, const sfx_so
     if (e < 0 || e >= nspec) throw std::invalid_argument("irregular element number out of range");
     irregular[e] = 1;
   }
+  a.irregular3 = irregular;
+  a.geo3_regular[0] = m.xix_regular;
+  a.geo3_regular[1] = m.jacobian_regular;
   a.geo3.assign(nloc * 10, 0.0f);
   const float *d9[9] = {m.xix, m.xiy, m.xiz, m.etax, m.etay, m.etaz, m.gammax, m.gammay, m.gammaz};
   for (int e = 0; e < nspec; e++)

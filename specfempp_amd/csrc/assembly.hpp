@@ -49,6 +49,8 @@ struct HostAssembly {
   // (nspec, 10, 125)
   bool general3d = false;
   std::vector<float> geo3;
+  std::vector<char> irregular3;           // (nspec) the element has its own geometry in geo3
+  float geo3_regular[2] = {0, 0};         // xix and jacobian of the others
   // properties per local point (kappa, mu; rho for mass and Stacey)
   std::vector<float> kappa, mu, rho;
   // Stacey entries: one per (element, local point) on an absorbing edge/face

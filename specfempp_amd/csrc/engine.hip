@@ -78,7 +78,14 @@ struct sfx_engine {
   DevBuf<int> gather, bnd_gather, bnd_slot, bnd_seg, src_order, src_ispec, rec_ispec, types;
   DevBuf<float> xix, xiz, gammax, gammaz, jac, kappa, mu;
   DevBuf<float> geo;     // 2-D affine meshes: one geometry record per element (the forward stiffness reads it)
-  DevBuf<float> geo3;    // 3-D database meshes: per-point derivatives and jacobian (nspec, 10, 125)
+  // 3-D database meshes: per-point derivatives and jacobian of the irregular
+  // elements (., 10, 125), each element's row of them or -1; colored scatter:
+  // the contributions (elements, sources, Stacey entries) and every point's
+  // list of them
+  DevBuf<float> geo3, re3;
+  DevBuf<int> geo_of, off3;
+  DevBuf<uint32_t> ent3;
+  std::vector<int32_t> key3;  // color order of the elements
   // 2-D elastic engines (COLORED and GATHER): the patches that carry the
   // forward steps
   PatchPlan plan;
@@ -129,7 +136,7 @@ struct sfx_engine {
   float *rec_step = nullptr;
   bool initialized = false;
   bool a_stale = false;  // fused 3-D gather steps leave the stored acceleration behind
-  bool a_kept = false;   // 2-D patches: the stored acceleration may be nonzero (the colored kernels add to it)
+  bool a_kept = false;   // 2-D patches, 3-D database: the stored acceleration may be nonzero
   int nbseg = 0;         // Stacey segments (3-D)
   bool sources_off_boundary = false;  // 3-D gather: no source element has an absorbing face
   DevBuf<float> minv1;                // 3-D gather: M^-1 of one component (nglob_pad)
@@ -310,7 +317,7 @@ struct sfx_engine {
   // element holds one value of each at all of its points (bit for bit); empty
   // otherwise
   std::vector<float> element_properties() const {
-    if (!gather2d() && !gather_path()) return {};
+    if (!gather2d() && !gather_path() && !h.general3d) return {};
     const size_t npe = h.npe;
     std::vector<float> kmu(2 * static_cast<size_t>(h.nspec));
     auto same = [](float a, float b) { return std::memcmp(&a, &b, sizeof(float)) == 0; };
@@ -324,7 +331,7 @@ struct sfx_engine {
     return kmu;
   }
   void upload_element_properties(hipStream_t s) {
-    if (!gather_path()) return;
+    if (!gather_path() && !h.general3d) return;
     const std::vector<float> kmu = element_properties();
     if (kmu.empty())
       kmu_e.alloc(0);
@@ -333,6 +340,56 @@ struct sfx_engine {
   }
 
   bool block_path() const { return h.dim == 3 && run.scatter == SFX_SCATTER_BLOCK; }
+  bool summed3() const { return h.general3d && run.scatter == SFX_SCATTER_COLORED; }
+  General3D general3d() const {
+    return General3D{geo_of.p, geo3.p, h.geo3_regular[0], h.geo3_regular[1], kappa.p, mu.p, kmu_e.p};
+  }
+  void upload_general_3d(hipStream_t s) {
+    std::vector<int32_t> row(h.nspec, -1);
+    std::vector<float> g;
+    int n = 0;
+    const size_t w = 10 * static_cast<size_t>(h.npe);
+    for (int e = 0; e < h.nspec; e++)
+      if (h.irregular3[e]) {
+        row[e] = n++;
+        g.insert(g.end(), h.geo3.begin() + e * w, h.geo3.begin() + (e + 1) * w);
+      }
+    geo_of.upload(row, s);
+    geo3.upload(g, s);
+    SFX_HIP(hipStreamSynchronize(s));
+    if (!summed3()) return;
+    // contributions of a point: sources in order, elements in color order,
+    // Stacey entries in order
+    const int npe = h.npe, nspec = h.nspec;
+    std::vector<int> order(nspec);
+    for (int e = 0; e < nspec; e++) order[key3[e]] = e;
+    std::vector<int> off(static_cast<size_t>(h.nglob) + 1, 0);
+    if ((static_cast<int64_t>(nspec) + h.nsrc + (h.bnd_gather.size() + 124) / 125) * 375 > UINT32_MAX)
+      throw std::invalid_argument("3-D mesh too large: its contributions exceed 32-bit device indexing");
+    auto each = [&](auto &&put) {
+      for (int k = 0; k < h.nsrc; k++)
+        for (int p = 0; p < npe; p++) put(h.gather[static_cast<size_t>(h.src_ispec[k]) * npe + p], (static_cast<uint32_t>(nspec) + k) * 375u + p);
+      for (int e : order)
+        for (int p = 0; p < npe; p++) put(h.gather[static_cast<size_t>(e) * npe + p], e * 375u + p);
+      for (size_t q = 0; q < h.bnd_gather.size(); q++)
+        put(h.bnd_gather[q], static_cast<uint32_t>((static_cast<size_t>(nspec) + h.nsrc + q / 125) * 375 + q % 125));
+    };
+    each([&](int g_, uint32_t) { off[g_ + 1]++; });
+    for (int g_ = 0; g_ < h.nglob; g_++) off[g_ + 1] += off[g_];
+    std::vector<uint32_t> ent(off.back());
+    std::vector<int> fill(off.begin(), off.end() - 1);
+    each([&](int g_, uint32_t o) { ent[fill[g_]++] = o; });
+    off3.upload(off, s);
+    ent3.upload(ent, s);
+    re3.alloc((static_cast<size_t>(nspec) + h.nsrc + (h.bnd_gather.size() + 124) / 125) * 375);
+    SFX_HIP(hipStreamSynchronize(s));
+  }
+  void forces_3d(Fields ff, int istep) {
+    if (istep < 0 || istep >= run.nstep) throw std::invalid_argument("istep out of range");
+    launch_forces_3d_general(stream, h.nspec, gather.p, general3d(), q, ff, h.nsrc, istep, src_array.p, stf.p,
+                             static_cast<int>(h.bnd_gather.size()), bnd_gather.p, bnd_normal.p, bnd_weight.p, bnd_rvp.p,
+                             bnd_rvs.p, re3.p);
+  }
 
   // Stacey entries regrouped for the block path: entry slot = owner * 386 +
   // slot of its point for the block of its element (lattice.hpp), entries
@@ -394,7 +451,7 @@ struct sfx_engine {
     kappa.upload(permuted(h.kappa), s);
     mu.upload(permuted(h.mu), s);
     upload_element_properties(s);
-    if (h.general3d) geo3.upload(permuted(h.geo3, 10 * static_cast<size_t>(h.npe)), s);
+    if (h.general3d) upload_general_3d(s);
     if (h.dim == 2) {
       xix.upload(permuted(h.xix), s);
       xiz.upload(permuted(h.xiz), s);
@@ -571,7 +628,7 @@ struct sfx_engine {
         launch_stiffness_2d(stream, first, count, atomic, gather.p, xix.p, xiz.p, gammax.p, gammaz.p, jac.p, kappa.p,
                             mu.p, q, ff, rec_mode, rec_index.p, rec_step, nullptr, 0, geo.p);
       else if (h.general3d)
-        launch_stiffness_3d_general(stream, first, count, atomic, gather.p, geo3.p, kappa.p, mu.p, q, ff);
+        launch_stiffness_3d_general(stream, h.nspec, gather.p, general3d(), q, ff);
       else
         launch_stiffness_3d(stream, first, count, atomic, gather.p, kappa.p, mu.p, h.xix3, h.ety3, h.gaz3, h.jac3, q,
                             ff);
@@ -688,6 +745,29 @@ struct sfx_engine {
       launch_assemble_update_3d(stream, lat, re_p, zero.p, ff, nc, minv1.p, h.absorb_mask);
       if (evs) SFX_HIP(hipEventRecord(evs[4], stream));
       a_stale = true;
+      return;
+    }
+    if (summed3()) {
+      if (a_kept) {  // fused steps leave a zero acceleration
+        const size_t stride = static_cast<size_t>(h.ncomp) * h.nglob_pad;
+        launch_fill(stream, fields.p + 2 * stride, stride, 0.0f);
+        a_kept = false;
+      }
+      if (evs) SFX_HIP(hipEventRecord(evs[0], stream));
+      if (evs) SFX_HIP(hipEventRecord(evs[1], stream));
+      forces_3d(ff, istep);
+      if (evs) SFX_HIP(hipEventRecord(evs[2], stream));
+      if (istep % run.nstep_between_samples == 0) {
+        const int isig = istep / run.nstep_between_samples;
+        if (isig >= nsig) throw std::invalid_argument("seismogram step out of range");
+        bool need_a = false;
+        for (int it = 0; it < run.nseismo_types; it++) need_a = need_a || run.seismo_types[it] != SFX_DISPLACEMENT;
+        launch_seismograms_3d_general(stream, h.nrec, run.nseismo_types, types.p, isig, rec_ispec.p, gather.p, rec_h.p,
+                                      ff, nc.dto2, seismo.p, off3.p, ent3.p, re3.p, need_a);
+      }
+      if (evs) SFX_HIP(hipEventRecord(evs[3], stream));
+      launch_update_3d_general(stream, h.nglob, off3.p, ent3.p, re3.p, ff, nc, 0);
+      if (evs) SFX_HIP(hipEventRecord(evs[4], stream));
       return;
     }
     if (h.coupled()) {
@@ -817,6 +897,10 @@ struct sfx_engine {
     } else if (patches()) {
       if (istep < 0 || istep >= run.nstep) throw std::invalid_argument("istep out of range");
       patch_force(istep);
+    } else if (summed3()) {
+      forces_3d(ff, istep);
+      launch_update_3d_general(stream, h.nglob, off3.p, ent3.p, re3.p, ff, nc, 1);
+      a_kept = true;
     } else {
       if (h.coupled()) couple_into_elastic(ff);
       sources(ff, istep);
@@ -1023,6 +1107,14 @@ template <class Build> int create(Build &&build, const sfx_run_desc *run, sfx_en
     // engines carry them too
     color_elements(e->h, run->scatter);
     e->host_only = host_only;
+    if (e->summed3()) {
+      // all elements in one launch, in mesh order; the colors order the sums
+      e->key3 = e->h.inv_perm;
+      std::iota(e->h.perm.begin(), e->h.perm.end(), 0);
+      e->h.inv_perm = e->h.perm;
+      e->h.color_offsets = {0, e->h.nspec};
+      e->h.ncolors_el = 1;
+    }
     if (e->patches()) {
       // a point's contributions are summed by element in compute order
       // (gather) or in color order
@@ -1119,7 +1211,7 @@ int sfx_get_layout(const sfx_engine *e, int64_t *s) {
     check_engine(e);
     if (!s) throw std::invalid_argument("null output");
     s[0] = e->h.dim == 2 ? e->geom2d_form() : (e->h.general3d ? GEOM2D_POINT : GEOM2D_RECORD);
-    s[1] = e->element_properties().empty() ? 0 : 1;
+    s[1] = e->h.general3d || e->element_properties().empty() ? 0 : 1;
     s[2] = e->run.scatter;
     s[3] = e->gather2d() ? 1 : 0;
   });

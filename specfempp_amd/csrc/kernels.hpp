@@ -6,6 +6,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cstdint>
+
 namespace sfx {
 
 // GLL constants passed by value: they live in scalar registers, so the
@@ -203,12 +205,33 @@ void launch_divide_corrector(hipStream_t s, int ncomp, Fields f, NewmarkConst nc
 void launch_fill(hipStream_t s, float *p, size_t n, float value);
 
 // ---- 3-D general hexahedra (general3d.hip) ----
-// Stiffness over device element slots [first, first + count) with per-point
-// geometry geo (nspec, 10, 125): xix, xiy, xiz, etax, etay, etaz, gammax,
-// gammay, gammaz, jacobian.
-void launch_stiffness_3d_general(hipStream_t s, int first, int count, bool atomic, const int *gather,
-                                 const float *geo, const float *kappa, const float *mu, const GllConst &q,
+// Geometry and material of a database mesh: geo (irregular elements, 10, 125):
+// xix, xiy, xiz, etax, etay, etaz, gammax, gammay, gammaz, jacobian; geo_of:
+// each element's row, or -1 for a regular one (xr, jr); kappa and mu per point,
+// or (kmu) one pair per element.
+struct General3D {
+  const int *geo_of;
+  const float *geo;
+  float xr, jr;
+  const float *kappa, *mu, *kmu;
+};
+// Element forces added to f.a with atomics.
+void launch_stiffness_3d_general(hipStream_t s, int nspec, const int *gather, const General3D &m, const GllConst &q,
                                  Fields f);
+// Element forces, source terms and Stacey terms into re: blocks of 375 floats
+// (component, 125), one per element, one per source, then one per 125 Stacey
+// entries.
+void launch_forces_3d_general(hipStream_t s, int nspec, const int *gather, const General3D &m, const GllConst &q,
+                              Fields f, int nsrc, int istep, const float *array, const float *stf, int nbnd,
+                              const int *bgather, const float *normal, const float *weight, const float *rho_vp,
+                              const float *rho_vs, float *re);
+// Per point the sum of its contributions ent[off[g] .. off[g + 1]) (offsets
+// into re), divided by the mass; then corrector and predictor, or (divide) a.
+void launch_update_3d_general(hipStream_t s, int nglob, const int *off, const uint32_t *ent, const float *re, Fields f,
+                              NewmarkConst nc, int divide);
+void launch_seismograms_3d_general(hipStream_t s, int nrec, int ntypes, const int *types, int isig, const int *ispec,
+                                   const int *gather, const float *h, Fields f, float dto2, float *seismo,
+                                   const int *off, const uint32_t *ent, const float *re, int need_a);
 
 // ---- 2-D acoustic medium and elastic-acoustic coupling (acoustic.hip) ----
 // Acoustic stiffness over device element slots [first, first + count) of the
