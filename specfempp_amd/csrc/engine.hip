@@ -90,6 +90,9 @@ struct sfx_engine {
   // forward steps
   PatchPlan plan;
   PatchDevice patch;
+  DevBuf<char> adj_lists;   // adjoint sources by patch, rows of the kernels
+  DevBuf<float> adj_work;   // the adjoint field's boundary state and contributions
+  PatchPairTables pair{};
   // 3-D gather path: (kappa, mu) per element when both are the same at all
   // points of every element
   DevBuf<float> kmu_e;
@@ -258,7 +261,8 @@ struct sfx_engine {
   // The gather scatter rounds every product and sum on its own, as the oracle
   // does, and keeps the last acceleration; the colored one contracts them and
   // leaves the acceleration zero, where its other kernels accumulate.
-  void patch_steps(int first, int count, hipEvent_t *evs = nullptr) {
+  // record: the Stacey elements' forces go to the adjoint's record.
+  void patch_steps(int first, int count, hipEvent_t *evs = nullptr, bool record_on = false) {
     if (count <= 0) return;
     const bool exact = gather2d();
     if (!exact && a_kept) {
@@ -275,27 +279,114 @@ struct sfx_engine {
     for (int j = 0; j < count; j++) {
       const bool last = j == count - 1;
       launch_patch_step(stream, patch.pe, npatch(), h.nrec, exact, t, st, q,
-                        PatchLaunch{nullptr, nullptr, first + j, j & 1, j > 0, 1, exact && last});
+                        PatchLaunch{nullptr, nullptr, first + j, j & 1, j > 0, 1, exact && last,
+                                    record_on ? record.p : nullptr, record_stride()});
       throttle.tick();
     }
     if (evs) SFX_HIP(hipEventRecord(evs[2], stream));
     const int rd = count & 1;
     if ((first + count - 1) % run.nstep_between_samples == 0)
-      launch_patch_step(stream, patch.pe, 0, h.nrec, exact, t, st, q, PatchLaunch{nullptr, nullptr, first + count, rd, 1, 1, 0});
+      launch_patch_step(stream, patch.pe, 0, h.nrec, exact, t, st, q, PatchLaunch{nullptr, nullptr, first + count, rd, 1, 1, 0, nullptr, 0});
     if (evs) SFX_HIP(hipEventRecord(evs[3], stream));
     launch_patch_boundary(stream, exact, t, st, nc, rd, 1, exact);
     if (evs) SFX_HIP(hipEventRecord(evs[4], stream));
     if (exact) a_kept = true;
   }
   // update_wavefields of the forward field: a = M^-1 f of step istep
-  void patch_force(int istep) {
+  long long record_stride() const { return static_cast<long long>(nstacey) * h.npe * h.ncomp; }
+  void patch_force(int istep, bool record_on = false) {
     const bool exact = gather2d();
     const Fields ff = f();
     const PatchTables t = patch_tables();
     const PatchState st = patch.state(ff.u, ff.v, ff.a);
-    launch_patch_step(stream, patch.pe, npatch(), 0, exact, t, st, q, PatchLaunch{nullptr, nullptr, istep, 0, 0, 0, 0});
+    launch_patch_step(stream, patch.pe, npatch(), 0, exact, t, st, q, 
+                      PatchLaunch{nullptr, nullptr, istep, 0, 0, 0, 0, record_on ? record.p : nullptr, record_stride()});
     launch_patch_boundary(stream, exact, t, st, nc, 1, 0, 0);
     a_kept = true;
+  }
+  // Recorded forward run: fused steps between the checkpoints; a checkpoint
+  // step and the last one stop at the corrected state, which is kept.
+  void patch_record() {
+    const Fields ff = f();
+    const size_t n3 = 3 * static_cast<size_t>(h.ncomp) * h.nglob_pad;
+    for (int i = 0; i < run.nstep;) {
+      int end = i;
+      while (end < run.nstep - 1 && !is_checkpoint(end)) end++;
+      patch_steps(i, end - i, nullptr, true);
+      patch_force(end, true);
+      launch_divide_corrector(stream, h.ncomp, ff, nc, 0, 1);
+      if (end % run.nstep_between_samples == 0) seismograms(ff, end / run.nstep_between_samples, 0);
+      if (is_checkpoint(end))
+        SFX_HIP(hipMemcpyAsync(snapshots.p + static_cast<size_t>(end / snapshot_every) * n3, fields.p,
+                               n3 * sizeof(float), hipMemcpyDeviceToDevice, stream));
+      if (end < run.nstep - 1) {
+        launch_predictor(stream, h.ncomp, ff, nc);
+        a_kept = false;
+      }
+      i = end + 1;
+    }
+  }
+  // adjoint sources by patch and element, in application order within an element
+  void upload_adjoint_lists() {
+    const size_t np = plan.head.size();
+    std::vector<int32_t> patch_of(plan.elem.size());
+    for (size_t k = 0; k < np; k++)
+      for (int i = plan.head[k].el0; i < plan.head[k].el0 + plan.head[k].nel; i++) patch_of[i] = static_cast<int32_t>(k);
+    std::vector<std::pair<int32_t, int32_t>> src;  // (plan element, source) in application order
+    for (int32_t v : h.adj_order) src.push_back({plan.slot_of[0][h.adj_ispec[v]], v});
+    std::stable_sort(src.begin(), src.end(), [](const auto &a, const auto &b) { return a.first < b.first; });
+    std::vector<int2> head(np, int2{0, 0});
+    std::vector<int4> el;
+    std::vector<int> id;
+    size_t i = 0;
+    for (size_t k = 0; k < np; k++) {
+      head[k].x = static_cast<int>(el.size());
+      while (i < src.size() && patch_of[src[i].first] == static_cast<int32_t>(k)) {
+        const int32_t e = src[i].first;
+        const int first = static_cast<int>(id.size());
+        for (; i < src.size() && src[i].first == e; i++) id.push_back(src[i].second);
+        el.push_back(make_int4(e - plan.head[k].el0, first, static_cast<int>(id.size()), 0));
+      }
+      head[k].y = static_cast<int>(el.size());
+    }
+    std::vector<int> kslot(plan.elem.size());
+    for (size_t j = 0; j < plan.elem.size(); j++) kslot[j] = h.inv_perm[plan.elem[j]];
+    PatchBlob b;
+    const size_t o_head = b.add(head), o_el = b.add(el), o_id = b.add(id), o_k = b.add(kslot);
+    adj_lists.upload(b.bytes, stream);
+    SFX_HIP(hipStreamSynchronize(stream));
+    pair.adj_head = reinterpret_cast<const int2 *>(adj_lists.p + o_head);
+    pair.adj_el = reinterpret_cast<const int4 *>(adj_lists.p + o_el);
+    pair.adj_id = reinterpret_cast<const int *>(adj_lists.p + o_id);
+    pair.kslot = reinterpret_cast<const int *>(adj_lists.p + o_k);
+    pair.adj_array = adj_array.p;
+    pair.adj_stf = adj_stf.p;
+    pair.adj_step = 2 * static_cast<long long>(h.nadj);
+  }
+  // Steps hi, hi - 1, ..., lo of the combined loop, one launch each, from and
+  // to predicted states of both fields.
+  void patch_pair_steps(int hi, int lo, Fields adj, Fields bwd, float *Kmu, float *Kkappa, Throttle &throttle) {
+    const PatchTables t = patch_tables();
+    const size_t nb = t.nbnd, nr = patch.rb[1] - patch.rb[0];
+    adj_work.ensure(std::max<size_t>(4 * nb + 4 * nr, 1));
+    float2 *const rb = reinterpret_cast<float2 *>(adj_work.p + 4 * nb);
+    const PatchState sa{adj.u, adj.v, adj.a, adj_work.p, {rb, rb + nr}};
+    const PatchState sb = patch.state(bwd.u, bwd.v, bwd.a);
+    PatchPairTables p = pair;
+    p.Kmu = Kmu;
+    p.Kkappa = Kkappa;
+    p.R = racc.p;
+    const int top = (run.nstep - 1) / run.nstep_between_samples;
+    for (int i = hi; i >= lo; i--) {
+      launch_patch_pair(stream, patch.pe, npatch(), h.nrec, t, sa, sb, q,
+                        PatchPairLaunch{i, (hi - i) & 1, i < hi, top, record.p + static_cast<size_t>(i) * record_stride()},
+                        p);
+      throttle.tick();
+    }
+    const int rd = (hi - lo + 1) & 1;
+    if (lo % run.nstep_between_samples == 0)
+      launch_patch_pair(stream, patch.pe, 0, h.nrec, t, sa, sb, q, PatchPairLaunch{lo - 1, rd, 1, top, nullptr}, p);
+    launch_patch_pair_boundary(stream, t, sa, sb, nc, rd, racc.p);
   }
   const int *device_order() {
     if (h.lattice_of.empty()) return nullptr;
@@ -1017,7 +1108,7 @@ struct sfx_engine {
       launch_update_pair(stream, h.ncomp, adj, bwd, nc, 1, racc.p);
       launch_step_tick(stream, d_step.p, -1);
     };
-    const bool graphs = graph_2d();
+    const bool graphs = graph_2d() && !patches();
     if (graphs) set_step(nstep - 1);
     Throttle throttle(stream);
     int isig = 0;
@@ -1025,6 +1116,15 @@ struct sfx_engine {
       const bool first = istep == nstep - 1;
       const bool ckpt = is_checkpoint(istep);
       const bool sample = istep % nsb == 0;
+      if (patches() && !first && !ckpt) {
+        int lo = istep;
+        while (lo > 0 && !is_checkpoint(lo - 1)) lo--;
+        patch_pair_steps(istep, lo, adj, bwd, Kmu, Kkappa, throttle);
+        for (; istep >= lo; istep--)
+          if (istep % nsb == 0) isig++;
+        istep++;  // the loop steps on from lo
+        continue;
+      }
       if (graphs && !first && !ckpt) {
         if (!g_adj) g_adj = capture(enqueue_regular);
         SFX_HIP(hipGraphLaunch(g_adj, stream));
@@ -1730,10 +1830,11 @@ int sfx_forward_record(sfx_engine *e, int snapshot_every) {
     e->recorded = false;
     e->recording = true;
     try {
-      const bool graphs = e->graph_2d();
+      const bool graphs = e->graph_2d() && !e->patches();
       if (graphs) e->set_step(0);
       Throttle throttle(e->stream);
-      for (int istep = 0; istep < e->run.nstep; istep++) {
+      if (e->patches()) e->patch_record();
+      for (int istep = e->patches() ? e->run.nstep : 0; istep < e->run.nstep; istep++) {
         const bool last = istep == e->run.nstep - 1;
         if (graphs && !last && !e->is_checkpoint(istep)) {
           if (!e->g_rec) e->g_rec = e->capture([&] { e->enqueue_forward_2d(true); });
@@ -1764,6 +1865,7 @@ int sfx_set_adjoint_sources(sfx_engine *e, int nadj, const sfx_receiver *positio
     e->adj_slot.upload(e->slots_of(e->h.adj_ispec), s);
     e->adj_array.upload(e->h.adj_array, s);
     e->adj_stf.upload(e->h.adj_stf, s);
+    if (e->patches()) e->upload_adjoint_lists();
     SFX_HIP(hipStreamSynchronize(s));
     e->adj_ready = true;
     e->invalidate_graphs();

@@ -410,16 +410,6 @@ Entries plan_stacey(const PatchPlan &plan, const std::vector<const HostAssembly 
   return out;
 }
 
-// Arrays laid one after the other (256-byte boundaries) for one copy.
-struct Blob {
-  std::vector<char> bytes;
-  template <class T> size_t add(const std::vector<T> &v) {
-    const size_t at = (bytes.size() + 255) / 256 * 256;
-    bytes.resize(at + v.size() * sizeof(T));
-    if (!v.empty()) std::memcpy(bytes.data() + at, v.data(), v.size() * sizeof(T));
-    return at;
-  }
-};
 template <class T> void point_to(const T *&p, const DevBuf<char> &mem, size_t at) {
   p = reinterpret_cast<const T *>(mem.p + at);
 }
@@ -463,7 +453,7 @@ void PatchDevice::upload_properties(const PatchPlan &plan, const std::vector<con
         rp.push_back(h.bnd_rho_vp[q]);
         rs.push_back(h.bnd_rho_vs[q]);
       }
-  Blob b;
+  PatchBlob b;
   const size_t o[] = {b.add(km), b.add(kv), b.add(mv), b.add(n), b.add(w), b.add(rp), b.add(rs)};
   props_mem.upload(b.bytes, s);
   SFX_HIP(hipStreamSynchronize(s));
@@ -578,7 +568,14 @@ void PatchDevice::upload(const PatchPlan &plan, const std::vector<const HostAsse
   }
   while (rec_end.size() < meshes.size()) rec_end.push_back(static_cast<int>(v_rec.size()));
   if (!v_seg_pt.empty()) v_seg_off.push_back(nentry);
-  Blob b;
+  std::vector<int> v_rec_row(plan.elem.size());
+  for (const PatchHead &hd : heads)
+    for (int i = hd.el0; i < hd.el0 + hd.nel; i++) {
+      const int none = meshes[hd.sim]->nspec_none;
+      v_rec_row[i] = plan.elem[i] >= none ? plan.elem[i] - none : -1;
+    }
+  PatchBlob b;
+  const size_t o_row = b.add(v_rec_row);
   const size_t o_head = b.add(heads), o_tab = b.add(plan.tab), o_sim = b.add(sims), o_bpt = b.add(plan.bpt),
                o_boff = b.add(plan.boff), o_bslot = b.add(plan.bslot), o_segp = b.add(v_seg_pt),
                o_segl = b.add(v_seg_loc), o_sego = b.add(v_seg_off), o_srce = b.add(v_src_el),
@@ -637,6 +634,7 @@ void PatchDevice::upload(const PatchPlan &plan, const std::vector<const HostAsse
   point_to(t.rec_h, tables_mem, o_rech);
   point_to(t.rp_of, tables_mem, o_rpof);
   point_to(t.rmap, tables_mem, o_rmap);
+  point_to(t.rec_row, tables_mem, o_row);
   t.geom.mode = mode;
   point_to(mode == GEOM2D_RECORD ? t.geom.record : mode == GEOM2D_POINT ? t.geom.xix : t.geom.ctrl, tables_mem,
            o_geo[0]);

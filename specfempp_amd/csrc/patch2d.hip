@@ -212,39 +212,40 @@ __device__ __forceinline__ BoundaryState boundary_state(const PatchTables &T, co
   return {S.u + T.nint, S.u + T.np + static_cast<size_t>(T.nint), S.v + T.nint, S.v + T.np + static_cast<size_t>(T.nint)};
 }
 
-// Samples of step n - 1 at one receiver, by one wavefront (compute_seismogram
+// Samples of step `step` at one receiver, by one wavefront (compute_seismogram
 // .tpp:103-135): u, corrected v and a at its element's points, from the
 // snapshot the last launch took of interior points and, for boundary points,
-// from the state and contributions that launch left.
+// from the state and contributions that launch left in buffers rd.  sign: of
+// the time step; top: sample index of step 0 when the steps run backwards, or -1.
 template <int GEOM, bool EPROP, bool EXACT>
-__device__ __forceinline__ void sample_receiver(int r, bool store, int n, const PatchTables &T, const PatchState &S,
-                                                const GllConst &q, const PatchLaunch &L) {
+__device__ __forceinline__ void sample_receiver(int r, bool store, int step, int top, float sign, int rd,
+                                                const PatchTables &T, const PatchState &S, const GllConst &q) {
   const int lane = threadIdx.x & 63;
   const int p = lane < 25 ? lane : 0;
   const int4 rc = T.rec[r];
   const int rp = T.rp_of[r * 25 + p];
   const PatchSim sim = T.sim[rc.z];
   const float hw = lane < 25 ? T.rec_h[static_cast<size_t>(rc.x) * 25 + p] : 0.0f;
-  store = store && n >= 1 && n - 1 < sim.nstep && (n - 1) % sim.nsb == 0 && lane == 0;
-  const int isig = n >= 1 ? (n - 1) / sim.nsb : 0;
+  store = store && step >= 0 && step < sim.nstep && step % sim.nsb == 0 && lane == 0;
+  const int isig = top >= 0 ? top - step / sim.nsb : step / sim.nsb;
   float x[6];
   if (rp >= 0) {
-    const float *smp = T.snap + 6 * (static_cast<size_t>((n - 1) & 1) * T.nrow + rp);
+    const float *smp = T.snap + 6 * (static_cast<size_t>(rd) * T.nrow + rp);
 #pragma unroll
     for (int i = 0; i < 6; i++) x[i] = smp[i];
   } else {
 #pragma clang fp contract(off)
     const int b = -1 - rp;
-    const BoundaryState bs = boundary_state(T, S, L.rd);
+    const BoundaryState bs = boundary_state(T, S, rd);
     const float u[2] = {bs.u0[b], bs.u1[b]}, v[2] = {bs.v0[b], bs.v1[b]};
     float s[2];
     const int k0 = T.boff[b];
-    boundary_force(S.rb[L.rd], k0, T.boff[b + 1] - k0, s);
+    boundary_force(S.rb[rd], k0, T.boff[b + 1] - k0, s);
 #pragma unroll
     for (int c = 0; c < 2; c++) {
       const float a = s[c] * T.minv[c * static_cast<size_t>(T.np) + T.nint + b];
       x[c] = u[c];
-      x[2 + c] = mad<EXACT>(sim.dto2, a, v[c]);
+      x[2 + c] = mad<EXACT>(sign * sim.dto2, a, v[c]);
       x[4 + c] = a;
     }
   }
@@ -298,7 +299,9 @@ __device__ __forceinline__ void sample_receiver(int r, bool store, int n, const 
 // the element's other rows from LDS.  Workgroups past the patches sample the
 // receivers, one wavefront each.
 // Five wavefronts per SIMD (96 registers): 269 us at 1000 x 900 with four.
-template <int PE, int GEOM, bool EPROP, bool EXACT>
+// RECORD (contracted form): the Stacey elements' forces are kept for the adjoint
+// run; in a form of its own, as its branches cost the plain step 1 us in 8.
+template <int PE, int GEOM, bool EPROP, bool EXACT, bool RECORD>
 __global__ __launch_bounds__(patch_threads<PE>()) __attribute__((amdgpu_waves_per_eu(5))) void patch_step_kernel(int npatch, int nrec, PatchTables T,
                                                                         PatchState S, GllConst q, PatchLaunch L) {
   constexpr int NT = patch_threads<PE>();
@@ -317,7 +320,7 @@ __global__ __launch_bounds__(patch_threads<PE>()) __attribute__((amdgpu_waves_pe
   if (L.next && blockIdx.x == 0 && t == 0) *L.next = n + 1;
   if (static_cast<int>(blockIdx.x) >= npatch) {
     const int r = (blockIdx.x - npatch) * (NT / 64) + (t >> 6);  // wavefronts past the last receiver repeat it
-    sample_receiver<GEOM, EPROP, EXACT>(r < nrec ? r : nrec - 1, r < nrec, n, T, S, q, L);
+    sample_receiver<GEOM, EPROP, EXACT>(r < nrec ? r : nrec - 1, r < nrec, n - 1, -1, 1.0f, L.rd, T, S, q);
     return;
   }
   const PatchHead h = T.head[xcd_block(blockIdx.x, npatch)];
@@ -500,6 +503,10 @@ __global__ __launch_bounds__(patch_threads<PE>()) __attribute__((amdgpu_waves_pe
       r[c] = -mad<EXACT>(wrow, t1, q.w[i] * t2);
     }
     *reinterpret_cast<float2 *>(&se[lc * 50 + 2 * (row * 5 + i)]) = make_float2(r[0], r[1]);
+    if constexpr (RECORD)
+      if (T.rec_row[e] >= 0)
+        *reinterpret_cast<float2 *>(L.rec + n * L.rec_stride + (static_cast<size_t>(T.rec_row[e]) * 25 + row * 5 + i) * 2) =
+            make_float2(r[0], r[1]);
   }
   __syncthreads();
 
@@ -538,6 +545,10 @@ __global__ __launch_bounds__(patch_threads<PE>()) __attribute__((amdgpu_waves_pe
         se[2 * sp + 1] += s[1];
       } else {
         reinterpret_cast<float2 *>(sF)[sg - h.seg0] = make_float2(s[0], s[1]);
+        if constexpr (RECORD)  // a Stacey element's record holds its force with the traction
+          *reinterpret_cast<float2 *>(L.rec + n * L.rec_stride +
+                                      (static_cast<size_t>(T.rec_row[h.el0 + sp / 25]) * 25 + sp % 25) * 2) =
+              make_float2(se[2 * sp] + s[0], se[2 * sp + 1] + s[1]);
       }
     }
     __syncthreads();
@@ -589,7 +600,7 @@ __global__ __launch_bounds__(patch_threads<PE>()) __attribute__((amdgpu_waves_pe
       if (snapshot) {  // of a receiver's element point, before it was advanced
         const int rowi = T.rmap[h.rm0 + l];
         if (rowi >= 0) {
-          float *o = T.snap + 6 * (static_cast<size_t>(n & 1) * T.nrow + rowi);
+          float *o = T.snap + 6 * (static_cast<size_t>(L.rd ^ 1) * T.nrow + rowi);
           o[0] = su[0][l];
           o[1] = su[1][l];
           o[2] = w0;
@@ -603,6 +614,362 @@ __global__ __launch_bounds__(patch_threads<PE>()) __attribute__((amdgpu_waves_pe
       put(S.a + h.pt0, l, a0);
       put(S.a + np + h.pt0, l, a1);
     }
+  }
+}
+
+// One step of the combined adjoint + backward loop (time_marching.tpp:160-215)
+// of one patch: the adjoint field (A, forward in time, adjoint sources, Stacey)
+// and then the backward field (B, -dt, forward sources, the recorded force at
+// Stacey elements, compute_stiffness_interaction.tpp:119-136) go through the
+// phases of patch_step_kernel one after the other in the same LDS; the adjoint
+// gradients and accelerations stay in registers for the Frechet kernels'
+// products (frechet_derivative.hpp:58-118): Kmu, Kkappa per element point, R
+// (of the rho kernel) per point.
+template <int PE, int GEOM, bool EPROP>
+__global__ __launch_bounds__(patch_threads<PE>()) __attribute__((amdgpu_waves_per_eu(4))) void patch_pair_kernel(
+    int npatch, int nrec, PatchTables T, PatchState A, PatchState B, GllConst q, PatchPairLaunch L, PatchPairTables P) {
+  constexpr int NT = patch_threads<PE>();
+  constexpr int NP = PatchCap<PE>::points, NB = PatchCap<PE>::boundary;
+  constexpr int NI = (NP + NT - 1) / NT;
+  __shared__ float su[2][NP];
+  __shared__ float sv[2][NB];
+  __shared__ __align__(16) float se[PE * 100];
+  float *const sF = se + PE * 50;
+  float2 *const f2 = reinterpret_cast<float2 *>(se);
+  float2 *const fx = reinterpret_cast<float2 *>(sF);  // Stacey and source contributions
+
+  const int t = threadIdx.x;
+  if (static_cast<int>(blockIdx.x) >= npatch) {
+    const int r = (blockIdx.x - npatch) * (NT / 64) + (t >> 6);
+    sample_receiver<GEOM, EPROP, false>(r < nrec ? r : nrec - 1, r < nrec, L.step + 1, L.top, -1.0f, L.rd, T, B, q);
+    return;
+  }
+  const int patch = xcd_block(blockIdx.x, npatch);
+  const PatchHead h = T.head[patch];
+  const size_t np = T.np;
+  const uint16_t *__restrict__ tab = T.tab;
+  const int le = t / 5, row = t - le * 5;
+  const int lc = le < h.nel ? le : h.nel - 1;
+  const int e = h.el0 + lc;
+  const int rrow = T.rec_row[e];
+  const size_t krow = static_cast<size_t>(P.kslot[e]) * 25 + row * 5;
+  PatchPoint bp{0, 0, 1, 0};
+  if (h.nb > 0) bp = T.bpt[h.b0 + (t < h.nb ? t : h.nb - 1)];
+  const uint4 rw = *reinterpret_cast<const uint4 *>(reinterpret_cast<const char *>(tab + h.lidx) + (lc * 5 + row) * 16u);
+  const unsigned li[5] = {rw.x & 0xffffu, rw.x >> 16, rw.y & 0xffffu, rw.y >> 16, rw.z & 0xffffu};
+  constexpr int NC = GEOM == GEOM2D_POINT ? 1 : GEOM == GEOM2D_RECORD ? 8 : 2 * GEOM;
+  float ctrl[NC];
+  if constexpr (GEOM != GEOM2D_POINT) {
+    const float *c = (GEOM == GEOM2D_RECORD ? T.geom.record : T.geom.ctrl) + static_cast<size_t>(h.el0) * NC;
+#pragma unroll
+    for (int i = 0; i < NC; i++) ctrl[i] = at(c, lc * NC + i);
+  }
+  float ke = 0.0f, me = 0.0f;
+  if constexpr (EPROP) {
+    const float *km = T.kmu + 2 * static_cast<size_t>(h.el0);
+    ke = at(km, 2 * lc);
+    me = at(km, 2 * lc + 1);
+  }
+  float hrow[5], hwrow[5];
+#pragma unroll
+  for (int l = 0; l < 5; l++) {
+    hrow[l] = q.hp[row][l];
+    hwrow[l] = q.hpw[row][l];
+  }
+  const float wrow = q.w[row];
+  float xxi, zxi;
+  row_geometry<GEOM>(T.geom, row, ctrl, xxi, zxi);
+
+  float dua[5][4];          // adjoint gradients of the row
+  float aa[NI][2], ab[2];   // adjoint acceleration: interior, boundary point
+#pragma unroll
+  for (int fi = 0; fi < 2; fi++) {
+    const PatchState &S = fi ? B : A;
+    const Newmark<false> newmark{fi ? -h.dt : h.dt, fi ? -h.dto2 : h.dto2, h.dt2o2};
+    float *const u0p = S.u + h.pt0, *const u1p = S.u + np + h.pt0;
+    float *const v0p = S.v + h.pt0, *const v1p = S.v + np + h.pt0;
+    const float *const m0p = T.minv + h.pt0, *const m1p = T.minv + np + h.pt0;
+    float ui[NI][2];
+#pragma unroll
+    for (int k = 0; k < NI; k++) {
+      const int l = t + k * NT;
+      const unsigned g = l < h.nint ? l : h.nint - 1;
+      ui[k][0] = at(u0p, g);
+      ui[k][1] = at(u1p, g);
+    }
+    if (h.nb > 0) {
+      const int b = bp.b & 0x7fffffff;
+      const size_t o = T.nint + static_cast<size_t>(b);
+      const BoundaryState bs = boundary_state(T, S, L.rd);
+      float u[2] = {bs.u0[b], bs.u1[b]}, v[2] = {bs.v0[b], bs.v1[b]};
+      if (L.pending) {
+        const float m[2] = {T.minv[o], T.minv[np + o]};
+        float s[2];
+        boundary_force(S.rb[L.rd], bp.k0, bp.n, s);
+        if (fi == 0) {
+          ab[0] = s[0] * m[0];
+          ab[1] = s[1] * m[1];
+        } else if (t < h.nb && bp.b < 0) {
+          P.R[o] += h.dt * fmaf(ab[1], u[1], ab[0] * u[0]);
+        }
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+          float v1;
+          newmark(s[c] * m[c], u[c], v[c], v1);
+        }
+      }
+      if (t < h.nb) {
+        su[0][h.nint + t] = u[0];
+        su[1][h.nint + t] = u[1];
+        sv[0][t] = v[0];
+        sv[1][t] = v[1];
+        if (bp.b < 0) {
+          const BoundaryState to = boundary_state(T, S, L.rd ^ 1);
+          const_cast<float *>(to.u0)[b] = u[0];
+          const_cast<float *>(to.u1)[b] = u[1];
+          const_cast<float *>(to.v0)[b] = v[0];
+          const_cast<float *>(to.v1)[b] = v[1];
+        }
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < NI; k++)
+      if (t + k * NT < h.nint) {
+        su[0][t + k * NT] = ui[k][0];
+        su[1][t + k * NT] = ui[k][1];
+      }
+    __syncthreads();
+    float u[2][5];
+#pragma unroll
+    for (int i = 0; i < 5; i++)
+#pragma unroll
+      for (int c = 0; c < 2; c++) {
+        u[c][i] = su[c][li[i]];
+        se[lc * 50 + c * 25 + row * 5 + i] = u[c][i];
+      }
+    __syncthreads();
+    float F[2][5];
+#pragma unroll
+    for (int i = 0; i < 5; i++) {
+      float dxi[2], dga[2];
+#pragma unroll
+      for (int c = 0; c < 2; c++) {
+        dxi[c] = q.hp[i][0] * u[c][0];
+        dga[c] = hrow[0] * se[lc * 50 + c * 25 + i];
+#pragma unroll
+        for (int l = 1; l < 5; l++) {
+          dxi[c] = fmaf(q.hp[i][l], u[c][l], dxi[c]);
+          dga[c] = fmaf(hrow[l], se[lc * 50 + c * 25 + l * 5 + i], dga[c]);
+        }
+      }
+      const int p = row * 5 + i;
+      float xix, xiz, gammax, gammaz, J;
+      patch_geometry<GEOM>(T.geom, e, row, i, ctrl, xxi, zxi, xix, xiz, gammax, gammaz, J);
+      float kappa = ke, mu = me;
+      if constexpr (!EPROP) {
+        kappa = T.kappa[static_cast<size_t>(e) * 25 + p];
+        mu = T.mu[static_cast<size_t>(e) * 25 + p];
+      }
+      float du[2][2];
+#pragma unroll
+      for (int c = 0; c < 2; c++) {
+        du[c][0] = fmaf(xix, dxi[c], gammax * dga[c]);
+        du[c][1] = fmaf(xiz, dxi[c], gammaz * dga[c]);
+      }
+      const float lp2m = fmaf(4.0f / 3.0f, mu, kappa);
+      const float lambda = lp2m - 2.0f * mu;
+      const float sxx = fmaf(lp2m, du[0][0], lambda * du[1][1]);
+      const float szz = fmaf(lp2m, du[1][1], lambda * du[0][0]);
+      const float sxz = mu * (du[0][1] + du[1][0]);
+      F[0][i] = J * fmaf(sxx, xix, sxz * xiz);
+      F[1][i] = J * fmaf(sxz, xix, szz * xiz);
+      sF[lc * 25 + p] = J * fmaf(sxx, gammax, sxz * gammaz);
+      sF[PE * 25 + lc * 25 + p] = J * fmaf(sxz, gammax, szz * gammaz);
+      if (fi == 0) {
+        dua[i][0] = du[0][0];
+        dua[i][1] = du[0][1];
+        dua[i][2] = du[1][0];
+        dua[i][3] = du[1][1];
+      } else if (le < h.nel) {
+        // the strain kernels, as stiffness_pair_2d_kernel forms them
+        const float kap2 = lp2m - mu;
+        const float asxz = 0.5f * (dua[i][2] + dua[i][1]), bsxz = 0.5f * (du[1][0] + du[0][1]);
+        const float kk = (dua[i][0] + dua[i][3]) * (du[0][0] + du[1][1]);
+        const float km = dua[i][0] * du[0][0] + dua[i][3] * du[1][1] + 2.0f * asxz * bsxz - (1.0f / 3.0f) * kk;
+        P.Kkappa[krow + i] += -1.0f * kap2 * h.dt * kk;
+        P.Kmu[krow + i] += -2.0f * mu * h.dt * km;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    float vi[NI][2], mi[NI][2], ri[NI];
+    int ea[NI], eb[NI];
+#pragma unroll
+    for (int k = 0; k < NI; k++) {
+      const int l = t + k * NT;
+      const int ll = l < h.nint ? l : h.nint - 1;
+      vi[k][0] = at(v0p, ll);
+      vi[k][1] = at(v1p, ll);
+      mi[k][0] = at(m0p, ll);
+      mi[k][1] = mi[k][0];
+      if (h.nseg > 0) mi[k][1] = at(m1p, ll);
+      ri[k] = fi ? at(P.R + h.pt0, ll) : 0.0f;
+      ea[k] = at(tab + h.enta, ll);
+      eb[k] = at(tab + h.entb, ll >= h.n1 && h.n1 < h.nint ? ll - h.n1 : 0);
+    }
+    float2 rr[5];
+#pragma unroll
+    for (int i = 0; i < 5; i++) rr[i] = make_float2(0.0f, 0.0f);
+    if (fi && rrow >= 0)
+#pragma unroll
+      for (int i = 0; i < 5; i++)
+        rr[i] = *reinterpret_cast<const float2 *>(L.rec + (static_cast<size_t>(rrow) * 25 + row * 5 + i) * 2);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 5; i++) {
+      float r[2];
+#pragma unroll
+      for (int c = 0; c < 2; c++) {
+        float t1 = F[c][0] * q.hpw[i][0], t2 = sF[c * PE * 25 + lc * 25 + i] * hwrow[0];
+#pragma unroll
+        for (int l = 1; l < 5; l++) {
+          t1 = fmaf(F[c][l], q.hpw[i][l], t1);
+          t2 = fmaf(sF[c * PE * 25 + lc * 25 + l * 5 + i], hwrow[l], t2);
+        }
+        r[c] = -fmaf(wrow, t1, q.w[i] * t2);
+      }
+      f2[lc * 25 + row * 5 + i] = fi && rrow >= 0 ? rr[i] : make_float2(r[0], r[1]);
+    }
+    __syncthreads();
+    // the Stacey and source contributions of this field; the other field's
+    // are zero
+    for (int sg = t; sg < h.nseg; sg += NT) {
+      float s[2] = {0.0f, 0.0f};
+      if (fi == 0) {
+        const int l = T.seg_loc[h.seg0 + sg];
+        float v[2];
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+          if (l < h.nint)
+            v[c] = S.v[c * np + h.pt0 + l];
+          else
+            v[c] = sv[c][l - h.nint];
+        }
+        for (int k = T.seg_off[h.seg0 + sg]; k < T.seg_off[h.seg0 + sg + 1]; k++) {
+          const float nv[2] = {T.bnormal[2 * k], T.bnormal[2 * k + 1]};
+          const float w = T.bweight[k], rvp = T.brvp[k], rvs = T.brvs[k];
+          const float vn = fmaf(v[1], nv[1], v[0] * nv[0]);
+          const float nn = fmaf(nv[0], nv[0], nv[1] * nv[1]);
+          const float j1 = sqrtf(nn);
+#pragma unroll
+          for (int d = 0; d < 2; d++) {
+            const float fac = fmaf(rvs, v[d], (vn * nv[d] / (j1 * j1)) * (rvp - rvs));
+            s[d] += -1.0f * fac * j1 * w;
+          }
+        }
+      }
+      fx[sg] = make_float2(s[0], s[1]);
+    }
+    for (int k = t / 25; k < h.nsrc && t < NT / 25 * 25; k += NT / 25) {
+      const int p = t % 25;
+      float o[2] = {0.0f, 0.0f};
+      if (fi == 1) {
+        const int4 s4 = T.src_el[h.src0 + k];
+        for (int i = s4.y; i < s4.z; i++) {
+          const int id = T.src_id[i];
+          const float amp = T.stf[L.step * T.stf_step + id * T.stf_src];
+#pragma unroll
+          for (int c = 0; c < 2; c++) o[c] += amp * T.src_array[(static_cast<size_t>(id) * 2 + c) * 25 + p];
+        }
+      }
+      fx[h.nseg + k * 25 + p] = make_float2(o[0], o[1]);
+    }
+    if (fi == 0) {
+      // adjoint sources join their element's force
+      const int2 as = P.adj_head[patch];
+      for (int k = as.x + t / 25; k < as.y && t < NT / 25 * 25; k += NT / 25) {
+        const int p = t % 25;
+        const int4 s4 = P.adj_el[k];
+        float o[2] = {0.0f, 0.0f};
+        for (int i = s4.y; i < s4.z; i++) {
+          const int id = P.adj_id[i];
+          const float amp = P.adj_stf[L.step * P.adj_step + id];
+#pragma unroll
+          for (int c = 0; c < 2; c++) o[c] += amp * P.adj_array[(static_cast<size_t>(id) * 2 + c) * 25 + p];
+        }
+        const float2 x = f2[s4.x * 25 + p];
+        f2[s4.x * 25 + p] = make_float2(o[0] + x.x, o[1] + x.y);
+      }
+    }
+    __syncthreads();
+    {
+      float2 *out = S.rb[L.rd ^ 1];
+      for (int k = t; k < h.nbent; k += NT) out[T.bslot[h.be0 + k]] = f2[tab[h.bent + k]];
+    }
+    const bool snapshot = fi && h.rm0 >= 0 && L.step % h.nsb == 0;
+#pragma unroll
+    for (int k = 0; k < NI; k++) {
+      const int l = t + k * NT;
+      if (l >= h.nint) continue;
+      const float2 s = interior_force(h, tab, se, l, ea[k], eb[k]);
+      const float a0 = s.x * mi[k][0], a1 = s.y * mi[k][1];
+      float x0 = su[0][l], x1 = su[1][l], v0 = vi[k][0], v1 = vi[k][1], w0, w1;
+      if (fi == 0) {
+        aa[k][0] = a0;
+        aa[k][1] = a1;
+      } else {
+        put(P.R + h.pt0, l, ri[k] + h.dt * fmaf(aa[k][1], x1, aa[k][0] * x0));
+      }
+      newmark(a0, x0, v0, w0);
+      newmark(a1, x1, v1, w1);
+      put(u0p, l, x0);
+      put(u1p, l, x1);
+      put(v0p, l, v0);
+      put(v1p, l, v1);
+      if (snapshot) {
+        const int rowi = T.rmap[h.rm0 + l];
+        if (rowi >= 0) {
+          float *o = T.snap + 6 * (static_cast<size_t>(L.rd ^ 1) * T.nrow + rowi);
+          o[0] = su[0][l];
+          o[1] = su[1][l];
+          o[2] = w0;
+          o[3] = w1;
+          o[4] = a0;
+          o[5] = a1;
+        }
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// The boundary points of both fields after the last of a run of such steps.
+__global__ __launch_bounds__(256) void patch_pair_boundary_kernel(PatchTables T, PatchState A, PatchState B,
+                                                                  NewmarkConst nc, int rd, float *__restrict__ R) {
+  const int b = blockIdx.x * 256 + threadIdx.x;
+  if (b >= T.nbnd) return;
+  const int k0 = T.boff[b], n = T.boff[b + 1] - k0;
+  float aa[2];
+#pragma unroll
+  for (int fi = 0; fi < 2; fi++) {
+    const PatchState &S = fi ? B : A;
+    const Newmark<false> nm{fi ? -nc.dt : nc.dt, fi ? -nc.dto2 : nc.dto2, nc.dt2o2};
+    float s[2], rho = 0.0f;
+    boundary_force(S.rb[rd], k0, n, s);
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      const size_t o = c * static_cast<size_t>(T.np) + T.nint + b;
+      const float a = s[c] * T.minv[o];
+      float u = rd ? S.ub[c * static_cast<size_t>(T.nbnd) + b] : S.u[o];
+      float v = rd ? S.ub[(2 + c) * static_cast<size_t>(T.nbnd) + b] : S.v[o], v1;
+      if (fi)
+        rho = fmaf(aa[c], u, rho);
+      else
+        aa[c] = a;
+      nm(a, u, v, v1);
+      S.u[o] = u;
+      S.v[o] = v;
+    }
+    if (fi) R[T.nint + b] += nc.dt * rho;
   }
 }
 
@@ -648,9 +1015,11 @@ void launch_step(hipStream_t s, int npatch, int nrec, bool exact, const PatchTab
   constexpr int NT = patch_threads<PE>();
   const dim3 grid(npatch + (nrec + NT / 64 - 1) / (NT / 64)), block(NT);
   if (exact)
-    hipLaunchKernelGGL((patch_step_kernel<PE, GEOM, EPROP, true>), grid, block, 0, s, npatch, nrec, t, st, q, l);
+    hipLaunchKernelGGL((patch_step_kernel<PE, GEOM, EPROP, true, false>), grid, block, 0, s, npatch, nrec, t, st, q, l);
+  else if (l.rec)
+    hipLaunchKernelGGL((patch_step_kernel<PE, GEOM, EPROP, false, true>), grid, block, 0, s, npatch, nrec, t, st, q, l);
   else
-    hipLaunchKernelGGL((patch_step_kernel<PE, GEOM, EPROP, false>), grid, block, 0, s, npatch, nrec, t, st, q, l);
+    hipLaunchKernelGGL((patch_step_kernel<PE, GEOM, EPROP, false, false>), grid, block, 0, s, npatch, nrec, t, st, q, l);
 }
 
 template <int PE, int GEOM>
@@ -671,6 +1040,28 @@ void launch_step_geom(hipStream_t s, int npatch, int nrec, bool exact, const Pat
     case GEOM2D_CTRL9: return launch_step_prop<PE, GEOM2D_CTRL9>(s, npatch, nrec, exact, t, st, q, l);
     case GEOM2D_POINT: return launch_step_prop<PE, GEOM2D_POINT>(s, npatch, nrec, exact, t, st, q, l);
     default: throw std::invalid_argument("patch step: unknown geometry form");
+  }
+}
+
+template <int PE, int GEOM>
+void launch_pair_prop(hipStream_t s, int npatch, int nrec, const PatchTables &t, const PatchState &a,
+                      const PatchState &b, const GllConst &q, const PatchPairLaunch &l, const PatchPairTables &p) {
+  constexpr int NT = patch_threads<PE>();
+  const dim3 grid(npatch + (nrec + NT / 64 - 1) / (NT / 64)), block(NT);
+  if (t.kmu)
+    hipLaunchKernelGGL((patch_pair_kernel<PE, GEOM, true>), grid, block, 0, s, npatch, nrec, t, a, b, q, l, p);
+  else
+    hipLaunchKernelGGL((patch_pair_kernel<PE, GEOM, false>), grid, block, 0, s, npatch, nrec, t, a, b, q, l, p);
+}
+template <int PE>
+void launch_pair_geom(hipStream_t s, int npatch, int nrec, const PatchTables &t, const PatchState &a,
+                      const PatchState &b, const GllConst &q, const PatchPairLaunch &l, const PatchPairTables &p) {
+  switch (t.geom.mode) {
+    case GEOM2D_RECORD: return launch_pair_prop<PE, GEOM2D_RECORD>(s, npatch, nrec, t, a, b, q, l, p);
+    case GEOM2D_CTRL4: return launch_pair_prop<PE, GEOM2D_CTRL4>(s, npatch, nrec, t, a, b, q, l, p);
+    case GEOM2D_CTRL9: return launch_pair_prop<PE, GEOM2D_CTRL9>(s, npatch, nrec, t, a, b, q, l, p);
+    case GEOM2D_POINT: return launch_pair_prop<PE, GEOM2D_POINT>(s, npatch, nrec, t, a, b, q, l, p);
+    default: throw std::invalid_argument("patch pair: unknown geometry form");
   }
 }
 
@@ -696,6 +1087,22 @@ void launch_patch_boundary(hipStream_t s, bool exact, const PatchTables &t, cons
   else
     hipLaunchKernelGGL(patch_boundary_kernel<false>, grid, dim3(256), 0, s, t, st,
                        (Newmark<false>{nc.dt, nc.dto2, nc.dt2o2}), rd, advance, store_a);
+}
+
+void launch_patch_pair(hipStream_t s, int pe, int npatch, int nrec, const PatchTables &t, const PatchState &adj,
+                       const PatchState &bwd, const GllConst &q, const PatchPairLaunch &l, const PatchPairTables &p) {
+  if (!l.pending || t.ntypes <= 0) nrec = 0;
+  if (npatch + nrec <= 0) return;
+  if (pe == PATCH_LARGE)
+    launch_pair_geom<PATCH_LARGE>(s, npatch, nrec, t, adj, bwd, q, l, p);
+  else
+    launch_pair_geom<PATCH_SMALL>(s, npatch, nrec, t, adj, bwd, q, l, p);
+}
+
+void launch_patch_pair_boundary(hipStream_t s, const PatchTables &t, const PatchState &adj, const PatchState &bwd,
+                                NewmarkConst nc, int rd, float *R) {
+  if (t.nbnd > 0)
+    hipLaunchKernelGGL(patch_pair_boundary_kernel, dim3((t.nbnd + 255) / 256), dim3(256), 0, s, t, adj, bwd, nc, rd, R);
 }
 
 void launch_take(hipStream_t s, int n, const int *index, const float *src, float *dst) {

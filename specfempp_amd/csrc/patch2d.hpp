@@ -21,6 +21,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <cstring>
 #include <vector>
 
 #include "assembly.hpp"
@@ -130,10 +131,11 @@ struct PatchTables {
   const int *rp_of;               // (nrec, 25): row of snap of each receiver element point, or -1 - boundary point
   const int *rmap;
   int nrow;                       // rows of snap
+  const int *rec_row;             // plan order: Stacey element of the adjoint's record, or -1
   const int *types;
   int ntypes;
   const float *minv;              // (2, np)
-  float *snap;                    // (2, rows, 6): u, corrected v, a, by step parity
+  float *snap;                    // (2, rows, 6): u, corrected v, a, by launch parity
   float *seismo;
   int nint, np, nbnd;
 };
@@ -156,8 +158,37 @@ struct PatchLaunch {
   int pending;   // the contributions of step - 1 are summed first
   int advance;   // 1: corrector and predictor; 0: only a = M^-1 f (seam calls)
   int store_a;   // advance: keep a as well
+  float *rec;    // contracted form: the Stacey elements' forces of step n go to rec + n * rec_stride, or null
+  long long rec_stride;
 };
 
+// One launch of the combined adjoint + backward loop (contracted form).
+struct PatchPairLaunch {
+  int step, rd, pending;
+  int top;           // sample index of step 0
+  const float *rec;  // the Stacey elements' forces of this step
+};
+struct PatchPairTables {
+  const int2 *adj_head;    // adjoint source elements of each patch: [x, y) of adj_el
+  const int4 *adj_el;      // local element, sources [y, z) of adj_id
+  const int *adj_id;
+  const float *adj_array;  // (sources, 2, 25)
+  const float *adj_stf;    // [step * adj_step + id]
+  long long adj_step;
+  const int *kslot;        // plan order: element of Kmu, Kkappa
+  float *Kmu, *Kkappa, *R;
+};
+
+// Arrays laid one after the other (256-byte boundaries) for one copy.
+struct PatchBlob {
+  std::vector<char> bytes;
+  template <class T> size_t add(const std::vector<T> &v) {
+    const size_t at = (bytes.size() + 255) / 256 * 256;
+    bytes.resize(at + v.size() * sizeof(T));
+    if (!v.empty()) std::memcpy(bytes.data() + at, v.data(), v.size() * sizeof(T));
+    return at;
+  }
+};
 // Device copies of a plan and of what the kernel reads beside it, in three
 // allocations: tables, properties (set again by upload_properties) and the
 // kernel's own buffers.
@@ -188,6 +219,10 @@ void launch_patch_step(hipStream_t s, int pe, int npatch, int nrec, bool exact, 
 // corrector and predictor into state A (a too with store_a), else a only.
 void launch_patch_boundary(hipStream_t s, bool exact, const PatchTables &t, const PatchState &st, NewmarkConst nc,
                            int rd, int advance, int store_a);
+void launch_patch_pair(hipStream_t s, int pe, int npatch, int nrec, const PatchTables &t, const PatchState &adj,
+                       const PatchState &bwd, const GllConst &q, const PatchPairLaunch &l, const PatchPairTables &p);
+void launch_patch_pair_boundary(hipStream_t s, const PatchTables &t, const PatchState &adj, const PatchState &bwd,
+                                NewmarkConst nc, int rd, float *R);
 // dst[i] = src[index[i]] / dst[index[i]] = src[i]
 void launch_take(hipStream_t s, int n, const int *index, const float *src, float *dst);
 void launch_put(hipStream_t s, int n, const int *index, const float *src, float *dst);

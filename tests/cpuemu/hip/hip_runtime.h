@@ -30,6 +30,7 @@ struct float4 { float x, y, z, w; };
 struct float2 { float x, y; };
 inline float4 make_float4(float a, float b, float c, float d) { return float4{a, b, c, d}; }
 inline float2 make_float2(float a, float b) { return float2{a, b}; }
+struct int2 { int x, y; };
 struct int4 { int x, y, z, w; };
 inline int4 make_int4(int a, int b, int c, int d) { return int4{a, b, c, d}; }
 struct uint4 { unsigned x, y, z, w; };
