@@ -147,6 +147,12 @@ struct sfx_engine {
   // inverse; nglob_ac_pad each), per-point tables in slot order, the
   // interface entries, and the sources and receivers of each medium
   DevBuf<float> ac_fields, rho_inv, ac_stacey;
+  // their contributions and every point's list of them (colored scatter)
+  DevBuf<float> cpl_re, cpl_dd;
+  DevBuf<uint32_t> cpl_ent, cpl_list;
+  DevBuf<int> cpl_off;
+  CoupledStep cpl{};
+  bool coupled_sums = false;
   DevBuf<int> ac_dirichlet, cpl_ac_self, cpl_ac_other, cpl_el_self, cpl_el_other, src_order_ac, rec_el, rec_ac;
   DevBuf<float> cpl_ac_coef, cpl_el_coef;
   int nsrc_order_el = 0;
@@ -482,6 +488,86 @@ struct sfx_engine {
                              bnd_rvs.p, re3.p);
   }
 
+  // Contributions of every point of a mesh with acoustic elements, in the order
+  // the color launches add them: interface entries, sources, elements in slot
+  // order, Stacey entries.  Meshes beyond 30-bit indices keep the color launches.
+  void upload_coupled(hipStream_t s) {
+    const size_t nb = h.bnd_gather.size(), nci = h.cpl_ac_self.size(), nce = h.cpl_el_self.size();
+    const size_t nel = h.color_offsets[h.ncolors_el], nac = h.nspec - nel, nse = h.src_order_el.size(),
+                 nsa = h.src_order_ac.size();
+    const size_t src_el = 50 * nel, bnd = src_el + 50 * nse, ac = bnd + 50 * ((nb + 24) / 25), src_ac = ac + 25 * nac,
+                 cpi = src_ac + 25 * nsa, total = cpi + nci;
+    coupled_sums = run.scatter == SFX_SCATTER_COLORED && total < CONTRIB_NONE && nce < CONTRIB_NONE;
+    if (!coupled_sums) return;
+    // points: elastic ones, then acoustic ones
+    const size_t np = static_cast<size_t>(h.nglob_el) + h.nglob_ac;
+    auto each = [&](auto &&put) {
+      auto put_ac = [&](size_t g, size_t o) { put(h.nglob_el + g, static_cast<uint32_t>(o)); };
+      for (size_t k = 0; k < nce; k++) put(h.cpl_el_self[k], CONTRIB_TERM | static_cast<uint32_t>(k));
+      for (size_t k = 0; k < nci; k++) put_ac(h.cpl_ac_self[k], cpi + k);
+      for (size_t k = 0; k < nse; k++)
+        for (int p = 0; p < 25; p++)
+          put(h.gather[static_cast<size_t>(h.src_ispec[h.src_order_el[k]]) * 25 + p],
+              static_cast<uint32_t>(src_el + 50 * k + p));
+      for (size_t k = 0; k < nsa; k++)
+        for (int p = 0; p < 25; p++)
+          put_ac(h.gather[static_cast<size_t>(h.src_ispec[h.src_order_ac[k]]) * 25 + p], src_ac + 25 * k + p);
+      for (size_t e = 0; e < nel; e++)
+        for (int p = 0; p < 25; p++)
+          put(h.gather[static_cast<size_t>(h.perm[e]) * 25 + p], static_cast<uint32_t>(50 * e + p));
+      for (size_t e = 0; e < nac; e++)
+        for (int p = 0; p < 25; p++)
+          put_ac(h.gather[static_cast<size_t>(h.perm[nel + e]) * 25 + p], ac + 25 * e + p);
+      for (size_t k = 0; k < nb; k++) put(h.bnd_gather[k], static_cast<uint32_t>(bnd + k / 25 * 50 + k % 25));
+    };
+    std::vector<int> count(np, 0), row(np, -1), off(1, 0);
+    each([&](size_t g, uint32_t) { count[g]++; });
+    int rows = 0;
+    for (size_t g = 0; g < np; g++)
+      if (count[g] > 4) {
+        row[g] = rows++;
+        off.push_back(off.back() + count[g]);
+      }
+    std::vector<uint32_t> ent(4 * np, CONTRIB_NONE), list(off.back());
+    std::fill(count.begin(), count.end(), 0);
+    each([&](size_t g, uint32_t o) {
+      if (row[g] >= 0)
+        list[off[row[g]] + count[g]] = o;
+      else
+        ent[4 * g + count[g]] = o;
+      count[g]++;
+    });
+    for (size_t g = 0; g < np; g++)
+      if (row[g] >= 0) ent[4 * g] = CONTRIB_LIST | static_cast<uint32_t>(row[g]);
+    cpl_ent.upload(ent, s);
+    cpl_list.upload(list, s);
+    cpl_off.upload(off, s);
+    cpl_re.alloc(total);
+    cpl_dd.alloc(h.nglob_ac_pad);
+    launch_fill(s, cpl_dd.p, cpl_dd.n, 0.0f);
+    SFX_HIP(hipStreamSynchronize(s));
+    const auto i32 = [](size_t n) { return static_cast<int>(n); };
+    const auto u32 = [](size_t n) { return static_cast<uint32_t>(n); };
+    const uint4 *rec = reinterpret_cast<const uint4 *>(cpl_ent.p);
+    cpl = CoupledStep{
+        .nel = i32(nel), .nac = i32(nac), .nsrc_el = i32(nse), .nsrc_ac = i32(nsa), .nbnd = i32(nb), .ncpl_ac = i32(nci),
+        .nglob_el = h.nglob_el, .nglob_ac = h.nglob_ac,
+        .gather = gather.p, .pg = PointGeom2D{xix.p, xiz.p, gammax.p, gammaz.p, kappa.p, mu.p}, .jac = jac.p,
+        .rho_inv = rho_inv.p, .ac_stacey = ac_stacey.p, .ac_dirichlet = ac_dirichlet.p,
+        .nsrc = h.nsrc, .order_el = src_order.p, .order_ac = src_order_ac.p, .src_ispec = src_ispec.p,
+        .src_array = src_array.p, .stf = stf.p,
+        .bnd_gather = bnd_gather.p, .bnd_normal = bnd_normal.p, .bnd_weight = bnd_weight.p, .bnd_rvp = bnd_rvp.p,
+        .bnd_rvs = bnd_rvs.p,
+        .ac_other = cpl_ac_other.p, .el_other = cpl_el_other.p, .ac_coef = cpl_ac_coef.p,
+        .el_coef = cpl_el_coef.p,
+        .re = cpl_re.p, .at_src_el = u32(src_el), .at_bnd = u32(bnd), .at_ac = u32(ac), .at_src_ac = u32(src_ac),
+        .at_cpl = u32(cpi),
+        .ent_el = rec, .ent_ac = rec + h.nglob_el, .list_off = cpl_off.p, .list = cpl_list.p, .dd = cpl_dd.p,
+        .nrec_el = i32(h.rec_el.size()), .nrec_ac = i32(h.rec_ac.size()), .nrec = h.nrec, .ntypes = run.nseismo_types,
+        .rec_el = rec_el.p, .rec_ac = rec_ac.p, .types = types.p, .rec_ispec = rec_ispec.p, .rec_h = rec_h.p,
+        .seismo = seismo.p};
+  }
+
   // Stacey entries regrouped for the block path: entry slot = owner * 386 +
   // slot of its point for the block of its element (lattice.hpp), entries
   // sorted (stably) by that slot, one segment per slot.
@@ -642,6 +728,7 @@ struct sfx_engine {
     types.upload(t, s);
     seismo.alloc(static_cast<size_t>(nsig) * run.nseismo_types * h.nrec * h.ncomp);
     if (seismo.n) launch_fill(s, seismo.p, seismo.n, 0.0f);
+    if (h.coupled()) upload_coupled(s);
     const size_t stride = static_cast<size_t>(h.ncomp) * h.nglob_pad;
     fields.alloc(4 * stride);
     launch_fill(s, fields.p, 4 * stride, 0.0f);
@@ -867,6 +954,22 @@ struct sfx_engine {
       // from the corrected chi_dot_dot, seismograms of both media, and the
       // next step's predictors (the elastic one fused with its corrector)
       if (recording) throw std::invalid_argument("adjoint runs are implemented for elastic meshes");
+      if (coupled_sums) {
+        if (istep < 0 || istep >= run.nstep) throw std::invalid_argument("istep out of range");
+        const bool sample = istep % run.nstep_between_samples == 0;
+        const int isig = istep / run.nstep_between_samples;
+        if (sample && isig >= nsig) throw std::invalid_argument("seismogram step out of range");
+        if (evs) SFX_HIP(hipEventRecord(evs[0], stream));
+        if (evs) SFX_HIP(hipEventRecord(evs[1], stream));
+        launch_coupled_forces(stream, cpl, q, istep, ff, fa());
+        if (evs) SFX_HIP(hipEventRecord(evs[2], stream));
+        launch_coupled_acoustic(stream, cpl, fa(), nc);
+        if (sample) launch_coupled_seismograms(stream, cpl, q, isig, ff, fa(), nc.dto2);
+        if (evs) SFX_HIP(hipEventRecord(evs[3], stream));
+        launch_coupled_update(stream, cpl, ff, fa(), nc);
+        if (evs) SFX_HIP(hipEventRecord(evs[4], stream));
+        return;
+      }
       if (evs) SFX_HIP(hipEventRecord(evs[0], stream));
       update_acoustic(istep, 1);
       couple_into_elastic(ff);

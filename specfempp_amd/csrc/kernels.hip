@@ -633,32 +633,6 @@ __global__ __launch_bounds__(128) void sources_kernel(int npe, int nsrc, int ist
 // Seismograms: one block per receiver, Lagrange interpolation of the
 // element field, block reduction.
 // ---------------------------------------------------------------------------
-// Pressure at element point p of 2-D element e (include/medium/dim2/elastic/
-// isotropic/wavefield.hpp:49-85): -(lambda + 2/3 mu) div u from the element's
-// displacement (su, staged in LDS), the per-point derivatives and properties;
-// the factor is formed in double as the reference's double constant makes it.
-__device__ __forceinline__ float pressure_2d(const PointGeom2D &pg, const GllConst &q, const float (*su)[25], int e,
-                                             int p) {
-  const int iz = p / 5, ix = p - (p / 5) * 5;
-  float dxi[2] = {0.0f, 0.0f}, dga[2] = {0.0f, 0.0f};
-#pragma unroll
-  for (int l = 0; l < 5; l++) {
-#pragma unroll
-    for (int c = 0; c < 2; c++) {
-      dxi[c] += q.hp[ix][l] * su[c][iz * 5 + l];
-      dga[c] += q.hp[iz][l] * su[c][l * 5 + ix];
-    }
-  }
-  const size_t idx = static_cast<size_t>(e) * 25 + p;
-  const float du00 = pg.xix[idx] * dxi[0] + pg.gammax[idx] * dga[0];
-  const float du11 = pg.xiz[idx] * dxi[1] + pg.gammaz[idx] * dga[1];
-  const float mu = pg.mu[idx];
-  const float lp2m = pg.kappa[idx] + (4.0f / 3.0f) * mu;
-  const float lambda = lp2m - 2.0f * mu;
-  const double fac = static_cast<double>(lambda) + (2.0 / 3.0) * static_cast<double>(mu);
-  return static_cast<float>(-1.0 * (fac * static_cast<double>(du00 + du11)));
-}
-
 template <int D>
 __global__ __launch_bounds__(128) void seismogram_kernel(int npe, int nrec, int ntypes, const int *__restrict__ types,
                                                          int isig, const int *__restrict__ ispec,

@@ -106,7 +106,7 @@ void launch_sources_re(hipStream_t s, int nsrc, int istep, const int *ispec, con
 void launch_stacey_re(hipStream_t s, int nseg, const int *seg, const int *gather, const int *slot,
                       const float *normal, const float *weight, const float *rho_vp, const float *rho_vs, Fields f,
                       float *re);
-// Both of the above in one launch (one extra block for the sources); only
+// Both of the above in one launch (one extra block per source); only
 // valid when no source element has an absorbing face.
 void launch_stacey_sources_re(hipStream_t s, int nseg, const int *seg, const int *gather, const int *slot,
                               const float *normal, const float *weight, const float *rho_vp, const float *rho_vs,
@@ -175,6 +175,31 @@ void launch_sources(hipStream_t s, int dim, int npe, int nsrc, int istep, const 
 struct PointGeom2D {
   const float *xix, *xiz, *gammax, *gammaz, *kappa, *mu;
 };
+// Pressure at element point p of 2-D element e (include/medium/dim2/elastic/
+// isotropic/wavefield.hpp:49-85): -(lambda + 2/3 mu) div u from the element's
+// displacement (su, staged in LDS), the per-point derivatives and properties;
+// the factor is formed in double as the reference's double constant makes it.
+__device__ __forceinline__ float pressure_2d(const PointGeom2D &pg, const GllConst &q, const float (*su)[25], int e,
+                                             int p) {
+  const int iz = p / 5, ix = p - (p / 5) * 5;
+  float dxi[2] = {0.0f, 0.0f}, dga[2] = {0.0f, 0.0f};
+#pragma unroll
+  for (int l = 0; l < 5; l++) {
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      dxi[c] += q.hp[ix][l] * su[c][iz * 5 + l];
+      dga[c] += q.hp[iz][l] * su[c][l * 5 + ix];
+    }
+  }
+  const size_t idx = static_cast<size_t>(e) * 25 + p;
+  const float du00 = pg.xix[idx] * dxi[0] + pg.gammax[idx] * dga[0];
+  const float du11 = pg.xiz[idx] * dxi[1] + pg.gammaz[idx] * dga[1];
+  const float mu = pg.mu[idx];
+  const float lp2m = pg.kappa[idx] + (4.0f / 3.0f) * mu;
+  const float lambda = lp2m - 2.0f * mu;
+  const double fac = static_cast<double>(lambda) + (2.0 / 3.0) * static_cast<double>(mu);
+  return static_cast<float>(-1.0 * (fac * static_cast<double>(du00 + du11)));
+}
 // corrected = 1: sample the state after the (not yet applied) mass division and
 // corrector of this step, i.e. u, v + dt/2 a M^-1, a M^-1.  Types 0..2
 // displacement, velocity, acceleration; 3 pressure (2-D).
@@ -250,6 +275,55 @@ void launch_coupling_2d(hipStream_t s, int n, const int *self, const int *other,
 // Acoustic sources order[0..norder): a += stf * array / kappa.
 void launch_acoustic_sources(hipStream_t s, int norder, int nsrc, int istep, const int *order, const int *ispec,
                              const int *gather, const float *array, const float *stf, const float *kappa, Fields f);
+// Forward steps of a mesh with both media (colored scatter) without color
+// launches: forces of all elements, sources, Stacey entries and interface
+// points are stored as contributions, which the point kernels sum in the order
+// the color launches add them.
+struct CoupledStep {
+  // elements: elastic slots [0, nel), acoustic slots [nel, nel + nac)
+  int nel, nac, nsrc_el, nsrc_ac, nbnd, ncpl_ac, nglob_el, nglob_ac;
+  const int *gather;
+  PointGeom2D pg;
+  const float *jac, *rho_inv, *ac_stacey;
+  const int *ac_dirichlet;
+  // sources
+  int nsrc;
+  const int *order_el, *order_ac, *src_ispec;
+  const float *src_array, *stf;
+  // Stacey entries of the elastic medium
+  const int *bnd_gather;
+  const float *bnd_normal, *bnd_weight, *bnd_rvp, *bnd_rvs;
+  // interface entries
+  const int *ac_other, *el_other;
+  const float *ac_coef, *el_coef;
+  // contributions, in this order: elastic elements (50 each: component, point),
+  // elastic sources (50 each), Stacey entries (50 per 25), acoustic elements
+  // (25 each), acoustic sources (25 each), interface entries (1 each)
+  float *re;
+  uint32_t at_src_el, at_bnd, at_ac, at_src_ac, at_cpl;
+  // Per point up to four contributions inline (CONTRIB_NONE: absent), or in x
+  // CONTRIB_LIST | row of the longer lists; CONTRIB_TERM | k is interface entry
+  // k of the elastic side.
+  const uint4 *ent_el, *ent_ac;
+  const int *list_off;
+  const uint32_t *list;
+  float *dd;  // chi_dot_dot of the step
+  // receivers
+  int nrec_el, nrec_ac, nrec, ntypes;
+  const int *rec_el, *rec_ac, *types, *rec_ispec;
+  const float *rec_h;
+  float *seismo;
+};
+constexpr uint32_t CONTRIB_TERM = 0x80000000u, CONTRIB_LIST = 0xC0000000u, CONTRIB_INDEX = 0x3FFFFFFFu,
+                   CONTRIB_NONE = 0x3FFFFFFFu;
+// el, ac: the fields of the two media.  Order within a step: forces, acoustic
+// (sums, mass division, corrector), seismograms, update (elastic update fused
+// with the next predictor, acoustic predictor).
+void launch_coupled_forces(hipStream_t s, const CoupledStep &m, const GllConst &q, int istep, Fields el, Fields ac);
+void launch_coupled_acoustic(hipStream_t s, const CoupledStep &m, Fields ac, NewmarkConst nc);
+void launch_coupled_seismograms(hipStream_t s, const CoupledStep &m, const GllConst &q, int isig, Fields el, Fields ac,
+                                float dto2);
+void launch_coupled_update(hipStream_t s, const CoupledStep &m, Fields el, Fields ac, NewmarkConst nc);
 // Seismograms of the receivers list[0..nlist) in acoustic elements.
 void launch_acoustic_seismograms(hipStream_t s, int nlist, const int *list, int nrec, int ntypes, const int *types,
                                  int isig, const int *ispec, const int *gather, const float *h, const float *xix,

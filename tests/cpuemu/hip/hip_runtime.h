@@ -69,6 +69,14 @@ inline float __shfl(float v, int lane, int width = 64) {
   emu::sync();
   return r;
 }
+inline int __syncthreads_or(int x) {
+  emu::shfl_buf[threadIdx.x] = x ? 1.0f : 0.0f;
+  emu::sync();
+  int any = 0;
+  for (unsigned t = 0; t < blockDim.x; t++) any |= emu::shfl_buf[t] != 0.0f;
+  emu::sync();
+  return any;
+}
 inline float unsafeAtomicAdd(float *p, float v) {
   std::lock_guard<std::mutex> g(emu::atom_mu);
   const float old = *p;
