@@ -959,23 +959,31 @@ __global__ __launch_bounds__(128) void elemforce_3d_kernel(Lattice lat, const fl
 // (the order of the 4-point row version below, so both give equal bits).
 __device__ __forceinline__ void assemble_tiled(const Lattice &lat, const float *__restrict__ re, int tx, int ty,
                                                int tz, int i, int j, int k, float acc[3]) {
-  bool first = true;
-  auto add = [&](int ex, int ey, int ez, int slot) {
-    if (ex < 0 || ey < 0 || ez < 0 || ex >= lat.nx || ey >= lat.ny || ez >= lat.nz) return;
-    const float *r = re + ((static_cast<size_t>(ez) * lat.ny + ey) * lat.nx + ex) * RE_ELEM + slot;
+  // every load is issued, absent contributions re-reading element 0's block:
+  // one round trip instead of one per contribution
+  const int dx[8] = {0, 0, 0, 0, 1, 1, 1, 1}, dy[8] = {0, 1, 0, 1, 0, 1, 0, 1}, dz[8] = {0, 0, 1, 1, 0, 0, 1, 1};
+  const int slot[8] = {(k * 4 + j) * 4 + i, 80 + k * 4 + i, 96 + j * 4 + i, 120 + i,
+                       64 + k * 4 + j,      112 + k,        116 + j,        124};
+  bool use[8];
+  float r[8][3];
 #pragma unroll
-    for (int c = 0; c < 3; c++) acc[c] = first ? r[c * RE_STRIDE] : acc[c] + r[c * RE_STRIDE];
-    first = false;
-  };
+  for (int n = 0; n < 8; n++) {
+    const int ex = tx - dx[n], ey = ty - dy[n], ez = tz - dz[n];
+    use[n] = (!dx[n] || i == 0) && (!dy[n] || j == 0) && (!dz[n] || k == 0) && ex >= 0 && ey >= 0 && ez >= 0 &&
+             ex < lat.nx && ey < lat.ny && ez < lat.nz;
+    const size_t e = use[n] ? (static_cast<size_t>(ez) * lat.ny + ey) * lat.nx + ex : 0;
+#pragma unroll
+    for (int c = 0; c < 3; c++) r[n][c] = re[e * RE_ELEM + c * RE_STRIDE + slot[n]];
+  }
+  bool first = true;
   acc[0] = acc[1] = acc[2] = 0.0f;
-  add(tx, ty, tz, (k * 4 + j) * 4 + i);
-  if (j == 0) add(tx, ty - 1, tz, 80 + k * 4 + i);
-  if (k == 0) add(tx, ty, tz - 1, 96 + j * 4 + i);
-  if (j == 0 && k == 0) add(tx, ty - 1, tz - 1, 120 + i);
-  if (i == 0) add(tx - 1, ty, tz, 64 + k * 4 + j);
-  if (i == 0 && j == 0) add(tx - 1, ty - 1, tz, 112 + k);
-  if (i == 0 && k == 0) add(tx - 1, ty, tz - 1, 116 + j);
-  if (i == 0 && j == 0 && k == 0) add(tx - 1, ty - 1, tz - 1, 124);
+#pragma unroll
+  for (int n = 0; n < 8; n++)
+    if (use[n]) {
+#pragma unroll
+      for (int c = 0; c < 3; c++) acc[c] = first ? r[n][c] : acc[c] + r[n][c];
+      first = false;
+    }
 }
 
 // Device slot d -> (tile, local) and whether it is a lattice point.
@@ -1090,25 +1098,37 @@ __global__ __launch_bounds__(256) void assemble_3d_kernel(Lattice lat, const flo
   }
 }
 
-// One thread per element point adds every source in source order: two
-// sources in one element meet in the same thread, so plain adds suffice.
-__device__ __forceinline__ void sources_re_point(int p, int nsrc, int istep, const int *__restrict__ ispec,
+// Source s by one workgroup (of 128 or 256 threads): the workgroup of the first
+// source of an element adds all of that element's sources in source order, a
+// thread per element point, so plain adds suffice; the other workgroups of the
+// element leave.  A latency chain per element instead of one over all sources:
+// 16 sources took 9.5 us in one workgroup, 4.6 us in 16.
+__device__ __forceinline__ void sources_re_block(int s, int nsrc, int istep, const int *__restrict__ ispec,
                                                  const float *__restrict__ array, const float *__restrict__ stf,
                                                  float *__restrict__ re) {
-  const int slot = re_slot(p % 5, (p / 5) % 5, p / 25);
-  for (int s = 0; s < nsrc; s++) {
-    const float sv = stf[static_cast<size_t>(istep) * nsrc + s];
+  const int p = threadIdx.x;
+  const int e = ispec[s];
+  int earlier = 0;
+  for (int k = p; k < s; k += blockDim.x) earlier |= ispec[k] == e;
+  if (__syncthreads_or(earlier) || p >= 125) return;
+  float *own = re + static_cast<size_t>(e) * RE_ELEM + re_slot(p % 5, (p / 5) % 5, p / 25);
+  float r[3];
 #pragma unroll
-    for (int c = 0; c < 3; c++)
-      re[static_cast<size_t>(ispec[s]) * RE_ELEM + c * RE_STRIDE + slot] +=
-          sv * array[(static_cast<size_t>(s) * 3 + c) * 125 + p];
+  for (int c = 0; c < 3; c++) r[c] = own[c * RE_STRIDE];
+  for (int k = s; k < nsrc; k++) {
+    if (ispec[k] != e) continue;
+    const float sv = stf[static_cast<size_t>(istep) * nsrc + k];
+#pragma unroll
+    for (int c = 0; c < 3; c++) r[c] += sv * array[(static_cast<size_t>(k) * 3 + c) * 125 + p];
   }
+#pragma unroll
+  for (int c = 0; c < 3; c++) own[c * RE_STRIDE] = r[c];
 }
 
 __global__ __launch_bounds__(128) void sources_re_kernel(int nsrc, int istep, const int *__restrict__ ispec,
                                                          const float *__restrict__ array,
                                                          const float *__restrict__ stf, float *__restrict__ re) {
-  if (threadIdx.x < 125) sources_re_point(threadIdx.x, nsrc, istep, ispec, array, stf, re);
+  sources_re_block(blockIdx.x, nsrc, istep, ispec, array, stf, re);
 }
 
 // Seismogram samples of receiver r by one workgroup (its first 125 threads
@@ -1122,50 +1142,48 @@ __device__ __forceinline__ void seismogram_re_block(int r, Lattice lat, int nrec
   const int p = threadIdx.x;
   const int np = f.nglob_pad;
   float hw = 0.0f;
-  int L = 0;
-  float acc[3] = {0, 0, 0};
+  float u[3] = {0, 0, 0}, v[3] = {0, 0, 0}, a[3] = {0, 0, 0};
   if (p < 125) {
     const int e = ispec[r];
     const int ex = e % lat.nx, ey = (e / lat.nx) % lat.ny, ez = e / (lat.nx * lat.ny);
     const int i = p % 5, j = (p / 5) % 5, k = p / 25;
-    L = tiled_index(lat, ex, ey, ez, i, j, k);
+    const int L = tiled_index(lat, ex, ey, ez, i, j, k);
     hw = h[static_cast<size_t>(r) * 125 + p];
+    float m[3] = {0, 0, 0};
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+      const size_t o = static_cast<size_t>(c) * np + L;
+      u[c] = f.u[o];
+      if (need_a) {
+        v[c] = f.v[o];
+        m[c] = f.minv[o];
+      }
+    }
     // the assembled acceleration only for velocity and acceleration traces
-    if (need_a) assemble_tiled(lat, re, ex + (i >> 2), ey + (j >> 2), ez + (k >> 2), i & 3, j & 3, k & 3, acc);
+    if (need_a) {
+      assemble_tiled(lat, re, ex + (i >> 2), ey + (j >> 2), ez + (k >> 2), i & 3, j & 3, k & 3, a);
+#pragma unroll
+      for (int c = 0; c < 3; c++) a[c] = a[c] * m[c];
+    }
   }
   for (int it = 0; it < ntypes; it++) {
-    const int type = types[it];
-    float val[3];
+    const int row = types[it] < 2 ? types[it] : 2;
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-      float x = 0.0f;
-      if (p < 125) {
-        const size_t o = static_cast<size_t>(c) * np + L;
-        if (type == 0) {
-          x = f.u[o];
-        } else {
-          const float a = acc[c] * f.minv[o];
-          x = type == 1 ? f.v[o] + dto2 * a : a;
-        }
-      }
-      val[c] = hw * x;
-    }
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-      float s = val[c];
+      const float x = row == 0 ? u[c] : row == 1 ? v[c] + dto2 * a[c] : a[c];
+      float s = hw * x;
 #pragma unroll
       for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
       // the 125 points are in the first two waves; later waves hold zeros
-      if ((p & 63) == 0 && p < 128) red[c][p >> 6] = s;
+      if ((p & 63) == 0 && p < 128) red[row * 3 + c][p >> 6] = s;
     }
-    __syncthreads();
-    if (p == 0) {
-#pragma unroll
-      for (int c = 0; c < 3; c++)
-        seismo[((static_cast<size_t>(isig) * ntypes + it) * nrec + r) * 3 + c] = red[c][0] + red[c][1];
-    }
-    __syncthreads();
   }
+  __syncthreads();
+  if (p < 3)
+    for (int it = 0; it < ntypes; it++) {
+      const int row = (types[it] < 2 ? types[it] : 2) * 3 + p;
+      seismo[((static_cast<size_t>(isig) * ntypes + it) * nrec + r) * 3 + p] = red[row][0] + red[row][1];
+    }
 }
 
 // One thread per element point on the absorbing boundary; its entries (one per
@@ -1186,18 +1204,18 @@ __global__ __launch_bounds__(256) void stacey_re_kernel(int nseg, const int *__r
                                                         const int *__restrict__ rec_ispec,
                                                         const float *__restrict__ rec_h, float dto2,
                                                         float *__restrict__ seismo) {
-  // after the Stacey blocks: one block adding the sources (only launched so
+  // after the Stacey blocks: one block per source (only launched so
   // when no source element has an absorbing face: the two touch disjoint
   // entries), then one block per receiver for displacement traces, which read
   // only u
   if (seis_first >= 0 && static_cast<int>(blockIdx.x) >= seis_first) {
-    __shared__ float red[3][2];
+    __shared__ float red[9][2];
     seismogram_re_block(blockIdx.x - seis_first, lat, nrec, ntypes, types, isig, rec_ispec, rec_h, re, f, dto2,
                         seismo, 0, red);
     return;
   }
-  if (static_cast<int>(blockIdx.x) == src_block) {
-    if (threadIdx.x < 125) sources_re_point(threadIdx.x, nsrc, istep, src_ispec, src_array, stf, re);
+  if (src_block >= 0 && static_cast<int>(blockIdx.x) >= src_block) {
+    sources_re_block(blockIdx.x - src_block, nsrc, istep, src_ispec, src_array, stf, re);
     return;
   }
   const int sidx = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1238,7 +1256,7 @@ __global__ __launch_bounds__(128) void seismogram_re_kernel(Lattice lat, int nre
                                                             const float *__restrict__ h,
                                                             const float *__restrict__ re, Fields f, float dto2,
                                                             float *__restrict__ seismo, int need_a) {
-  __shared__ float red[3][2];
+  __shared__ float red[9][2];
   seismogram_re_block(blockIdx.x, lat, nrec, ntypes, types, isig, ispec, h, re, f, dto2, seismo, need_a, red);
 }
 
@@ -1462,7 +1480,7 @@ void launch_elemforce_3d(hipStream_t s, Lattice lat, const float *kappa, const f
 void launch_sources_re(hipStream_t s, int nsrc, int istep, const int *ispec, const float *array, const float *stf,
                        float *re) {
   if (nsrc <= 0) return;
-  hipLaunchKernelGGL(sources_re_kernel, dim3(1), dim3(128), 0, s, nsrc, istep, ispec, array, stf, re);
+  hipLaunchKernelGGL(sources_re_kernel, dim3(nsrc), dim3(128), 0, s, nsrc, istep, ispec, array, stf, re);
 }
 
 void launch_stacey_re(hipStream_t s, int nseg, const int *seg, const int *gather, const int *slot,
@@ -1483,7 +1501,7 @@ void launch_stacey_sources_re(hipStream_t s, int nseg, const int *seg, const int
   }
   const int nb = static_cast<int>(blocks(nseg, 256));
   const int src_block = nsrc > 0 ? nb : -1;
-  hipLaunchKernelGGL(stacey_re_kernel, dim3(nb + (nsrc > 0 ? 1 : 0)), dim3(256), 0, s, nseg, seg, gather, slot,
+  hipLaunchKernelGGL(stacey_re_kernel, dim3(nb + (nsrc > 0 ? nsrc : 0)), dim3(256), 0, s, nseg, seg, gather, slot,
                      normal, weight, rho_vp, rho_vs, f, re, src_block, nsrc, istep, src_ispec, src_array, stf, -1,
                      Lattice{}, 0, 0, nullptr, 0, nullptr, nullptr, 0.0f, nullptr);
 }
@@ -1495,7 +1513,7 @@ void launch_stacey_sources_seismo_re(hipStream_t s, int nseg, const int *seg, co
                                      float dto2, float *seismo) {
   const int nb = nseg > 0 ? static_cast<int>(blocks(nseg, 256)) : 0;
   const int src_block = nsrc > 0 ? nb : -1;
-  const int seis_first = nb + (nsrc > 0 ? 1 : 0);
+  const int seis_first = nb + (nsrc > 0 ? nsrc : 0);
   const int nrec_blocks = nrec > 0 && ntypes > 0 ? nrec : 0;
   if (seis_first + nrec_blocks == 0) return;
   hipLaunchKernelGGL(stacey_re_kernel, dim3(seis_first + nrec_blocks), dim3(256), 0, s, nseg, seg, gather, slot,
