@@ -6,7 +6,6 @@
 #include <cmath>
 #include <cstring>
 #include <numeric>
-#include <unordered_map>
 
 #include "../../include/specfempp_amd.h"
 
@@ -73,6 +72,18 @@ struct Bisection {
   }
 };
 
+// FNV-1a over 64-bit words of the values
+uint64_t hash_of(const std::vector<uint16_t> &v) {
+  uint64_t h = 0xcbf29ce484222325ull ^ v.size();
+  for (size_t i = 0; i < v.size(); i += 4) {
+    uint64_t w = 0;
+    std::memcpy(&w, &v[i], std::min<size_t>(4, v.size() - i) * 2);
+    h = (h ^ w) * 0x100000001b3ull;
+    h ^= h >> 29;
+  }
+  return h;
+}
+
 }  // namespace
 
 // Small patches while large ones would leave compute units without a
@@ -98,8 +109,6 @@ void add_patches(PatchPlan &plan, const HostAssembly &h, const std::vector<int32
   bis.split(0, ns, (ns + target - 1) / target);
   std::vector<std::pair<int, int>> groups = std::move(bis.out);
 
-  std::vector<int32_t> count(ng, 0);
-  for (size_t i = 0; i < static_cast<size_t>(ns) * npe; i++) count[h.gather[i]]++;
   // colored: the points of each element that have a Stacey term, and all of
   // an element with sources, have one more contribution each
   std::vector<int32_t> src_rank(colored ? ns : 0, -1);
@@ -112,127 +121,145 @@ void add_patches(PatchPlan &plan, const HostAssembly &h, const std::vector<int32
   if (colored) {
     for (int32_t q : h.bnd_slot) edge[q / npe].push_back(static_cast<uint8_t>(q % npe));
     for (int e = 0; e < ns; e++) {
-      if (src_rank[e] >= 0)
-        for (int p = 0; p < npe; p++) count[h.gather[static_cast<size_t>(e) * npe + p]]++;
       std::sort(edge[e].begin(), edge[e].end());
       edge[e].erase(std::unique(edge[e].begin(), edge[e].end()), edge[e].end());
-      for (uint8_t p : edge[e]) count[h.gather[static_cast<size_t>(e) * npe + p]]++;
     }
   }
   // boundary points, and the groups cut again until every one fits the
   // kernel's arrays (compact groups fit at once)
-  std::vector<int32_t> first(ng), stamp(ng);
-  std::vector<char> shared;
+  struct Point {
+    int32_t first, last;  // patches that visit it
+    int32_t count;        // contributions
+    int32_t shared;       // 1: a boundary point; index among a patch's visits
+  };
+  std::vector<Point> point(ng);
+  std::vector<char> shared(ng);
   for (;;) {
-    std::fill(first.begin(), first.end(), -1);
-    shared.assign(ng, 0);
-    for (size_t k = 0; k < groups.size(); k++)
-      for (int i = groups[k].first; i < groups[k].second; i++)
-        for (int p = 0; p < npe; p++) {
-          const int g = h.gather[static_cast<size_t>(order[i]) * npe + p];
-          if (first[g] < 0)
-            first[g] = static_cast<int32_t>(k);
-          else if (first[g] != static_cast<int32_t>(k))
-            shared[g] = 1;
-        }
-    std::fill(stamp.begin(), stamp.end(), -1);
-    std::vector<std::pair<int, int>> next;
-    bool again = false;
+    std::fill(point.begin(), point.end(), Point{-1, -1, 0, 0});
+    std::vector<int> npt(groups.size(), 0), nbd(groups.size(), 0), extra(groups.size(), 0);
     for (size_t k = 0; k < groups.size(); k++) {
-      int pts = 0, bnd = 0, extra = 0;
-      for (int i = groups[k].first; i < groups[k].second; i++)
+      const int32_t patch = static_cast<int32_t>(k);
+      for (int i = groups[k].first; i < groups[k].second; i++) {
+        if (colored) extra[k] += static_cast<int>(edge[order[i]].size()) + (src_rank[order[i]] >= 0 ? npe : 0);
+        const int32_t *ge = &h.gather[static_cast<size_t>(order[i]) * npe];
         for (int p = 0; p < npe; p++) {
-          if (colored && p == 0)
-            extra += static_cast<int>(edge[order[i]].size()) + (src_rank[order[i]] >= 0 ? npe : 0);
-          const int g = h.gather[static_cast<size_t>(order[i]) * npe + p];
-          if (stamp[g] == static_cast<int32_t>(k)) continue;
-          stamp[g] = static_cast<int32_t>(k);
-          pts++;
-          bnd += shared[g];
+          Point &x = point[ge[p]];
+          x.count++;
+          if (x.last == patch) continue;
+          x.last = patch;
+          npt[k]++;
+          if (x.first < 0) {
+            x.first = patch;
+            continue;
+          }
+          nbd[x.first] += !x.shared;
+          x.shared = 1;
+          nbd[k]++;
         }
-      if (pts > point_cap(pe) || bnd > boundary_cap(pe) || extra > pe * npe) {
+      }
+    }
+    std::vector<std::pair<int, int>> next;
+    for (size_t k = 0; k < groups.size(); k++)
+      if (npt[k] > point_cap(pe) || nbd[k] > boundary_cap(pe) || extra[k] > pe * npe) {
         const int m = bis.cut(groups[k].first, groups[k].second, (groups[k].second - groups[k].first) / 2);
         next.push_back({groups[k].first, m});
         next.push_back({m, groups[k].second});
-        again = true;
       } else {
         next.push_back(groups[k]);
       }
-    }
-    if (!again) break;
+    if (next.size() == groups.size()) break;
     groups = std::move(next);
   }
+  for (int g = 0; g < ng; g++) {
+    shared[g] = static_cast<char>(point[g].shared);
+    point[g].last = -1;
+  }
+  if (colored)
+    for (int e = 0; e < ns; e++) {
+      if (src_rank[e] >= 0)
+        for (int p = 0; p < npe; p++) point[h.gather[static_cast<size_t>(e) * npe + p]].count++;
+      for (uint8_t p : edge[e]) point[h.gather[static_cast<size_t>(e) * npe + p]].count++;
+    }
 
   // numbering: interior points patch by patch (by number of contributions,
   // then first visit), boundary points by first visit over the patches
-  std::vector<int32_t> local(ng, -1), dev(ng, -1);
+  std::vector<int32_t> dev(ng, -1);
   std::vector<int32_t> slot(ns);
   const int b_base = plan.nbnd;
-  std::unordered_multimap<size_t, int> seen;  // hash of a patch's tables -> a patch that has them
-  for (int k : plan.lead) seen.emplace(static_cast<uint32_t>(plan.head[k].pad[0]), k);
   // per boundary point: its contributions as (key, plan element, point)
   struct Entry {
     int32_t b, key, where;  // where: index into plan.bslot
   };
   std::vector<Entry> entries;
-  std::vector<uint16_t> t, cat;
+  std::vector<uint16_t> t, cat, bidx;
   std::vector<int> by, at, pos, seg, seg_key, lead;
-  std::vector<int32_t> pts[3], bnd;
-  for (const auto &gr : groups) {
+  std::vector<int32_t> visit;     // points of the patch, in the order of their first visit
+  std::vector<uint16_t> visited;  // index into it of each element point
+  std::vector<uint16_t> number;   // local number of each
+  plan.elem.reserve(plan.elem.size() + ns);
+  plan.head.reserve(plan.head.size() + groups.size());
+  for (size_t k = 0; k < groups.size(); k++) {
+    const auto &gr = groups[k];
+    const int32_t patch = static_cast<int32_t>(k);
     std::sort(order.begin() + gr.first, order.begin() + gr.second);
     PatchHead hd{};
     hd.el0 = static_cast<int>(plan.elem.size());
     hd.nel = gr.second - gr.first;
     hd.sim = mesh;
     const int32_t *el = &order[gr.first];
-    for (auto *v : {&pts[0], &pts[1], &pts[2], &bnd}) v->clear();
+    visit.clear();
+    visited.resize(static_cast<size_t>(hd.nel) * npe);
+    int n[4] = {0, 0, 0, 0};  // points with one, two and more contributions, boundary points
+    auto cls = [](const Point &x) { return x.first < 0 ? 3 : x.count == 1 ? 0 : x.count == 2 ? 1 : 2; };
     for (int i = 0; i < hd.nel; i++) {
       slot[el[i]] = static_cast<int32_t>(plan.elem.size());
       plan.elem.push_back(el[i]);
+      const int32_t *ge = &h.gather[static_cast<size_t>(el[i]) * npe];
       for (int p = 0; p < npe; p++) {
-        const int g = h.gather[static_cast<size_t>(el[i]) * npe + p];
-        if (local[g] == -2 - hd.el0) continue;
-        local[g] = -2 - hd.el0;  // visited by this patch
-        if (shared[g])
-          bnd.push_back(g);
-        else
-          pts[count[g] == 1 ? 0 : count[g] == 2 ? 1 : 2].push_back(g);
+        Point &x = point[ge[p]];
+        if (x.last != patch) {
+          x.last = patch;
+          if (shared[ge[p]]) x.first = -1;
+          x.shared = static_cast<int32_t>(visit.size());
+          visit.push_back(ge[p]);
+          n[cls(x)]++;
+        }
+        visited[static_cast<size_t>(i) * npe + p] = static_cast<uint16_t>(x.shared);
       }
     }
     hd.pt0 = plan.nint;
-    hd.n1 = static_cast<int>(pts[0].size());
-    hd.n2 = static_cast<int>(pts[1].size());
-    hd.nint = hd.n1 + hd.n2 + static_cast<int>(pts[2].size());
-    hd.nb = static_cast<int>(bnd.size());
+    hd.n1 = n[0];
+    hd.n2 = n[1];
+    hd.nint = n[0] + n[1] + n[2];
+    hd.nb = n[3];
     hd.b0 = static_cast<int>(plan.bpt.size());
-    int l = 0;
-    for (auto &cls : pts)
-      for (int g : cls) {
-        dev[g] = plan.nint++;
-        local[g] = l++;
+    const int l = static_cast<int>(visit.size());
+    number.resize(l);
+    int at_cls[4] = {0, hd.n1, hd.n1 + hd.n2, hd.nint};
+    for (int v = 0; v < l; v++) {
+      const int g = visit[v], c = cls(point[g]);
+      number[v] = static_cast<uint16_t>(at_cls[c]++);
+      if (c < 3) {
+        dev[g] = plan.nint + number[v];
+        continue;
       }
-    for (int g : bnd) {
       int32_t owner = 0;
       if (dev[g] < 0) {
         dev[g] = plan.nbnd++;
         owner = INT32_MIN;
       }
       plan.bpt.push_back({owner | dev[g], 0, 0, 0});
-      local[g] = l++;
     }
+    plan.nint += hd.nint;
     // 16-bit tables: rows, then the contributions of every local point in key
     // order (cat[at[l] .. at[l + 1]) of local point l)
     t.assign(static_cast<size_t>(hd.nel) * 40, 0);
+    for (int i = 0; i < hd.nel; i++)
+      for (int p = 0; p < npe; p++)
+        t[static_cast<size_t>(i) * 40 + p / 5 * 8 + p % 5] = number[visited[static_cast<size_t>(i) * npe + p]];
     by.resize(hd.nel);
     std::iota(by.begin(), by.end(), 0);
-    std::stable_sort(by.begin(), by.end(), [&](int a, int b) { return key[el[a]] < key[el[b]]; });
-    at.assign(l + 1, 0);
-    for (int i = 0; i < hd.nel; i++)
-      for (int p = 0; p < npe; p++) {
-        const int lp = local[h.gather[static_cast<size_t>(el[i]) * npe + p]];
-        t[static_cast<size_t>(i) * 40 + p / 5 * 8 + p % 5] = static_cast<uint16_t>(lp);
-        at[lp + 1]++;
-      }
+    std::sort(by.begin(), by.end(), [&](int a, int b) { return key[el[a]] != key[el[b]] ? key[el[a]] < key[el[b]] : a < b; });
     seg.clear();
     if (colored)
       for (int i = 0; i < hd.nel; i++)
@@ -240,7 +267,6 @@ void add_patches(PatchPlan &plan, const HostAssembly &h, const std::vector<int32
           seg.push_back(t[static_cast<size_t>(i) * 40 + p / 5 * 8 + p % 5]);
           seg_key.resize(seg.size());
           seg_key[seg.size() - 1] = ns + el[i];
-          at[seg.back() + 1]++;
         }
     // sources first (by element, in application order), Stacey terms last
     lead.clear();
@@ -248,71 +274,103 @@ void add_patches(PatchPlan &plan, const HostAssembly &h, const std::vector<int32
       for (int i = 0; i < hd.nel; i++)
         if (src_rank[el[i]] >= 0) lead.push_back(i);
     std::sort(lead.begin(), lead.end(), [&](int a, int b) { return src_rank[el[a]] < src_rank[el[b]]; });
-    for (int i : lead)
-      for (int p = 0; p < npe; p++) at[t[static_cast<size_t>(i) * 40 + p / 5 * 8 + p % 5] + 1]++;
     const int extra = pe * npe, src0 = extra + static_cast<int>(seg.size());
-    for (int i = 0; i < l; i++) at[i + 1] += at[i];
-    cat.resize(at[l]);
-    pos.assign(at.begin(), at.end() - 1);
-    for (size_t k = 0; k < lead.size(); k++)
-      for (int p = 0; p < npe; p++)
-        cat[pos[t[static_cast<size_t>(lead[k]) * 40 + p / 5 * 8 + p % 5]]++] = static_cast<uint16_t>(src0 + k * npe + p);
-    for (int i : by)
-      for (int p = 0; p < npe; p++)
-        cat[pos[t[static_cast<size_t>(i) * 40 + p / 5 * 8 + p % 5]]++] = static_cast<uint16_t>(i * npe + p);
-    for (size_t i = 0; i < seg.size(); i++) cat[pos[seg[i]]++] = static_cast<uint16_t>(extra + i);
-    auto mark = [&] { return static_cast<int>(t.size()); };
-    hd.enta = mark();
-    for (int i = 0; i < hd.nint; i++) t.push_back(cat[at[i]]);
-    hd.entb = mark();
-    for (int i = hd.n1; i < hd.nint; i++) t.push_back(cat[at[i] + 1]);
-    hd.off3 = mark();
-    uint16_t o3 = 0;
-    for (int i = hd.n1 + hd.n2; i < hd.nint; i++) {
-      t.push_back(o3);
-      o3 = static_cast<uint16_t>(o3 + at[i + 1] - at[i] - 2);
+    // Patches of equal connectivity share their tables.  These follow from the
+    // rows, the order of the elements and the additional contributions: a patch
+    // for which all of that has been seen takes them as they are.
+    std::vector<uint16_t> sig(t);
+    sig.insert(sig.end(), by.begin(), by.end());
+    for (const auto *v : {&seg, &lead}) {
+      sig.push_back(static_cast<uint16_t>(v->size()));
+      sig.insert(sig.end(), v->begin(), v->end());
     }
-    t.push_back(o3);
-    hd.ent3 = mark();
-    for (int i = hd.n1 + hd.n2; i < hd.nint; i++) t.insert(t.end(), cat.begin() + at[i] + 2, cat.begin() + at[i + 1]);
-    hd.bent = mark();
-    hd.be0 = static_cast<int>(plan.bslot.size());
-    for (int i = hd.nint; i < l; i++)
-      for (int j = at[i]; j < at[i + 1]; j++) {
-        t.push_back(cat[j]);
-        const int c = cat[j];
-        const int32_t k = c < extra  ? key[el[c / npe]]
-                          : c < src0 ? seg_key[c - extra]
-                                     : src_rank[el[lead[(c - src0) / npe]]] - static_cast<int32_t>(h.src_order.size());
-        entries.push_back({dev[bnd[i - hd.nint]], k, static_cast<int32_t>(plan.bslot.size())});
-        plan.bslot.push_back(0);
-        hd.nbent++;
+    for (int v : {hd.nel, hd.n1, hd.n2, hd.nint, l}) sig.push_back(static_cast<uint16_t>(v));
+    const uint64_t sig_hash = hash_of(sig);
+    const PatchPlan::Tables *same = nullptr;
+    for (auto it = plan.by_shape.equal_range(sig_hash); it.first != it.second && !same; ++it.first)
+      if (plan.tables[it.first->second].sig == sig) same = &plan.tables[it.first->second];
+    if (!same) {
+      at.assign(l + 1, 0);
+      for (int i = 0; i < hd.nel; i++)
+        for (int p = 0; p < npe; p++) at[t[static_cast<size_t>(i) * 40 + p / 5 * 8 + p % 5] + 1]++;
+      for (int v : seg) at[v + 1]++;
+      for (int i : lead)
+        for (int p = 0; p < npe; p++) at[t[static_cast<size_t>(i) * 40 + p / 5 * 8 + p % 5] + 1]++;
+      for (int i = 0; i < l; i++) at[i + 1] += at[i];
+      cat.resize(at[l]);
+      pos.assign(at.begin(), at.end() - 1);
+      for (size_t i = 0; i < lead.size(); i++)
+        for (int p = 0; p < npe; p++)
+          cat[pos[t[static_cast<size_t>(lead[i]) * 40 + p / 5 * 8 + p % 5]]++] =
+              static_cast<uint16_t>(src0 + i * npe + p);
+      for (int i : by)
+        for (int p = 0; p < npe; p++)
+          cat[pos[t[static_cast<size_t>(i) * 40 + p / 5 * 8 + p % 5]]++] = static_cast<uint16_t>(i * npe + p);
+      for (size_t i = 0; i < seg.size(); i++) cat[pos[seg[i]]++] = static_cast<uint16_t>(extra + i);
+      PatchPlan::Tables made;
+      auto mark = [&] { return static_cast<int>(t.size()); };
+      made.enta = mark();
+      for (int i = 0; i < hd.nint; i++) t.push_back(cat[at[i]]);
+      made.entb = mark();
+      for (int i = hd.n1; i < hd.nint; i++) t.push_back(cat[at[i] + 1]);
+      made.off3 = mark();
+      uint16_t o3 = 0;
+      for (int i = hd.n1 + hd.n2; i < hd.nint; i++) {
+        t.push_back(o3);
+        o3 = static_cast<uint16_t>(o3 + at[i + 1] - at[i] - 2);
       }
-    // patches of equal connectivity share their tables
-    uint64_t mix = 0xcbf29ce484222325ull;  // FNV-1a over the table's words
-    for (uint16_t v : t) mix = (mix ^ v) * 0x100000001b3ull;
-    const size_t hash = mix >> 32;
-    const PatchHead *same = nullptr;
-    const auto range = seen.equal_range(hash);
-    for (auto it = range.first; it != range.second && !same; ++it) {
-      const PatchHead &o = plan.head[it->second];
-      if (o.enta - o.lidx == hd.enta && o.entb - o.lidx == hd.entb && o.off3 - o.lidx == hd.off3 &&
-          o.ent3 - o.lidx == hd.ent3 && o.bent - o.lidx == hd.bent && o.nbent == hd.nbent &&
-          std::memcmp(&plan.tab[o.lidx], t.data(), t.size() * 2) == 0)
-        same = &o;
+      t.push_back(o3);
+      made.ent3 = mark();
+      for (int i = hd.n1 + hd.n2; i < hd.nint; i++)
+        t.insert(t.end(), cat.begin() + at[i] + 2, cat.begin() + at[i + 1]);
+      made.bent = mark();
+      for (int i = hd.nint; i < l; i++)
+        for (int j = at[i]; j < at[i + 1]; j++) {
+          t.push_back(cat[j]);
+          made.bidx.push_back(static_cast<uint16_t>(i - hd.nint));
+        }
+      // another order of the elements can give the same tables
+      made.size = t.size();
+      const uint64_t hash = hash_of(t);
+      const PatchPlan::Tables *equal = nullptr;
+      for (auto it = plan.by_tables.equal_range(hash); it.first != it.second && !equal; ++it.first) {
+        const PatchPlan::Tables &o = plan.tables[it.first->second];
+        if (o.enta == made.enta && o.entb == made.entb && o.off3 == made.off3 && o.ent3 == made.ent3 &&
+            o.bent == made.bent && o.bidx == made.bidx && o.size == t.size() &&
+            std::memcmp(&plan.tab[o.base], t.data(), t.size() * 2) == 0)
+          equal = &o;
+      }
+      const int row = static_cast<int>(plan.tables.size());
+      if (equal) {
+        made.base = equal->base;
+      } else {
+        plan.tab.resize((plan.tab.size() + 7) / 8 * 8, 0);  // rows are read 16 bytes at a time
+        made.base = static_cast<int>(plan.tab.size());
+        plan.tab.insert(plan.tab.end(), t.begin(), t.end());
+        plan.by_tables.emplace(hash, row);
+      }
+      made.sig = std::move(sig);
+      plan.tables.push_back(std::move(made));
+      plan.by_shape.emplace(sig_hash, row);
+      same = &plan.tables.back();
     }
-    int base;
-    if (same) {
-      base = same->lidx;
-    } else {
-      plan.tab.resize((plan.tab.size() + 7) / 8 * 8, 0);  // rows are read 16 bytes at a time
-      base = static_cast<int>(plan.tab.size());
-      plan.tab.insert(plan.tab.end(), t.begin(), t.end());
-      plan.lead.push_back(static_cast<int>(plan.head.size()));
-      seen.emplace(hash, static_cast<int>(plan.head.size()));
+    hd.lidx = same->base;
+    hd.enta = same->base + same->enta;
+    hd.entb = same->base + same->entb;
+    hd.off3 = same->base + same->off3;
+    hd.ent3 = same->base + same->ent3;
+    hd.bent = same->base + same->bent;
+    hd.nbent = static_cast<int>(same->bidx.size());
+    hd.be0 = static_cast<int>(plan.bslot.size());
+    for (int j = 0; j < hd.nbent; j++) {
+      const int c = plan.tab[static_cast<size_t>(hd.bent) + j];
+      const int32_t order_key = c < extra  ? key[el[c / npe]]
+                                : c < src0 ? seg_key[c - extra]
+                                           : src_rank[el[lead[(c - src0) / npe]]] - static_cast<int32_t>(h.src_order.size());
+      const int32_t b = plan.bpt[static_cast<size_t>(hd.b0) + same->bidx[j]].b & 0x7fffffff;
+      entries.push_back({b, order_key, static_cast<int32_t>(plan.bslot.size())});
+      plan.bslot.push_back(0);
     }
-    for (int *o : {&hd.lidx, &hd.enta, &hd.entb, &hd.off3, &hd.ent3, &hd.bent}) *o += base;
-    hd.pad[0] = static_cast<int>(hash);
     plan.head.push_back(hd);
   }
   if (plan.tab.size() > static_cast<size_t>(INT32_MAX) || plan.bslot.size() > static_cast<size_t>(INT32_MAX))
@@ -329,8 +387,8 @@ void add_patches(PatchPlan &plan, const HostAssembly &h, const std::vector<int32
   }
   if (plan.boff.empty()) plan.boff.push_back(0);
   for (size_t b = 0; b + 1 < off.size(); b++) {
-    std::stable_sort(grouped.begin() + off[b], grouped.begin() + off[b + 1],
-                     [](const Entry &x, const Entry &y) { return x.key < y.key; });
+    for (int32_t i = off[b] + 1; i < off[b + 1]; i++)  // a few entries: insertion
+      for (int32_t j = i; j > off[b] && grouped[j].key < grouped[j - 1].key; j--) std::swap(grouped[j], grouped[j - 1]);
     for (int32_t i = off[b]; i < off[b + 1]; i++) plan.bslot[grouped[i].where] = s_base + i;
     plan.boff.push_back(s_base + off[b + 1]);
   }
@@ -352,6 +410,9 @@ void finish_patches(PatchPlan &plan) {
     for (auto &g : d)
       if (g < 0) g = plan.nint + (-1 - g);
   if (plan.boff.empty()) plan.boff.push_back(0);
+  plan.tables = {};
+  plan.by_shape = {};
+  plan.by_tables = {};
 }
 
 void renumber_points(HostAssembly &h, const PatchPlan &plan) {
@@ -404,9 +465,10 @@ Entries plan_stacey(const PatchPlan &plan, const std::vector<const HostAssembly 
       out.q[fill[plan.slot_of[m][meshes[m]->bnd_slot[q] / 25]]++] = static_cast<int32_t>(q);
   for (const PatchHead &hd : plan.head)
     for (int i = hd.el0; i < hd.el0 + hd.nel; i++)
-      std::stable_sort(out.q.begin() + out.off[i], out.q.begin() + out.off[i + 1], [&](int32_t a, int32_t b) {
-        return meshes[hd.sim]->bnd_slot[a] < meshes[hd.sim]->bnd_slot[b];
-      });
+      if (out.off[i + 1] - out.off[i] > 1)
+        std::stable_sort(out.q.begin() + out.off[i], out.q.begin() + out.off[i + 1], [&](int32_t a, int32_t b) {
+          return meshes[hd.sim]->bnd_slot[a] < meshes[hd.sim]->bnd_slot[b];
+        });
   return out;
 }
 
@@ -591,10 +653,11 @@ void PatchDevice::upload(const PatchPlan &plan, const std::vector<const HostAsse
   }
   const int mode = record ? GEOM2D_RECORD : c4 ? GEOM2D_CTRL4 : c9 ? GEOM2D_CTRL9 : GEOM2D_POINT;
   auto take = [&](const std::vector<float> HostAssembly::*src_v, size_t width) {
-    std::vector<float> v(el.size() * width);
-    for (size_t i = 0; i < el.size(); i++)
-      std::memcpy(&v[i * width], &(el[i].h->*src_v)[el[i].e * width], width * sizeof(float));
-    return b.add(v);
+    const size_t at = b.room(el.size() * width * sizeof(float));
+    char *to = b.bytes.data() + at;
+    for (size_t i = 0; i < el.size(); i++, to += width * sizeof(float))
+      std::memcpy(to, (el[i].h->*src_v).data() + el[i].e * width, width * sizeof(float));
+    return at;
   };
   size_t o_geo[6] = {0, 0, 0, 0, 0, 0};
   if (mode == GEOM2D_RECORD) {

@@ -22,6 +22,7 @@
 
 #include <cstdint>
 #include <cstring>
+#include <unordered_map>
 #include <vector>
 
 #include "assembly.hpp"
@@ -82,7 +83,15 @@ struct PatchPlan {
   std::vector<int32_t> bslot;      // where each patch's boundary contributions go
   int nint = 0, nbnd = 0;          // interior and boundary points
   std::vector<int> patch_end;      // patches of the first k + 1 meshes
-  std::vector<int> lead;           // first patch of each distinct table set
+  // while meshes are added: the distinct tables, found by what they follow from
+  // and by their contents
+  struct Tables {
+    std::vector<uint16_t> sig, bidx;  // bidx: boundary point of each boundary contribution
+    int base = 0, enta = 0, entb = 0, off3 = 0, ent3 = 0, bent = 0;
+    size_t size = 0;
+  };
+  std::vector<Tables> tables;
+  std::unordered_multimap<uint64_t, int> by_shape, by_tables;
   std::vector<std::vector<int32_t>> device_of;  // per mesh: point -> device index (boundary ones offset by nint once finished)
   std::vector<std::vector<int32_t>> slot_of;    // per mesh: element -> position in elem
 };
@@ -182,9 +191,14 @@ struct PatchPairTables {
 // Arrays laid one after the other (256-byte boundaries) for one copy.
 struct PatchBlob {
   std::vector<char> bytes;
-  template <class T> size_t add(const std::vector<T> &v) {
+  size_t room(size_t n) {
     const size_t at = (bytes.size() + 255) / 256 * 256;
-    bytes.resize(at + v.size() * sizeof(T));
+    if (at + n > bytes.capacity()) bytes.reserve(2 * (at + n));
+    bytes.resize(at + n);
+    return at;
+  }
+  template <class T> size_t add(const std::vector<T> &v) {
+    const size_t at = room(v.size() * sizeof(T));
     if (!v.empty()) std::memcpy(bytes.data() + at, v.data(), v.size() * sizeof(T));
     return at;
   }
