@@ -67,12 +67,12 @@ __global__ __launch_bounds__(128) void acoustic_stiffness_2d_kernel(
     }
     const float xix = xix_[idx], xiz = xiz_[idx], gammax = gammax_[idx], gammaz = gammaz_[idx], J = jac_[idx];
     const float ri = rho_inv_[idx];
-    const float du0 = xix * dxi + gammax * dga;
-    const float du1 = xiz * dxi + gammaz * dga;
+    const float du0 = fmaf(xix, dxi, gammax * dga);
+    const float du1 = fmaf(xiz, dxi, gammaz * dga);
     const float T0 = ri * du0, T1 = ri * du1;
     // core/specfem/point/stress.hpp:118-139 for one component
-    sF[el][0][p] = J * (T0 * xix + T1 * xiz);
-    sF[el][1][p] = J * (T0 * gammax + T1 * gammaz);
+    sF[el][0][p] = J * fmaf(T0, xix, T1 * xiz);
+    sF[el][1][p] = J * fmaf(T0, gammax, T1 * gammaz);
   }
   __syncthreads();
   if (!active) return;
@@ -83,9 +83,9 @@ __global__ __launch_bounds__(128) void acoustic_stiffness_2d_kernel(
     t1 += sF[el][0][iz * 5 + l] * q.hpw[ix][l];
     t2 += sF[el][1][l * 5 + ix] * q.hpw[iz][l];
   }
-  float r = -(q.w[iz] * t1 + q.w[ix] * t2);
+  float r = -fmaf(q.w[iz], t1, q.w[ix] * t2);
   const float c = stacey_[idx];
-  if (c != 0.0f) r += -c * f.v[g];
+  if (c != 0.0f) r = fmaf(-c, f.v[g], r);
   if (dirichlet_[idx]) r = 0.0f;
   add_to<ATOMIC>(&f.a[g], r);
 }
@@ -107,7 +107,7 @@ __global__ __launch_bounds__(256) void coupling_2d_kernel(int n, const int *__re
     unsafeAtomicAdd(&dst.a[s], factor * nx * chi_dd);
     unsafeAtomicAdd(&dst.a[dst.nglob_pad + s], factor * nz * chi_dd);
   } else {
-    unsafeAtomicAdd(&dst.a[s], factor * (nx * src.u[o] + nz * src.u[src.nglob_pad + o]));
+    unsafeAtomicAdd(&dst.a[s], factor * fmaf(nx, src.u[o], nz * src.u[src.nglob_pad + o]));
   }
 }
 
@@ -161,8 +161,8 @@ __device__ __forceinline__ void acoustic_seismogram(int r, int nrec, int ntypes,
           dga += q.hp[iz][l] * sc[l * 5 + ix];
         }
         const float ri = rho_inv_[idx];
-        v0 = ri * (xix_[idx] * dxi + gammax_[idx] * dga);
-        v1 = ri * (xiz_[idx] * dxi + gammaz_[idx] * dga);
+        v0 = ri * fmaf(xix_[idx], dxi, gammax_[idx] * dga);
+        v1 = ri * fmaf(xiz_[idx], dxi, gammaz_[idx] * dga);
       }
       v0 *= hw;
       v1 *= hw;
@@ -207,6 +207,9 @@ __global__ __launch_bounds__(64) void acoustic_seismogram_kernel(
 __global__ __launch_bounds__(128) void coupled_forces_kernel(CoupledStep m, GllConst q, int istep, Fields el,
                                                              Fields ac, int b_ac, int b_src, int b_src_ac, int b_bnd,
                                                              int b_cpl) {
+#pragma clang fp contract(off)
+  // multiply-adds are written out as the separate launches' kernels contract
+  // them, so that steps taken through the seams give the same bits
   __shared__ float su[EA][2][25];
   __shared__ float sF[EA][4][25];
   const int t = threadIdx.x, b = blockIdx.x;
@@ -241,25 +244,25 @@ __global__ __launch_bounds__(128) void coupled_forces_kernel(CoupledStep m, GllC
       for (int l = 0; l < 5; l++) {
 #pragma unroll
         for (int c = 0; c < 2; c++) {
-          dxi[c] += hpx[l] * su[ei][c][iz * 5 + l];
-          dga[c] += hpz[l] * su[ei][c][l * 5 + ix];
+          dxi[c] = fmaf(hpx[l], su[ei][c][iz * 5 + l], dxi[c]);
+          dga[c] = fmaf(hpz[l], su[ei][c][l * 5 + ix], dga[c]);
         }
       }
       float du[2][2];
 #pragma unroll
       for (int c = 0; c < 2; c++) {
-        du[c][0] = xix * dxi[c] + gammax * dga[c];
-        du[c][1] = xiz * dxi[c] + gammaz * dga[c];
+        du[c][0] = fmaf(xix, dxi[c], gammax * dga[c]);
+        du[c][1] = fmaf(xiz, dxi[c], gammaz * dga[c]);
       }
-      const float lp2m = kappa + (4.0f / 3.0f) * mu;
+      const float lp2m = fmaf(4.0f / 3.0f, mu, kappa);
       const float lambda = lp2m - 2.0f * mu;
-      const float sxx = lp2m * du[0][0] + lambda * du[1][1];
-      const float szz = lp2m * du[1][1] + lambda * du[0][0];
+      const float sxx = fmaf(lp2m, du[0][0], lambda * du[1][1]);
+      const float szz = fmaf(lp2m, du[1][1], lambda * du[0][0]);
       const float sxz = mu * (du[0][1] + du[1][0]);
-      sF[ei][0][p] = J * (sxx * xix + sxz * xiz);
-      sF[ei][1][p] = J * (sxx * gammax + sxz * gammaz);
-      sF[ei][2][p] = J * (sxz * xix + szz * xiz);
-      sF[ei][3][p] = J * (sxz * gammax + szz * gammaz);
+      sF[ei][0][p] = J * fmaf(sxx, xix, sxz * xiz);
+      sF[ei][1][p] = J * fmaf(sxx, gammax, sxz * gammaz);
+      sF[ei][2][p] = J * fmaf(sxz, xix, szz * xiz);
+      sF[ei][3][p] = J * fmaf(sxz, gammax, szz * gammaz);
     }
     __syncthreads();
     if (!active) return;
@@ -268,12 +271,12 @@ __global__ __launch_bounds__(128) void coupled_forces_kernel(CoupledStep m, GllC
     for (int l = 0; l < 5; l++) {
 #pragma unroll
       for (int c = 0; c < 2; c++) {
-        t1[c] += sF[ei][2 * c][iz * 5 + l] * hwx[l];
-        t2[c] += sF[ei][2 * c + 1][l * 5 + ix] * hwz[l];
+        t1[c] = fmaf(sF[ei][2 * c][iz * 5 + l], hwx[l], t1[c]);
+        t2[c] = fmaf(sF[ei][2 * c + 1][l * 5 + ix], hwz[l], t2[c]);
       }
     }
 #pragma unroll
-    for (int c = 0; c < 2; c++) m.re[static_cast<size_t>(e) * 50 + c * 25 + p] = -(wz * t1[c] + wx * t2[c]);
+    for (int c = 0; c < 2; c++) m.re[static_cast<size_t>(e) * 50 + c * 25 + p] = -fmaf(wz, t1[c], wx * t2[c]);
     return;
   }
   if (b < b_src) {  // acoustic elements: the arithmetic of acoustic_stiffness_2d_kernel
@@ -292,25 +295,25 @@ __global__ __launch_bounds__(128) void coupled_forces_kernel(CoupledStep m, GllC
       float dxi = 0.0f, dga = 0.0f;
 #pragma unroll
       for (int l = 0; l < 5; l++) {
-        dxi += q.hp[ix][l] * su[ei][0][iz * 5 + l];
-        dga += q.hp[iz][l] * su[ei][0][l * 5 + ix];
+        dxi = fmaf(q.hp[ix][l], su[ei][0][iz * 5 + l], dxi);
+        dga = fmaf(q.hp[iz][l], su[ei][0][l * 5 + ix], dga);
       }
-      const float du0 = xix * dxi + gammax * dga;
-      const float du1 = xiz * dxi + gammaz * dga;
+      const float du0 = fmaf(xix, dxi, gammax * dga);
+      const float du1 = fmaf(xiz, dxi, gammaz * dga);
       const float T0 = ri * du0, T1 = ri * du1;
-      sF[ei][0][p] = J * (T0 * xix + T1 * xiz);
-      sF[ei][1][p] = J * (T0 * gammax + T1 * gammaz);
+      sF[ei][0][p] = J * fmaf(T0, xix, T1 * xiz);
+      sF[ei][1][p] = J * fmaf(T0, gammax, T1 * gammaz);
     }
     __syncthreads();
     if (!active) return;
     float t1 = 0.0f, t2 = 0.0f;
 #pragma unroll
     for (int l = 0; l < 5; l++) {
-      t1 += sF[ei][0][iz * 5 + l] * q.hpw[ix][l];
-      t2 += sF[ei][1][l * 5 + ix] * q.hpw[iz][l];
+      t1 = fmaf(sF[ei][0][iz * 5 + l], q.hpw[ix][l], t1);
+      t2 = fmaf(sF[ei][1][l * 5 + ix], q.hpw[iz][l], t2);
     }
-    float r = -(q.w[iz] * t1 + q.w[ix] * t2);
-    if (c != 0.0f) r += -c * v;
+    float r = -fmaf(q.w[iz], t1, q.w[ix] * t2);
+    if (c != 0.0f) r = fmaf(-c, v, r);
     if (free_surface) r = 0.0f;
     m.re[m.at_ac + static_cast<size_t>(e) * 25 + p] = r;
     return;
@@ -337,19 +340,17 @@ __global__ __launch_bounds__(128) void coupled_forces_kernel(CoupledStep m, GllC
     const int g = m.bnd_gather[k];
     const int np = el.nglob_pad;
     float n[2], v[2];
-    float vn = 0.0f, nn = 0.0f;
 #pragma unroll
     for (int d = 0; d < 2; d++) {
       n[d] = m.bnd_normal[k * 2 + d];
       v[d] = el.v[d * np + g];
-      vn += v[d] * n[d];
-      nn += n[d] * n[d];
     }
+    const float vn = fmaf(v[1], n[1], v[0] * n[0]), nn = fmaf(n[0], n[0], n[1] * n[1]);
     const float j1 = sqrtf(nn);
     const float w = m.bnd_weight[k], rvp = m.bnd_rvp[k], rvs = m.bnd_rvs[k];
 #pragma unroll
     for (int d = 0; d < 2; d++) {
-      const float fac = ((vn * n[d] / (j1 * j1)) * (rvp - rvs)) + v[d] * rvs;
+      const float fac = fmaf(rvs, v[d], (vn * n[d] / (j1 * j1)) * (rvp - rvs));
       m.re[m.at_bnd + static_cast<size_t>(k / 25) * 50 + d * 25 + k % 25] = -1.0f * fac * j1 * w;
     }
     return;
@@ -358,7 +359,7 @@ __global__ __launch_bounds__(128) void coupled_forces_kernel(CoupledStep m, GllC
   if (i >= m.ncpl_ac) return;
   const int o = m.ac_other[i];
   const float factor = m.ac_coef[3 * i], nx = m.ac_coef[3 * i + 1], nz = m.ac_coef[3 * i + 2];
-  m.re[m.at_cpl + static_cast<size_t>(i)] = factor * (nx * el.u[o] + nz * el.u[el.nglob_pad + o]);
+  m.re[m.at_cpl + static_cast<size_t>(i)] = factor * fmaf(nx, el.u[o], nz * el.u[el.nglob_pad + o]);
 }
 
 // s (the point's stored acceleration) + the contributions of its record e, in
@@ -414,19 +415,20 @@ __global__ __launch_bounds__(256) void coupled_acoustic_kernel(CoupledStep m, Fi
   const float a = s[0] * minv;
   m.dd[g] = a;
   f.a[g] = 0.0f;
-  f.v[g] = v + nc.dto2 * a;
+  f.v[g] = fmaf(nc.dto2, a, v);
 }
 
 // Elastic points: mass division, corrector and next predictor; acoustic points:
 // next predictor.
 __global__ __launch_bounds__(256) void coupled_update_kernel(CoupledStep m, Fields el, Fields ac, NewmarkConst nc,
                                                              int b_ac) {
+#pragma clang fp contract(off)
   if (static_cast<int>(blockIdx.x) >= b_ac) {
     const int g = (blockIdx.x - b_ac) * 256 + threadIdx.x;
     if (g >= m.nglob_ac) return;
     const float a = m.dd[g], v = ac.v[g];
-    ac.u[g] = ac.u[g] + (nc.dt * v + nc.dt2o2 * a);
-    ac.v[g] = v + nc.dto2 * a;
+    ac.u[g] = ac.u[g] + fmaf(nc.dt2o2, a, nc.dt * v);
+    ac.v[g] = fmaf(nc.dto2, a, v);
     return;
   }
   const int g = blockIdx.x * 256 + threadIdx.x;
@@ -446,9 +448,9 @@ __global__ __launch_bounds__(256) void coupled_update_kernel(CoupledStep m, Fiel
   for (int c = 0; c < 2; c++) {
     const size_t o = c * static_cast<size_t>(np) + g;
     const float a = s[c] * minv[c];
-    const float v1 = v[c] + nc.dto2 * a;
-    el.u[o] = u[c] + (nc.dt * v1 + nc.dt2o2 * a);
-    el.v[o] = v1 + nc.dto2 * a;
+    const float v1 = fmaf(nc.dto2, a, v[c]);
+    el.u[o] = u[c] + fmaf(nc.dt2o2, a, nc.dt * v1);
+    el.v[o] = fmaf(nc.dto2, a, v1);
     el.a[o] = 0.0f;
   }
 }
@@ -491,7 +493,7 @@ __global__ __launch_bounds__(64) void coupled_seismogram_kernel(CoupledStep m, G
       x[1] = 0.0f;
     } else {
 #pragma unroll
-      for (int c = 0; c < 2; c++) x[c] = type == 0 ? u[c] : type == 1 ? v[c] + dto2 * a[c] : a[c];
+      for (int c = 0; c < 2; c++) x[c] = type == 0 ? u[c] : type == 1 ? fmaf(dto2, a[c], v[c]) : a[c];
     }
 #pragma unroll
     for (int c = 0; c < 2; c++) {

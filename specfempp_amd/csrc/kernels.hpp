@@ -192,8 +192,8 @@ __device__ __forceinline__ float pressure_2d(const PointGeom2D &pg, const GllCon
     }
   }
   const size_t idx = static_cast<size_t>(e) * 25 + p;
-  const float du00 = pg.xix[idx] * dxi[0] + pg.gammax[idx] * dga[0];
-  const float du11 = pg.xiz[idx] * dxi[1] + pg.gammaz[idx] * dga[1];
+  const float du00 = fmaf(pg.xix[idx], dxi[0], pg.gammax[idx] * dga[0]);
+  const float du11 = fmaf(pg.xiz[idx], dxi[1], pg.gammaz[idx] * dga[1]);
   const float mu = pg.mu[idx];
   const float lp2m = pg.kappa[idx] + (4.0f / 3.0f) * mu;
   const float lambda = lp2m - 2.0f * mu;
