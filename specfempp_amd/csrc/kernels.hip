@@ -1226,9 +1226,13 @@ __global__ __launch_bounds__(256) void stacey_re_kernel(int nseg, const int *__r
   const int e = sl / 125, p = sl - (sl / 125) * 125;
   const int rs = re_slot(p % 5, (p / 5) % 5, p / 25);
   const int np = f.nglob_pad;
-  float v[3], t[3] = {0.0f, 0.0f, 0.0f};
+  float *own = re + static_cast<size_t>(e) * RE_ELEM + rs;
+  float v[3], r[3], t[3] = {0.0f, 0.0f, 0.0f};
 #pragma unroll
-  for (int d = 0; d < 3; d++) v[d] = f.v[d * np + g];
+  for (int d = 0; d < 3; d++) {
+    v[d] = f.v[d * np + g];
+    r[d] = own[d * RE_STRIDE];
+  }
   for (int q = q0; q < q1; q++) {
     float n[3];
     float vn = 0.0f, nn = 0.0f;
@@ -1247,7 +1251,7 @@ __global__ __launch_bounds__(256) void stacey_re_kernel(int nseg, const int *__r
     }
   }
 #pragma unroll
-  for (int d = 0; d < 3; d++) re[static_cast<size_t>(e) * RE_ELEM + d * RE_STRIDE + rs] += t[d];
+  for (int d = 0; d < 3; d++) own[d * RE_STRIDE] = r[d] + t[d];
 }
 
 __global__ __launch_bounds__(128) void seismogram_re_kernel(Lattice lat, int nrec, int ntypes,
