@@ -333,15 +333,18 @@ def algorithmic_bytes_2d(nspec: int, nglob: int, geometry: str = "point", elemen
       update_fused: a, M^-1, u, v read (32 B) and u, v, a written (24 B) per point
     With per-point geometry this is the data-model figure of 130 B per
     point-step (25/16 local points per point); model_per_pt_step keeps it.
-    The gather path instead stores the element forces (8 B per local point)
-    and its update reads them once with the inverse index (4 B per local
+    Gather scatter, counted as two kernels, stores the element forces (8 B per
+    local point) and its update reads them once with the inverse index (4 B per local
     point and 4 B per point), and u, v, M^-1 (24 B), writes u, v (16 B; the
     acceleration is recomputed only when a caller asks for it):
       elemforce_2d: gather index per local point, kappa and mu per local
                     point or (element_properties) one pair per element, the
                     geometry, the displacement (8 B per point), the forces
                     written
-      assemble_update_2d: index and forces read, the update as above."""
+      assemble_update_2d: index and forces read, the update as above.
+    The patches that carry whole runs keep the forces of their elements on
+    chip (patch_step): properties and geometry per element, u, v, M^-1 read
+    (24 B) and u, v written (16 B) per point."""
     geo = nspec * GEOMETRY_BYTES_PER_ELEMENT_2D[geometry]
     props = nspec * 8 if element_properties else nspec * 25 * 8
     if scatter == "gather":
@@ -351,7 +354,7 @@ def algorithmic_bytes_2d(nspec: int, nglob: int, geometry: str = "point", elemen
         stiff = nspec * 25 * 4 + props + geo + nglob * 24
         upd = nglob * 56
     model = nspec * 25 * 32 + nglob * 24 + nglob * 56  # per-point geometry, colored scatter, fused update
-    return {"stiffness_2d": stiff, "update_fused": upd, "per_pt_step": (stiff + upd) / nglob,
+    return {"stiffness_2d": stiff, "update_fused": upd, "patch_step": props + geo + nglob * 40, "per_pt_step": (stiff + upd) / nglob,
             "model_per_pt_step": model / nglob}
 
 
@@ -394,9 +397,10 @@ def config2_leg(n: int, steps: int, warmup: int, sample_steps: int = 5, scatter:
     # the bytes of the layout the engine chose (geometry source, properties
     # per point or per element)
     ab = algorithmic_bytes_2d(nspec, nglob, lay["geometry"], lay["element_properties"], scatter=scatter)
-    if scatter == "gather":
-        kern = {"elemforce_2d_kernel": (ab["stiffness_2d"], acc["stiffness_ms"]),
-                "assemble_update_2d_kernel": (ab["update_fused"], acc["update_ms"])}
+    patches = scatter in ("gather", "colored")
+    if patches:
+        kern = {"patch_step_kernel": (ab["patch_step"], acc["stiffness_ms"])}
+        ab["per_pt_step"] = ab["patch_step"] / nglob
     else:
         kern = {"stiffness_2d_kernel": (ab["stiffness_2d"], acc["stiffness_ms"]),
                 "update_fused_kernel": (ab["update_fused"], acc["update_ms"])}
