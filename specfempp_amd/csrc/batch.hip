@@ -482,7 +482,7 @@ struct sfx_batch {
     if (k <= 0) return;
     const PatchState st = patch.state(pfields.p, pfields.p + 2 * pts, nullptr);
     launch_patch_step(stream, patch.pe, patch.patch_end[k - 1], patch.rec_end[k - 1], true, patch_tables(), st, q,
-                      PatchLaunch{ctr.p + par, ctr.p + (par ^ 1), 0, par, 1, 1, 0, nullptr, 0});
+                      PatchLaunch{ctr.p + par, ctr.p + (par ^ 1), 0, par, 1, 1, 0, 0, nullptr, 0});
   }
 
   void reset() {

@@ -265,18 +265,28 @@ struct sfx_engine {
   // Steps [first, first + count), one launch each; then the boundary points,
   // whose last contributions are still open, and the last step's samples.
   // The gather scatter rounds every product and sum on its own, as the oracle
-  // does, and keeps the last acceleration; the colored one contracts them and
-  // leaves the acceleration zero, where its other kernels accumulate.
+  // does, and keeps the last acceleration; the colored one contracts them,
+  // adds a force held in the stored acceleration to the first step's and leaves
+  // the acceleration zero, where its other kernels accumulate.
   // record: the Stacey elements' forces go to the adjoint's record.
   void patch_steps(int first, int count, hipEvent_t *evs = nullptr, bool record_on = false) {
     if (count <= 0) return;
     const bool exact = gather2d();
-    if (!exact && a_kept) {
-      const size_t stride = static_cast<size_t>(h.ncomp) * h.nglob_pad;
-      launch_fill(stream, fields.p + 2 * stride, stride, 0.0f);
-      a_kept = false;
-    }
     const Fields ff = f();
+    if (!exact && a_kept) {
+      // phase by phase, as fused steps do not read the stored acceleration
+      if (evs) SFX_HIP(hipEventRecord(evs[0], stream));
+      if (evs) SFX_HIP(hipEventRecord(evs[1], stream));
+      patch_force(first, record_on);
+      if (evs) SFX_HIP(hipEventRecord(evs[2], stream));
+      if (evs) SFX_HIP(hipEventRecord(evs[3], stream));
+      patch_corrected(first);
+      launch_predictor(stream, h.ncomp, ff, nc);
+      if (evs) SFX_HIP(hipEventRecord(evs[4], stream));
+      a_kept = false;
+      patch_steps(first + 1, count - 1, nullptr, record_on);
+      return;
+    }
     const PatchTables t = patch_tables();
     const PatchState st = patch.state(ff.u, ff.v, ff.a);
     if (evs) SFX_HIP(hipEventRecord(evs[0], stream));
@@ -285,30 +295,39 @@ struct sfx_engine {
     for (int j = 0; j < count; j++) {
       const bool last = j == count - 1;
       launch_patch_step(stream, patch.pe, npatch(), h.nrec, exact, t, st, q,
-                        PatchLaunch{nullptr, nullptr, first + j, j & 1, j > 0, 1, exact && last,
+                        PatchLaunch{nullptr, nullptr, first + j, j & 1, j > 0, 1, exact && last, 0,
                                     record_on ? record.p : nullptr, record_stride()});
       throttle.tick();
     }
     if (evs) SFX_HIP(hipEventRecord(evs[2], stream));
     const int rd = count & 1;
     if ((first + count - 1) % run.nstep_between_samples == 0)
-      launch_patch_step(stream, patch.pe, 0, h.nrec, exact, t, st, q, PatchLaunch{nullptr, nullptr, first + count, rd, 1, 1, 0, nullptr, 0});
+      launch_patch_step(stream, patch.pe, 0, h.nrec, exact, t, st, q,
+                        PatchLaunch{nullptr, nullptr, first + count, rd, 1, 1, 0, 0, nullptr, 0});
     if (evs) SFX_HIP(hipEventRecord(evs[3], stream));
-    launch_patch_boundary(stream, exact, t, st, nc, rd, 1, exact);
+    launch_patch_boundary(stream, exact, t, st, nc, rd, 1, exact, 0);
     if (evs) SFX_HIP(hipEventRecord(evs[4], stream));
     if (exact) a_kept = true;
   }
-  // update_wavefields of the forward field: a = M^-1 f of step istep
   long long record_stride() const { return static_cast<long long>(nstacey) * h.npe * h.ncomp; }
+  // update_wavefields of the forward field: a = M^-1 f of step istep; colored,
+  // f joins the force that the stored acceleration holds
   void patch_force(int istep, bool record_on = false) {
     const bool exact = gather2d();
+    const int add = !exact && a_kept;
     const Fields ff = f();
     const PatchTables t = patch_tables();
     const PatchState st = patch.state(ff.u, ff.v, ff.a);
-    launch_patch_step(stream, patch.pe, npatch(), 0, exact, t, st, q, 
-                      PatchLaunch{nullptr, nullptr, istep, 0, 0, 0, 0, record_on ? record.p : nullptr, record_stride()});
-    launch_patch_boundary(stream, exact, t, st, nc, 1, 0, 0);
+    launch_patch_step(stream, patch.pe, npatch(), 0, exact, t, st, q,
+                      PatchLaunch{nullptr, nullptr, istep, 0, 0, 0, 0, add, record_on ? record.p : nullptr,
+                                  record_stride()});
+    launch_patch_boundary(stream, exact, t, st, nc, 1, 0, 0, add);
     a_kept = true;
+  }
+  // corrector and sample after patch_force
+  void patch_corrected(int istep) {
+    launch_divide_corrector(stream, h.ncomp, f(), nc, 0, 1);
+    if (istep % run.nstep_between_samples == 0) seismograms(f(), istep / run.nstep_between_samples, 0);
   }
   // Recorded forward run: fused steps between the checkpoints; a checkpoint
   // step and the last one stop at the corrected state, which is kept.
@@ -320,8 +339,7 @@ struct sfx_engine {
       while (end < run.nstep - 1 && !is_checkpoint(end)) end++;
       patch_steps(i, end - i, nullptr, true);
       patch_force(end, true);
-      launch_divide_corrector(stream, h.ncomp, ff, nc, 0, 1);
-      if (end % run.nstep_between_samples == 0) seismograms(ff, end / run.nstep_between_samples, 0);
+      patch_corrected(end);
       if (is_checkpoint(end))
         SFX_HIP(hipMemcpyAsync(snapshots.p + static_cast<size_t>(end / snapshot_every) * n3, fields.p,
                                n3 * sizeof(float), hipMemcpyDeviceToDevice, stream));
@@ -926,11 +944,7 @@ struct sfx_engine {
       return;
     }
     if (summed3()) {
-      if (a_kept) {  // fused steps leave a zero acceleration
-        const size_t stride = static_cast<size_t>(h.ncomp) * h.nglob_pad;
-        launch_fill(stream, fields.p + 2 * stride, stride, 0.0f);
-        a_kept = false;
-      }
+      const bool add = a_kept;  // fused steps leave a zero acceleration
       if (evs) SFX_HIP(hipEventRecord(evs[0], stream));
       if (evs) SFX_HIP(hipEventRecord(evs[1], stream));
       forces_3d(ff, istep);
@@ -941,10 +955,11 @@ struct sfx_engine {
         bool need_a = false;
         for (int it = 0; it < run.nseismo_types; it++) need_a = need_a || run.seismo_types[it] != SFX_DISPLACEMENT;
         launch_seismograms_3d_general(stream, h.nrec, run.nseismo_types, types.p, isig, rec_ispec.p, gather.p, rec_h.p,
-                                      ff, nc.dto2, seismo.p, off3.p, ent3.p, re3.p, need_a);
+                                      ff, nc.dto2, seismo.p, off3.p, ent3.p, re3.p, need_a, add);
       }
       if (evs) SFX_HIP(hipEventRecord(evs[3], stream));
-      launch_update_3d_general(stream, h.nglob, off3.p, ent3.p, re3.p, ff, nc, 0);
+      launch_update_3d_general(stream, h.nglob, off3.p, ent3.p, re3.p, ff, nc, 0, add);
+      a_kept = false;
       if (evs) SFX_HIP(hipEventRecord(evs[4], stream));
       return;
     }
@@ -1093,7 +1108,7 @@ struct sfx_engine {
       patch_force(istep);
     } else if (summed3()) {
       forces_3d(ff, istep);
-      launch_update_3d_general(stream, h.nglob, off3.p, ent3.p, re3.p, ff, nc, 1);
+      launch_update_3d_general(stream, h.nglob, off3.p, ent3.p, re3.p, ff, nc, 1, a_kept);
       a_kept = true;
     } else {
       if (h.coupled()) couple_into_elastic(ff);

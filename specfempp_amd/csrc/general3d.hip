@@ -203,12 +203,11 @@ __global__ __launch_bounds__(128) void forces_3d_general_kernel(int nspec, int n
   }
 }
 
-// Sum of a point's contributions [k0, k1) of ent (offsets of their first
+// Adds to s a point's contributions [k0, k1) of ent (offsets of their first
 // component), in order; the first four entries' loads are issued together
 // (indices clamped to the last one).
 __device__ __forceinline__ void point_force(const uint32_t *__restrict__ ent, const float *__restrict__ re, int k0, int k1,
                                             float s[3]) {
-  s[0] = s[1] = s[2] = 0.0f;
   if (k1 <= k0) return;
   uint32_t o[4];
   float r[4][3];
@@ -229,11 +228,11 @@ __device__ __forceinline__ void point_force(const uint32_t *__restrict__ ent, co
 }
 
 // One thread per point: a = M^-1 f; divide: a is stored; else corrector and
-// the next predictor on u, v.
+// the next predictor on u, v.  add: the sum starts from the stored a.
 __global__ __launch_bounds__(256) void update_3d_general_kernel(int nglob, const int *__restrict__ off,
                                                                 const uint32_t *__restrict__ ent,
                                                                 const float *__restrict__ re, Fields f,
-                                                                NewmarkConst nc, int divide) {
+                                                                NewmarkConst nc, int divide, int add) {
   const int g = blockIdx.x * 256 + threadIdx.x;
   if (g >= nglob) return;
   float m[3], u[3], v[3], s[3];
@@ -243,6 +242,7 @@ __global__ __launch_bounds__(256) void update_3d_general_kernel(int nglob, const
     m[c] = f.minv[o];
     u[c] = f.u[o];
     v[c] = f.v[o];
+    s[c] = add ? f.a[o] : 0.0f;
   }
   point_force(ent, re, off[g], off[g + 1], s);
 #pragma unroll
@@ -256,6 +256,7 @@ __global__ __launch_bounds__(256) void update_3d_general_kernel(int nglob, const
     const float v1 = v[c] + nc.dto2 * ac;
     f.u[o] = u[c] + (nc.dt * v1 + nc.dt2o2 * ac);
     f.v[o] = v1 + nc.dto2 * ac;
+    if (add) f.a[o] = 0.0f;
   }
 }
 
@@ -269,7 +270,8 @@ __global__ __launch_bounds__(128) void seismogram_3d_general_kernel(int nrec, in
                                                                     float *__restrict__ seismo,
                                                                     const int *__restrict__ off,
                                                                     const uint32_t *__restrict__ ent,
-                                                                    const float *__restrict__ re, int need_a) {
+                                                                    const float *__restrict__ re, int need_a,
+                                                                    int add) {
   __shared__ float red[4][3][2];
   const int r = blockIdx.x, p = threadIdx.x;
   const int g = p < 125 ? gather[static_cast<size_t>(ispec[r]) * 125 + p] : 0;
@@ -283,6 +285,7 @@ __global__ __launch_bounds__(128) void seismogram_3d_general_kernel(int nrec, in
       u[c] = f.u[o];
       v[c] = f.v[o];
       m[c] = f.minv[o];
+      if (add) a[c] = f.a[o];
     }
     if (need_a) {
       point_force(ent, re, off[g], off[g + 1], a);
@@ -326,18 +329,18 @@ void launch_forces_3d_general(hipStream_t s, int nspec, const int *gather, const
 }
 
 void launch_update_3d_general(hipStream_t s, int nglob, const int *off, const uint32_t *ent, const float *re, Fields f,
-                              NewmarkConst nc, int divide) {
+                              NewmarkConst nc, int divide, int add) {
   if (nglob > 0)
     hipLaunchKernelGGL(update_3d_general_kernel, dim3(groups(nglob, 256)), dim3(256), 0, s, nglob, off, ent, re, f, nc,
-                       divide);
+                       divide, add);
 }
 
 void launch_seismograms_3d_general(hipStream_t s, int nrec, int ntypes, const int *types, int isig, const int *ispec,
                                    const int *gather, const float *h, Fields f, float dto2, float *seismo,
-                                   const int *off, const uint32_t *ent, const float *re, int need_a) {
+                                   const int *off, const uint32_t *ent, const float *re, int need_a, int add) {
   if (nrec > 0 && ntypes > 0)
     hipLaunchKernelGGL(seismogram_3d_general_kernel, dim3(nrec), dim3(128), 0, s, nrec, ntypes, types, isig, ispec,
-                       gather, h, f, dto2, seismo, off, ent, re, need_a);
+                       gather, h, f, dto2, seismo, off, ent, re, need_a, add);
 }
 
 }  // namespace sfx

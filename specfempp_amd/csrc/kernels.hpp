@@ -252,11 +252,12 @@ void launch_forces_3d_general(hipStream_t s, int nspec, const int *gather, const
                               const float *rho_vs, float *re);
 // Per point the sum of its contributions ent[off[g] .. off[g + 1]) (offsets
 // into re), divided by the mass; then corrector and predictor, or (divide) a.
+// add: the sums start from the stored a, which corrector and predictor clear.
 void launch_update_3d_general(hipStream_t s, int nglob, const int *off, const uint32_t *ent, const float *re, Fields f,
-                              NewmarkConst nc, int divide);
+                              NewmarkConst nc, int divide, int add);
 void launch_seismograms_3d_general(hipStream_t s, int nrec, int ntypes, const int *types, int isig, const int *ispec,
                                    const int *gather, const float *h, Fields f, float dto2, float *seismo,
-                                   const int *off, const uint32_t *ent, const float *re, int need_a);
+                                   const int *off, const uint32_t *ent, const float *re, int need_a, int add);
 
 // ---- 2-D acoustic medium and elastic-acoustic coupling (acoustic.hip) ----
 // Acoustic stiffness over device element slots [first, first + count) of the

@@ -142,12 +142,18 @@ template <int PE> constexpr int patch_threads() { return (PE * 5 + 63) / 64 * 64
 
 // Sum of an interior point's contributions in order, the first one (table
 // entry ea) given: its local index l tells how many there are (the points are
-// sorted by that number).
+// sorted by that number).  a0, a1: the patch's stored acceleration the sum
+// starts from, or null.
 __device__ __forceinline__ float2 interior_force(const PatchHead &h, const uint16_t *__restrict__ tab,
-                                                 const float *st, int l, int ea, int eb) {
+                                                 const float *st, int l, int ea, int eb, const float *a0 = nullptr,
+                                                 const float *a1 = nullptr) {
 #pragma clang fp contract(off)
   const float2 *f = reinterpret_cast<const float2 *>(st);
   float2 s = f[ea];
+  if (a0) {
+    s.x = at(a0, l) + s.x;
+    s.y = at(a1, l) + s.y;
+  }
   if (l >= h.n1) {
     const float2 r = f[eb];
     s.x += r.x;
@@ -180,15 +186,16 @@ template <bool EXACT> struct Newmark {
   }
 };
 
-// Sum of n contributions from k0 on, in order; the first four are loaded
-// together (indices clamped to the last one).
-__device__ __forceinline__ void boundary_force(const float2 *__restrict__ rb, int k0, int n, float s[2]) {
+// Sum of n contributions from k0 on, in order, after a0 and a1; the first four
+// are loaded together (indices clamped to the last one).
+__device__ __forceinline__ void boundary_force(const float2 *__restrict__ rb, int k0, int n, float s[2],
+                                               float a0 = 0.0f, float a1 = 0.0f) {
 #pragma clang fp contract(off)
   float2 r[4];
 #pragma unroll
   for (int j = 0; j < 4; j++) r[j] = rb[k0 + (j < n ? j : n - 1)];
-  s[0] = 0.0f;
-  s[1] = 0.0f;
+  s[0] = a0;
+  s[1] = a1;
 #pragma unroll
   for (int j = 0; j < 4; j++)
     if (j < n) {
@@ -583,11 +590,12 @@ __global__ __launch_bounds__(patch_threads<PE>()) __attribute__((amdgpu_waves_pe
     for (int k = t; k < h.nbent; k += NT) out[T.bslot[h.be0 + k]] = f[tab[h.bent + k]];
   }
   const bool snapshot = h.rm0 >= 0 && L.advance && n % h.nsb == 0;
+  const float *const a0p = !EXACT && L.add_a ? S.a + h.pt0 : nullptr, *const a1p = a0p ? S.a + np + h.pt0 : nullptr;
 #pragma unroll
   for (int k = 0; k < NI; k++) {
     const int l = t + k * NT;
     if (l >= h.nint) continue;
-    const float2 s = interior_force(h, tab, se, l, ea[k], eb[k]);
+    const float2 s = interior_force(h, tab, se, l, ea[k], eb[k], a0p, a1p);
     const float a0 = s.x * mi[k][0], a1 = s.y * mi[k][1];
     if (L.advance) {
       float u0 = su[0][l], u1 = su[1][l], v0 = vi[k][0], v1 = vi[k][1], w0, w1;
@@ -976,13 +984,14 @@ __global__ __launch_bounds__(256) void patch_pair_boundary_kernel(PatchTables T,
 // One thread per boundary point: see launch_patch_boundary.
 template <bool EXACT>
 __global__ __launch_bounds__(256) void patch_boundary_kernel(PatchTables T, PatchState S, Newmark<EXACT> nm, int rd,
-                                                             int advance, int store_a) {
+                                                             int advance, int store_a, int add_a) {
 #pragma clang fp contract(off)
   const int b = blockIdx.x * 256 + threadIdx.x;
   if (b >= T.nbnd) return;
   float s[2];
   const int k0 = T.boff[b];
-  boundary_force(S.rb[rd], k0, T.boff[b + 1] - k0, s);
+  const float *const stored = S.a + T.nint + b;
+  boundary_force(S.rb[rd], k0, T.boff[b + 1] - k0, s, add_a ? stored[0] : 0.0f, add_a ? stored[T.np] : 0.0f);
 #pragma unroll
   for (int c = 0; c < 2; c++) {
     const size_t o = c * static_cast<size_t>(T.np) + T.nint + b;
@@ -1078,15 +1087,15 @@ void launch_patch_step(hipStream_t s, int pe, int npatch, int nrec, bool exact, 
 }
 
 void launch_patch_boundary(hipStream_t s, bool exact, const PatchTables &t, const PatchState &st, NewmarkConst nc,
-                           int rd, int advance, int store_a) {
+                           int rd, int advance, int store_a, int add_a) {
   if (t.nbnd <= 0) return;
   const dim3 grid((t.nbnd + 255) / 256);
   if (exact)
     hipLaunchKernelGGL(patch_boundary_kernel<true>, grid, dim3(256), 0, s, t, st,
-                       (Newmark<true>{nc.dt, nc.dto2, nc.dt2o2}), rd, advance, store_a);
+                       (Newmark<true>{nc.dt, nc.dto2, nc.dt2o2}), rd, advance, store_a, add_a);
   else
     hipLaunchKernelGGL(patch_boundary_kernel<false>, grid, dim3(256), 0, s, t, st,
-                       (Newmark<false>{nc.dt, nc.dto2, nc.dt2o2}), rd, advance, store_a);
+                       (Newmark<false>{nc.dt, nc.dto2, nc.dt2o2}), rd, advance, store_a, add_a);
 }
 
 void launch_patch_pair(hipStream_t s, int pe, int npatch, int nrec, const PatchTables &t, const PatchState &adj,
