@@ -412,14 +412,56 @@ struct sfx_engine {
       launch_patch_pair(stream, patch.pe, 0, h.nrec, t, sa, sb, q, PatchPairLaunch{lo - 1, rd, 1, top, nullptr}, p);
     launch_patch_pair_boundary(stream, t, sa, sb, nc, rd, racc.p);
   }
+  // d_lattice with stage beside it, or null where the device has no memory left
+  // for the two (the host permutes then)
   const int *device_order() {
-    if (h.lattice_of.empty()) return nullptr;
-    if (!d_lattice.p) {
-      d_lattice.upload(h.lattice_of, stream);
+    if (d_lattice.p && stage.p) return d_lattice.p;
+    try {
       stage.alloc(h.lattice_of.size());
+      d_lattice.upload(h.lattice_of, stream);
       SFX_HIP(hipStreamSynchronize(stream));
+    } catch (const HipError &) {
+      (void)hipGetLastError();
+      stage.alloc(0);
+      d_lattice.alloc(0);
     }
     return d_lattice.p;
+  }
+  // one component of a field, between the device's and the API's point order
+  void read_component(const float *src, float *out) {
+    const size_t ng = h.nglob_el;
+    if (h.lattice_of.empty()) {
+      SFX_HIP(hipStreamSynchronize(stream));
+      SFX_HIP(hipMemcpy(out, src, ng * sizeof(float), hipMemcpyDeviceToHost));
+      return;
+    }
+    if (const int *order = device_order()) {
+      launch_take(stream, static_cast<int>(ng), order, src, stage.p);
+      SFX_HIP(hipStreamSynchronize(stream));
+      SFX_HIP(hipMemcpy(out, stage.p, ng * sizeof(float), hipMemcpyDeviceToHost));
+      return;
+    }
+    std::vector<float> buf(h.nglob_pad);
+    SFX_HIP(hipStreamSynchronize(stream));
+    SFX_HIP(hipMemcpy(buf.data(), src, buf.size() * sizeof(float), hipMemcpyDeviceToHost));
+    for (size_t g = 0; g < ng; g++) out[g] = buf[h.lattice_of[g]];
+  }
+  void write_component(float *dst, const float *in) {
+    const size_t ng = h.nglob_el;
+    SFX_HIP(hipStreamSynchronize(stream));
+    if (h.lattice_of.empty()) {
+      SFX_HIP(hipMemcpy(dst, in, ng * sizeof(float), hipMemcpyHostToDevice));
+      return;
+    }
+    if (const int *order = device_order()) {
+      SFX_HIP(hipMemcpy(stage.p, in, ng * sizeof(float), hipMemcpyHostToDevice));
+      launch_put(stream, static_cast<int>(ng), order, stage.p, dst);
+      SFX_HIP(hipStreamSynchronize(stream));
+      return;
+    }
+    std::vector<float> buf(h.nglob_pad, 0.0f);
+    for (size_t g = 0; g < ng; g++) buf[h.lattice_of[g]] = in[g];
+    SFX_HIP(hipMemcpy(dst, buf.data(), buf.size() * sizeof(float), hipMemcpyHostToDevice));
   }
   // where the 2-D gather scatter takes each point's geometry from
   int geom2d_form() const {
@@ -1839,16 +1881,8 @@ int sfx_get_wavefield(const sfx_engine *ce, int wavefield, int which, float *out
     if (wavefield == SFX_WAVEFIELD_FORWARD && which == 2) e->refresh_acceleration();
     Fields F = e->wavefield(wavefield);
     const float *arrays[4] = {F.u, F.v, F.a, F.minv};
-    // the device permutes to the reference's point order; one copy per component
-    const int ng = e->h.nglob_el;
-    const int *order = e->device_order();
-    for (int c = 0; c < e->h.ncomp; c++) {
-      const float *src = arrays[which] + static_cast<size_t>(c) * e->h.nglob_pad;
-      if (order) launch_take(e->stream, ng, order, src, e->stage.p);
-      SFX_HIP(hipStreamSynchronize(e->stream));
-      SFX_HIP(hipMemcpy(out + static_cast<size_t>(c) * ng, order ? e->stage.p : src, ng * sizeof(float),
-                        hipMemcpyDeviceToHost));
-    }
+    for (int c = 0; c < e->h.ncomp; c++)
+      e->read_component(arrays[which] + static_cast<size_t>(c) * e->h.nglob_pad, out + static_cast<size_t>(c) * e->h.nglob_el);
   }, stream_of(ce));
 }
 
@@ -1863,16 +1897,8 @@ int sfx_set_wavefield(sfx_engine *e, int wavefield, int which, const float *in) 
     if (!in) throw std::invalid_argument("null input");
     Fields F = e->wavefield(wavefield);
     float *arrays[3] = {F.u, F.v, F.a};
-    const int ng = e->h.nglob_el;
-    const int *order = e->device_order();
-    for (int c = 0; c < e->h.ncomp; c++) {
-      float *dst = arrays[which] + static_cast<size_t>(c) * e->h.nglob_pad;
-      SFX_HIP(hipStreamSynchronize(e->stream));
-      SFX_HIP(hipMemcpy(order ? e->stage.p : dst, in + static_cast<size_t>(c) * ng, ng * sizeof(float),
-                        hipMemcpyHostToDevice));
-      if (order) launch_put(e->stream, ng, order, e->stage.p, dst);
-    }
-    SFX_HIP(hipStreamSynchronize(e->stream));
+    for (int c = 0; c < e->h.ncomp; c++)
+      e->write_component(arrays[which] + static_cast<size_t>(c) * e->h.nglob_pad, in + static_cast<size_t>(c) * e->h.nglob_el);
     if (wavefield == SFX_WAVEFIELD_FORWARD && which == 2) e->a_stale = false, e->a_kept = true;
   }, stream_of(e));
 }

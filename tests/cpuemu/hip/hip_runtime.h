@@ -89,7 +89,7 @@ inline float __builtin_amdgcn_rcpf(float x) { return 1.0f / x; }
 inline float sqrtf_(float x) { return std::sqrt(x); }
 
 typedef int hipError_t;
-enum { hipSuccess = 0, hipErrorNotSupported = 801 };
+enum { hipSuccess = 0, hipErrorOutOfMemory = 2, hipErrorNotSupported = 801 };
 typedef void *hipStream_t;
 typedef void *hipEvent_t;
 typedef void *hipGraph_t;
@@ -99,7 +99,15 @@ enum { hipStreamCaptureModeThreadLocal = 0, hipEventDisableTiming = 2 };
 
 inline const char *hipGetErrorString(hipError_t e) { return e ? "emulated error" : "no error"; }
 inline hipError_t hipGetLastError() { return hipSuccess; }
+namespace emu {
+inline std::atomic<long> mallocs_left{-1};  // allocations that still succeed; -1: all
+}
+// for tests: the n-th allocation from now on and all after it fail (n < 0: none)
+extern "C" __attribute__((used)) inline void emu_allow_mallocs(long n) { emu::mallocs_left = n; }
 template <class T> inline hipError_t hipMalloc(T **p, size_t n) {
+  *p = nullptr;
+  if (emu::mallocs_left == 0) return hipErrorOutOfMemory;
+  if (emu::mallocs_left > 0) emu::mallocs_left--;
   *p = static_cast<T *>(std::malloc(n ? n : 1));
   std::memset(*p, 0x7f, n);  // poison: reads of never-written device memory show up as huge values
   return hipSuccess;
@@ -108,7 +116,14 @@ inline hipError_t hipFree(void *p) { std::free(p); return hipSuccess; }
 inline hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { std::memcpy(d, s, n); return hipSuccess; }
 inline hipError_t hipStreamCreate(hipStream_t *s) { *s = (void *)1; return hipSuccess; }
 inline hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
-inline hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+namespace emu {
+inline std::atomic<int> launches{0};  // under way, of all host threads
+}
+// what other host threads have launched ends before this returns
+inline hipError_t hipStreamSynchronize(hipStream_t) {
+  while (emu::launches) std::this_thread::yield();
+  return hipSuccess;
+}
 inline hipError_t hipEventCreate(hipEvent_t *e) { *e = (void *)1; return hipSuccess; }
 inline hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { *e = (void *)1; return hipSuccess; }
 inline hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
@@ -151,6 +166,9 @@ void launch(void (*k)(P...), dim3 grid, dim3 block, size_t, hipStream_t, A &&...
     });
     return;
   }
+  static std::mutex one_at_a_time;  // streams of several host threads
+  launches++;
+  std::lock_guard<std::mutex> lock(one_at_a_time);
   shfl_buf.assign(nt, 0.0f);
   // nt pool threads run the blocks one after another; each block gets a fresh
   // barrier for __syncthreads, which a thread leaves when its kernel returns
@@ -183,6 +201,7 @@ void launch(void (*k)(P...), dim3 grid, dim3 block, size_t, hipStream_t, A &&...
   stop = true;
   start.arrive_and_wait();
   for (auto &x : th) x.join();
+  launches--;
 }
 }  // namespace emu
 #define hipLaunchKernelGGL(...) emu::launch(__VA_ARGS__)
