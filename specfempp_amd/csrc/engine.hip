@@ -97,9 +97,11 @@ struct sfx_engine {
   // points of every element
   DevBuf<float> kmu_e;
   // API point order -> device order (lattice_of on the device) and a
-  // component's staging copy, at first use
+  // component's staging copy, at first use; both belong to the call that holds
+  // the mutex
   DevBuf<int> d_lattice;
   DevBuf<float> stage;
+  std::mutex stage_mutex;
   DevBuf<float> bnd_normal, bnd_weight, bnd_rvp, bnd_rvs;
   DevBuf<float> src_array, stf, rec_h, seismo;
   DevBuf<float> fields;  // u, v, a, minv: 4 * ncomp * nglob_pad
@@ -435,6 +437,7 @@ struct sfx_engine {
       SFX_HIP(hipMemcpy(out, src, ng * sizeof(float), hipMemcpyDeviceToHost));
       return;
     }
+    std::lock_guard<std::mutex> lock(stage_mutex);
     if (const int *order = device_order()) {
       launch_take(stream, static_cast<int>(ng), order, src, stage.p);
       SFX_HIP(hipStreamSynchronize(stream));
@@ -453,6 +456,7 @@ struct sfx_engine {
       SFX_HIP(hipMemcpy(dst, in, ng * sizeof(float), hipMemcpyHostToDevice));
       return;
     }
+    std::lock_guard<std::mutex> lock(stage_mutex);
     if (const int *order = device_order()) {
       SFX_HIP(hipMemcpy(stage.p, in, ng * sizeof(float), hipMemcpyHostToDevice));
       launch_put(stream, static_cast<int>(ng), order, stage.p, dst);
