@@ -271,7 +271,7 @@ struct sfx_engine {
   // adds a force held in the stored acceleration to the first step's and leaves
   // the acceleration zero, where its other kernels accumulate.
   // record: the Stacey elements' forces go to the adjoint's record.
-  void patch_steps(int first, int count, hipEvent_t *evs = nullptr, bool record_on = false) {
+  void patch_steps(int first, int count, Throttle &throttle, hipEvent_t *evs = nullptr, bool record_on = false) {
     if (count <= 0) return;
     const bool exact = gather2d();
     const Fields ff = f();
@@ -286,14 +286,14 @@ struct sfx_engine {
       launch_predictor(stream, h.ncomp, ff, nc);
       if (evs) SFX_HIP(hipEventRecord(evs[4], stream));
       a_kept = false;
-      patch_steps(first + 1, count - 1, nullptr, record_on);
+      throttle.tick();
+      patch_steps(first + 1, count - 1, throttle, nullptr, record_on);
       return;
     }
     const PatchTables t = patch_tables();
     const PatchState st = patch.state(ff.u, ff.v, ff.a);
     if (evs) SFX_HIP(hipEventRecord(evs[0], stream));
     if (evs) SFX_HIP(hipEventRecord(evs[1], stream));
-    Throttle throttle(stream);
     for (int j = 0; j < count; j++) {
       const bool last = j == count - 1;
       launch_patch_step(stream, patch.pe, npatch(), h.nrec, exact, t, st, q,
@@ -333,13 +333,13 @@ struct sfx_engine {
   }
   // Recorded forward run: fused steps between the checkpoints; a checkpoint
   // step and the last one stop at the corrected state, which is kept.
-  void patch_record() {
+  void patch_record(Throttle &throttle) {
     const Fields ff = f();
     const size_t n3 = 3 * static_cast<size_t>(h.ncomp) * h.nglob_pad;
     for (int i = 0; i < run.nstep;) {
       int end = i;
       while (end < run.nstep - 1 && !is_checkpoint(end)) end++;
-      patch_steps(i, end - i, nullptr, true);
+      patch_steps(i, end - i, throttle, nullptr, true);
       patch_force(end, true);
       patch_corrected(end);
       if (is_checkpoint(end))
@@ -349,6 +349,7 @@ struct sfx_engine {
         launch_predictor(stream, h.ncomp, ff, nc);
         a_kept = false;
       }
+      throttle.tick();
       i = end + 1;
     }
   }
@@ -958,7 +959,8 @@ struct sfx_engine {
     }
     if (patches() && !recording) {
       if (istep < 0 || istep >= run.nstep) throw std::invalid_argument("istep out of range");
-      patch_steps(istep, 1, evs);
+      Throttle throttle(stream);
+      patch_steps(istep, 1, throttle, evs);
       return;
     }
     if (gather_path()) {
@@ -1749,7 +1751,8 @@ int sfx_run(sfx_engine *e, int first, int count) {
         e->ev.push_back(ev);
       }
       SFX_HIP(hipEventRecord(e->ev[0], e->stream));
-      e->patch_steps(first, count);
+      Throttle throttle(e->stream);
+      e->patch_steps(first, count, throttle);
       SFX_HIP(hipEventRecord(e->ev[1], e->stream));
       SFX_HIP(hipGetLastError());
       SFX_HIP(hipStreamSynchronize(e->stream));
@@ -1981,7 +1984,7 @@ int sfx_forward_record(sfx_engine *e, int snapshot_every) {
       const bool graphs = e->graph_2d() && !e->patches();
       if (graphs) e->set_step(0);
       Throttle throttle(e->stream);
-      if (e->patches()) e->patch_record();
+      if (e->patches()) e->patch_record(throttle);
       for (int istep = e->patches() ? e->run.nstep : 0; istep < e->run.nstep; istep++) {
         const bool last = istep == e->run.nstep - 1;
         if (graphs && !last && !e->is_checkpoint(istep)) {

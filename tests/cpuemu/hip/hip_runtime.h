@@ -4,6 +4,7 @@
 // (shared by the threads of the running block); __syncthreads is a barrier
 // that exited threads drop out of.
 #pragma once
+#include <algorithm>
 #include <atomic>
 #include <barrier>
 #include <cmath>
@@ -118,17 +119,28 @@ inline hipError_t hipStreamCreate(hipStream_t *s) { *s = (void *)1; return hipSu
 inline hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 namespace emu {
 inline std::atomic<int> launches{0};  // under way, of all host threads
+inline std::atomic<long> launched{0}, waited{0}, most_queued{0};  // in all; waited for; most that were not
+struct Event { long at = 0; };
 }
+// for tests: the most launches that were queued without a wait since the last call
+extern "C" __attribute__((used)) inline long emu_most_queued() { return emu::most_queued.exchange(0); }
 // what other host threads have launched ends before this returns
 inline hipError_t hipStreamSynchronize(hipStream_t) {
   while (emu::launches) std::this_thread::yield();
+  emu::waited = emu::launched.load();
   return hipSuccess;
 }
-inline hipError_t hipEventCreate(hipEvent_t *e) { *e = (void *)1; return hipSuccess; }
-inline hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { *e = (void *)1; return hipSuccess; }
-inline hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
-inline hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
-inline hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+inline hipError_t hipEventCreate(hipEvent_t *e) { *e = new emu::Event(); return hipSuccess; }
+inline hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return hipEventCreate(e); }
+inline hipError_t hipEventDestroy(hipEvent_t e) { delete static_cast<emu::Event *>(e); return hipSuccess; }
+inline hipError_t hipEventRecord(hipEvent_t e, hipStream_t) {
+  static_cast<emu::Event *>(e)->at = emu::launched;
+  return hipSuccess;
+}
+inline hipError_t hipEventSynchronize(hipEvent_t e) {
+  emu::waited = std::max(emu::waited.load(), static_cast<emu::Event *>(e)->at);
+  return hipSuccess;
+}
 inline hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) { *ms = 0; return hipSuccess; }
 namespace emu {
 // stream capture: launches and async copies are recorded as closures and
@@ -168,6 +180,8 @@ void launch(void (*k)(P...), dim3 grid, dim3 block, size_t, hipStream_t, A &&...
   }
   static std::mutex one_at_a_time;  // streams of several host threads
   launches++;
+  launched++;
+  most_queued = std::max(most_queued.load(), launched - waited);
   std::lock_guard<std::mutex> lock(one_at_a_time);
   shfl_buf.assign(nt, 0.0f);
   // nt pool threads run the blocks one after another; each block gets a fresh
