@@ -209,10 +209,11 @@ void launch_seismograms(hipStream_t s, int dim, int npe, int nrec, int ntypes, c
                         int nsb = 1, int sig_top = -1, const int *rec_list = nullptr,
                         int nlist = -1);
 // Where the 2-D patches take an element point's geometry from.  Every form
-// gives the same bits: the control-node forms repeat the host's float
-// operations in the host's order (compute_partial_derivatives.cpp:46-91, no
-// fused multiply-add, correctly rounded division), so they trade 20 bytes per
-// point for 8 or 18 floats per element.
+// gives the same values, bit for bit but for the sign of a zero: the
+// control-node forms repeat the host's float operations in the host's order
+// (compute_partial_derivatives.cpp:46-91, no fused multiply-add, correctly
+// rounded division: division.hpp), so they trade 20 bytes per point for 8 or
+// 18 floats per element.
 enum Geom2DMode : int { GEOM2D_POINT = 0, GEOM2D_RECORD = 1, GEOM2D_CTRL4 = 4, GEOM2D_CTRL9 = 9 };
 struct Geom2D {
   int mode = GEOM2D_POINT;

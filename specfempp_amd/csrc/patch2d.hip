@@ -19,6 +19,7 @@
 // of its phases at five wavefronts per SIMD.  Workgroups of four wavefronts
 // matter: with five (64 elements) only 2.3 of 4 workgroups were resident per
 // CU and the same step took 318 us.
+#include "division.hpp"
 #include "lattice.hpp"
 #include "patch2d.hpp"
 
@@ -46,22 +47,6 @@ __device__ __forceinline__ int at(const uint16_t *a, unsigned i) {
 }
 __device__ __forceinline__ void put(float *a, unsigned i, float v) {
   *reinterpret_cast<float *>(reinterpret_cast<char *>(a) + (i * 4u)) = v;
-}
-
-// Correctly rounded 1 / b and a / b for b well inside the normal range
-// (Markstein's theorem: with y the rounded reciprocal, one residual step from
-// a faithful quotient rounds correctly; the first step makes it faithful).
-// The four quotients of a point share one reciprocal: 25 instructions instead
-// of four full divisions' 44.
-__device__ __forceinline__ float reciprocal(float b) {
-  float y = __builtin_amdgcn_rcpf(b);
-  y = fmaf(fmaf(-b, y, 1.0f), y, y);
-  return fmaf(fmaf(-b, y, 1.0f), y, y);
-}
-__device__ __forceinline__ float quotient(float a, float b, float y) {
-  float q = a * y;
-  q = fmaf(fmaf(-b, q, a), y, q);
-  return fmaf(fmaf(-b, q, a), y, q);
 }
 
 // The row constants of the four-node form: x and z derivatives in xi.
