@@ -245,11 +245,11 @@ struct sfx_engine {
 
   bool gather_path() const { return h.dim == 3 && run.scatter == SFX_SCATTER_GATHER; }
   bool gather2d() const { return h.dim == 2 && run.scatter == SFX_SCATTER_GATHER; }
-  // 2-D elastic meshes: forward steps run patch by patch
-  bool patches() const {
-    return h.dim == 2 && !h.coupled() && !host_only &&
-           (run.scatter == SFX_SCATTER_GATHER || run.scatter == SFX_SCATTER_COLORED);
+  // 2-D elastic meshes: forward steps run patch by patch (on the device)
+  bool patch_layout() const {
+    return h.dim == 2 && !h.coupled() && (run.scatter == SFX_SCATTER_GATHER || run.scatter == SFX_SCATTER_COLORED);
   }
+  bool patches() const { return patch_layout() && !host_only; }
   PatchTables patch_tables() const {
     PatchTables t = patch.t;
     t.src_array = src_array.p;
@@ -468,18 +468,18 @@ struct sfx_engine {
     for (size_t g = 0; g < ng; g++) buf[h.lattice_of[g]] = in[g];
     SFX_HIP(hipMemcpy(dst, buf.data(), buf.size() * sizeof(float), hipMemcpyHostToDevice));
   }
-  // where the 2-D gather scatter takes each point's geometry from
+  // where 2-D steps take each point's geometry from
   int geom2d_form() const {
     if (h.dim != 2) return GEOM2D_POINT;
     if (!h.geo2d.empty()) return GEOM2D_RECORD;
-    if (gather2d() && (h.ngnod2d == 4 || h.ngnod2d == 9)) return h.ngnod2d;
+    if (patch_layout() && (h.ngnod2d == 4 || h.ngnod2d == 9)) return h.ngnod2d;
     return GEOM2D_POINT;
   }
-  // (kappa, mu) per element slot for the 2-D and 3-D gather paths when every
-  // element holds one value of each at all of its points (bit for bit); empty
-  // otherwise
+  // (kappa, mu) per element slot for the 2-D patches, the 3-D gather path and
+  // 3-D database meshes when every element holds one value of each at all of
+  // its points (bit for bit); empty otherwise
   std::vector<float> element_properties() const {
-    if (!gather2d() && !gather_path() && !h.general3d) return {};
+    if (!patch_layout() && !gather_path() && !h.general3d) return {};
     const size_t npe = h.npe;
     std::vector<float> kmu(2 * static_cast<size_t>(h.nspec));
     auto same = [](float a, float b) { return std::memcmp(&a, &b, sizeof(float)) == 0; };
@@ -1479,7 +1479,7 @@ int sfx_get_layout(const sfx_engine *e, int64_t *s) {
     s[0] = e->h.dim == 2 ? e->geom2d_form() : (e->h.general3d ? GEOM2D_POINT : GEOM2D_RECORD);
     s[1] = e->h.general3d || e->element_properties().empty() ? 0 : 1;
     s[2] = e->run.scatter;
-    s[3] = e->gather2d() ? 1 : 0;
+    s[3] = e->patch_layout() ? 1 : 0;
   });
 }
 

@@ -274,7 +274,7 @@ class _EngineBase:
     def layout(self):
         """The storage the engine chose: ``geometry`` "point", "element" or
         "control_nodes_4" / "control_nodes_9" (recomputed per point from the
-        element's control nodes, the same bits as the per-point arrays),
+        element's control nodes, the same values as the per-point arrays),
         ``element_properties`` (kappa and mu read once per element),
         ``scatter`` and ``row_order`` (points ordered by their place in the
         mesh)."""
