@@ -460,9 +460,11 @@ int sfx_batch_get_seismograms(const sfx_batch *batch, int i, float *out);
 int sfx_batch_get_info(const sfx_batch *batch, double *out8);
 
 /* ---- measurement -------------------------------------------------------------
- * Average device time (ms) of each kernel family over the last sfx_run, taken
- * with HIP events on the engine stream: out[0] stiffness, out[1] fused update,
- * out[2] boundary+source+seismogram, out[3] whole step. */
+ * Device times (ms) of the last sfx_run, from HIP events on the engine stream.
+ * out[0] stiffness, out[1] fused update, out[2] boundary+source+seismogram:
+ * averages over at most eight steps spread over the run; 0 for 2-D elastic runs
+ * of more than one step, where one launch or captured graph carries a step.
+ * out[3] the whole run divided by its steps. */
 int sfx_get_timings(const sfx_engine *engine, double *out4);
 
 #ifdef __cplusplus

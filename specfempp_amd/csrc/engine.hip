@@ -1786,40 +1786,45 @@ int sfx_run(sfx_engine *e, int first, int count) {
       return;
     }
     // The kernel times come from at most TIMED_STEPS steps spread over the run,
-    // each bracketed by 5 events read after the last step: events on every
+    // each bracketed by 5 events read after the last step (the step's time from
+    // two events around the run): events on every
     // step delayed its launches by about as long as a small mesh's kernels
     // take (9 x 11 x 7 elements: 47 us a step with them).
     constexpr int TIMED_STEPS = 8;
     const int timed = std::min(count, TIMED_STEPS);
-    const size_t need = 5 * static_cast<size_t>(timed);
+    const size_t need = 5 * static_cast<size_t>(timed) + 2;
     while (e->ev.size() < need) {
       hipEvent_t ev;
       SFX_HIP(hipEventCreate(&ev));
       e->ev.push_back(ev);
     }
+    hipEvent_t *const ends = &e->ev[5 * static_cast<size_t>(timed)];
+    SFX_HIP(hipEventRecord(ends[0], e->stream));
     Throttle throttle(e->stream);
     for (int i = 0, k = 0; i < count; i++) {
       const bool time_it = k < timed && i == static_cast<int>(static_cast<int64_t>(k) * count / timed);
       e->step(first + i, time_it ? &e->ev[5 * static_cast<size_t>(k++)] : nullptr, i == count - 1);
       throttle.tick();
     }
+    SFX_HIP(hipEventRecord(ends[1], e->stream));
     SFX_HIP(hipGetLastError());
     SFX_HIP(hipStreamSynchronize(e->stream));
-    double acc[4] = {0, 0, 0, 0};
+    double acc[3] = {0, 0, 0};
     for (int i = 0; i < timed; i++) {
       hipEvent_t *v = &e->ev[5 * static_cast<size_t>(i)];
-      float stiff, upd, src, bnd, all;
+      float stiff, upd, src, bnd;
       SFX_HIP(hipEventElapsedTime(&src, v[0], v[1]));
       SFX_HIP(hipEventElapsedTime(&stiff, v[1], v[2]));
       SFX_HIP(hipEventElapsedTime(&bnd, v[2], v[3]));
       SFX_HIP(hipEventElapsedTime(&upd, v[3], v[4]));
-      SFX_HIP(hipEventElapsedTime(&all, v[0], v[4]));
       acc[0] += stiff;
       acc[1] += upd;
       acc[2] += src + bnd;
-      acc[3] += all;
     }
-    for (int k = 0; k < 4; k++) e->timings[k] = timed ? acc[k] / timed : 0.0;
+    for (int k = 0; k < 3; k++) e->timings[k] = timed ? acc[k] / timed : 0.0;
+    float all = 0.0f;
+    SFX_HIP(hipEventElapsedTime(&all, ends[0], ends[1]));
+    e->timings[3] = count ? all / count : 0.0;
   }, stream_of(e));
 }
 

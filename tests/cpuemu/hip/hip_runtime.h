@@ -154,7 +154,11 @@ inline hipError_t hipEventSynchronize(hipEvent_t e) {
   emu::waited = std::max(emu::waited.load(), static_cast<emu::Event *>(e)->at);
   return hipSuccess;
 }
-inline hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) { *ms = 0; return hipSuccess; }
+// a launch takes one millisecond
+inline hipError_t hipEventElapsedTime(float *ms, hipEvent_t a, hipEvent_t b) {
+  *ms = static_cast<float>(static_cast<emu::Event *>(b)->at - static_cast<emu::Event *>(a)->at);
+  return hipSuccess;
+}
 namespace emu {
 // stream capture: launches and async copies are recorded as closures and
 // replayed by hipGraphLaunch

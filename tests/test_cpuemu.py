@@ -9,6 +9,7 @@ oracle:
 - the 3-D mesh-database path (general hexahedra) on a small irregular mesh;
 - field reads and writes with no device memory left for their staging copy;
 - the number of launches that runs of many steps keep queued;
+- the times that a run reports;
 - the acoustic and coupled elastic-acoustic fixtures for a few steps (the
   regression case of an empty elastic receiver list, which once launched the
   elastic seismogram kernel on acoustic receivers).
@@ -33,7 +34,7 @@ def emu_lib(tmp_path_factory):
 
 @pytest.mark.parametrize("check", ["check_gather3d.py", "check_block3d.py", "check_paths2d.py",
                                    "check_acoustic2d.py", "check_database3d.py", "check_fields.py",
-                                   "check_queue.py"])
+                                   "check_queue.py", "check_timings.py"])
 def test_3d_paths_under_asan(emu_lib, check):
     lib = emu_lib
     asan = subprocess.run(["gcc", "-print-file-name=libasan.so"], capture_output=True, text=True,
