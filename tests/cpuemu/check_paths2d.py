@@ -115,6 +115,22 @@ eng.adjoint_run()
 check("adjoint run with checkpoints (atomic)", all(np.isfinite(v).all() for v in eng.kernels().values()))
 eng.close()
 
+# the same on patches, every third step sampled: traces, record and kernels of
+# the atomic scatter, whose loop runs step by step
+both = []
+for scatter in ("colored", "atomic"):
+    eng = Engine2D(mesh, SRC, REC, DT, NSTEP, 3, TYPES, scatter=scatter)
+    eng.initialize()
+    eng.set_field("displacement", 1e-3 * np.random.default_rng(3).standard_normal(eng.field("displacement").shape))
+    eng.forward_record(5)
+    got = [eng.seismograms(), eng.stacey_record()]
+    eng.set_adjoint_sources(REC, stf)
+    eng.adjoint_run()
+    both.append(got + [eng.seismograms()] + list(eng.kernels().values()))
+    eng.close()
+worst = max(rel_l2(a, b) for a, b in zip(*both))
+check("adjoint run on patches, every third step sampled", worst <= 1e-4, f"{worst:.2e}")
+
 # wavefield snapshots between fused steps (the test_gpu_wavefields sequence)
 
 
@@ -185,8 +201,9 @@ for chunk in (2, 64):
     check(f"chunk {chunk}", ok and e <= 1e-5, f"{e:.2e}")
 
 # a small batch of unequal meshes and step counts, every scatter: the
-# one-launch-per-step scatter against the engines' gather path bit for bit,
-# the colored one against their colored path, the atomic one within 1e-6
+# one-launch-per-step scatter against the engines' gather path bit for bit, the
+# colored and atomic ones within 1e-5 of the engines' patches (this build
+# contracts no products but those that the patches write out)
 SIZES = ((4, 5), (6, 8), (3, 8))
 single = {}
 for scatter in ("gather", "colored"):
@@ -207,8 +224,8 @@ for scatter, epb, graphs in (("gather", 2, True), ("gather", 5, False), ("gather
     b.run()
     ref = single["colored" if scatter == "atomic" else scatter]
     got = [b.seismograms(i) for i in range(len(SIZES))]
-    if scatter == "atomic":
-        ok = all(rel_l2(got[i].astype(np.float64), ref[i].astype(np.float64)) <= 1e-6 for i in range(len(SIZES)))
+    if scatter != "gather":
+        ok = all(rel_l2(got[i].astype(np.float64), ref[i].astype(np.float64)) <= 1e-5 for i in range(len(SIZES)))
     else:
         ok = all(np.array_equal(got[i], ref[i]) for i in range(len(SIZES)))
     info = b.info()
@@ -224,7 +241,7 @@ for e in engs:
     e.close()
 b.set_config(5, False, "colored")
 b.run()
-check("colored batch of atomic-scatter engines", all(np.array_equal(b.seismograms(i), single["colored"][i])
+check("colored batch of atomic-scatter engines", all(rel_l2(b.seismograms(i), single["colored"][i]) <= 1e-5
                                                      for i in range(len(SIZES))))
 b.close()
 
@@ -244,6 +261,28 @@ b.set_config(5, True, "gather")
 b.run()
 check("batch gather, every third step sampled", all(np.array_equal(b.seismograms(i), ref3[i]) for i in range(len(SIZES))))
 b.close()
+
+# a mesh above the line at which patches hold 51 elements: a few fused and
+# recorded steps and a combined one
+n_large = 3
+big = meshes.quad_mesh(161, 150, 0, 161 * H, 0, 150 * H, materials=[meshes.elastic(2400.0, 3000.0, 1732.0)],
+                       absorbing=("bottom", "right", "left"))
+at = [dict(x=x, z=z) for x, z in ((85 * H, 70.4 * H), (84.2 * H, 71 * H))]
+shot = [dict(x=84.6 * H, z=70.7 * H, angle=30.0, f0=150.0, factor=1e10)]
+r_big, _ = oracle.Oracle2D(big, 4, 1, DT).forward(shot, at, n_large, DT, 1, ("displacement", "acceleration"))
+for scatter in ("gather", "colored"):
+    eng = Engine2D(big, shot, at, DT, n_large, 1, ("displacement", "acceleration"), scatter=scatter)
+    eng.initialize()
+    eng.run()
+    e = rel_l2(eng.seismograms().astype(np.float64), r_big)
+    if scatter == "colored":
+        eng.initialize()
+        eng.forward_record(0)
+        eng.set_adjoint_sources(at, 1e-6 * rng.standard_normal((2, n_large, 2)))
+        eng.adjoint_run()
+        e = max(e, 0.0 if all(np.isfinite(v).all() for v in eng.kernels().values()) else 1.0)
+    eng.close()
+    check(f"large patches {scatter}", e <= 1e-5 and np.abs(r_big).max() > 0, f"{e:.2e}")
 
 print("failures:", failures, flush=True)
 sys.exit(1 if failures else 0)
