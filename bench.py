@@ -327,7 +327,7 @@ def algorithmic_bytes_2d(nspec: int, nglob: int, geometry: str = "point", elemen
                    layout): xix, xiz, gammax, gammaz, J per local point
                    (20 B x 25 / element), one 32-byte record per element
                    (affine elements), or the element's 4 or 9 control nodes
-                   (8 B each) from which the gather path recomputes it; the
+                   (8 B each) from which the patches recompute it; the
                    displacement gathered once per point (8 B), the
                    acceleration read-modify-written once per point (16 B)
       update_fused: a, M^-1, u, v read (32 B) and u, v, a written (24 B) per point

@@ -164,16 +164,23 @@ typedef struct {
 } sfx_run_desc;
 
 /* Scatter of element forces into the global acceleration.  COLORED groups the
- * elements into colors whose members share no global point and adds with plain
- * read-modify-write, one launch per color; ATOMIC adds every element point with
+ * elements into colors whose members share no global point; a point's forces are
+ * added in color order: by plain read-modify-write, one launch per color
+ * (structured 3-D meshes, the adjoint and backward wavefields' phases), or on
+ * chip or from stored contributions in the same order (whole steps and the
+ * forward wavefield's phases of 2-D elastic and of 3-D database meshes, whole
+ * steps of meshes with acoustic elements).  ATOMIC adds every element point with
  * a float atomic in one launch (the reference's atomic_add_on_device,
- * include/compute/fields/data_access.tpp:683-720). */
+ * include/compute/fields/data_access.tpp:683-720).  With both, an update or a
+ * step adds its forces to what the stored acceleration holds (the predictor
+ * clears it). */
 #define SFX_SCATTER_COLORED 0
 #define SFX_SCATTER_ATOMIC 1
-/* GATHER (3-D structured meshes): the stiffness kernel stores each element's
- * forces with coalesced writes; the fused update then sums, for every global
- * point, the contributions of its elements in a fixed order (deterministic,
- * no atomics, the acceleration is never stored between the two). */
+/* GATHER: every global point's contributions are summed in a fixed order
+ * (deterministic, no atomics) from the step's own forces alone.  3-D structured
+ * meshes: the stiffness kernel stores each element's forces with coalesced
+ * writes, the fused update sums them.  2-D elastic meshes (forward runs): summed
+ * on chip in element order, every product and sum rounded on its own. */
 #define SFX_SCATTER_GATHER 2
 /* BLOCK (3-D structured meshes with even nx, ny, nz): one workgroup computes
  * 2 x 2 x 2 elements, sums their forces in on-chip memory in a fixed order and

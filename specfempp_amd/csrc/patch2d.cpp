@@ -87,8 +87,12 @@ uint64_t hash_of(const std::vector<uint16_t> &v) {
 }  // namespace
 
 // Small patches while large ones would leave compute units without a
-// workgroup: at 6,400 elements 8.4 against 8.9 us a step, at 23,000 11.2 and
-// 11.5 us, at 900,000 257 and 247 us (small, large).
+// workgroup.  us a step, small and large (colored, 8 sources, 32 receivers; the
+// gather form 0.5 to 4 more, in the same order): 6,400 elements 8.62 and 9.19;
+// 16,900 9.63 and 9.61; 23,187 10.58 and 11.19; 30,000 11.88 and 11.30; 39,900
+// 12.88 and 12.84; 50,000 15.22 and 14.69; 61,103 20.79 and 20.04; 90,000 24.73
+// and 24.15; 160,000 39.03 and 37.34; 250,000 54.43 and 54.75; 490,000 128.1 and
+// 113.5.  How many rounds of workgroups a size makes moves both forms alike.
 int patch_elements(int64_t nspec) { return nspec > 24000 ? PATCH_LARGE : PATCH_SMALL; }
 
 void add_patches(PatchPlan &plan, const HostAssembly &h, const std::vector<int32_t> &key, bool colored) {

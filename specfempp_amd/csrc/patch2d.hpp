@@ -4,8 +4,8 @@
 // A point all of whose elements lie in one patch is interior to it: the
 // patch's workgroup assembles its force, divides by the mass and applies the
 // corrector and the next predictor, with no force leaving the chip.  Points
-// shared by several patches (about 1 in 16 at 64 elements a patch) are
-// boundary points: every patch stores the element contributions of its
+// shared by several patches (1 in 13 with 45 elements a patch, 1 in 9.5 with 21)
+// are boundary points: every patch stores the element contributions of its
 // boundary points, and the next launch sums them (in every patch that needs
 // the point, all with the same operands), so one launch carries a time step
 // and no grid-wide synchronisation is needed.  Boundary state and
