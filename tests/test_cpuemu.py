@@ -37,9 +37,10 @@ def emu_lib(tmp_path_factory):
                                    "check_queue.py", "check_timings.py"])
 def test_3d_paths_under_asan(emu_lib, check):
     lib = emu_lib
-    asan = subprocess.run(["gcc", "-print-file-name=libasan.so"], capture_output=True, text=True,
-                          check=True).stdout.strip()
-    env = dict(os.environ, LD_PRELOAD=asan, ASAN_OPTIONS="detect_leaks=0")
+    # libstdc++ beside it, so that ASan finds the function that throws
+    preload = [subprocess.run(["gcc", f"-print-file-name={name}"], capture_output=True, text=True, check=True).stdout.strip()
+               for name in ("libasan.so", "libstdc++.so")]
+    env = dict(os.environ, LD_PRELOAD=" ".join(preload), ASAN_OPTIONS="detect_leaks=0")
     extra = ["2"] if check == "check_acoustic2d.py" else []  # steps of each acoustic run
     r = subprocess.run([sys.executable, os.path.join(HERE, "cpuemu", check), lib] + extra, env=env,
                        capture_output=True, text=True, timeout=3600)
