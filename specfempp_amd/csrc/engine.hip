@@ -8,6 +8,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <future>
 #include <memory>
 #include <mutex>
 #include <numeric>
@@ -684,12 +685,13 @@ struct sfx_engine {
     snap.alloc(static_cast<size_t>(h.nrec) * 125 * 6);
   }
 
-  void upload() {
+  // number_points: puts the points in device order; called once what does not
+  // depend on their order is on the device
+  template <class F> void upload(F &&number_points) {
     lat = Lattice{h.nx, h.ny, h.nz, h.nx + 1, h.ny + 1, h.nz + 1, h.nint_pad};
     SFX_HIP(hipGetDevice(&device));
     SFX_HIP(hipStreamCreate(&stream));
     hipStream_t s = stream;
-    gather.upload(permuted(h.gather), s);
     kappa.upload(permuted(h.kappa), s);
     mu.upload(permuted(h.mu), s);
     upload_element_properties(s);
@@ -713,6 +715,10 @@ struct sfx_engine {
       }
       rec_index.upload(ri, s);
       bnd_rec.upload(br, s);
+    }
+    number_points();
+    gather.upload(permuted(h.gather), s);
+    if (h.dim == 2) {
       if (patches()) {
         const float dt = static_cast<float>(run.dt);
         const PatchSim sim{dt, static_cast<float>(dt / 2.0), static_cast<float>(dt * dt / 2.0), run.nstep,
@@ -1381,20 +1387,31 @@ template <class Build> int create(Build &&build, const sfx_run_desc *run, sfx_en
       e->h.color_offsets = {0, e->h.nspec};
       e->h.ncolors_el = 1;
     }
-    if (e->patches()) {
-      // a point's contributions are summed by element in compute order
-      // (gather) or in color order
-      e->plan.pe = patch_elements(e->h.nspec);
-      std::vector<int32_t> key(e->h.nspec);
-      std::iota(key.begin(), key.end(), 0);
-      const bool colored = run->scatter == SFX_SCATTER_COLORED;
-      add_patches(e->plan, e->h, colored ? e->h.inv_perm : key, colored);
-      finish_patches(e->plan);
-      renumber_points(e->h, e->plan);
-      e->plan.device_of.clear();
-    }
     e->nsig = (run->nstep + run->nstep_between_samples - 1) / run->nstep_between_samples;
-    if (!host_only) e->upload();
+    if (e->patches()) {
+      // The plan is made while the arrays that do not depend on it go to the
+      // device (from about 2,000 elements on: below that it takes less than
+      // starting a thread).  The future's end waits for it if the upload fails.
+      auto make_plan = [&e, run] {
+        // a point's contributions are summed by element in compute order
+        // (gather) or in color order
+        e->plan.pe = patch_elements(e->h.nspec);
+        std::vector<int32_t> key(e->h.nspec);
+        std::iota(key.begin(), key.end(), 0);
+        const bool colored = run->scatter == SFX_SCATTER_COLORED;
+        add_patches(e->plan, e->h, colored ? e->h.inv_perm : key, colored);
+        finish_patches(e->plan);
+      };
+      std::future<void> plan = e->h.nspec < 2000 ? std::async(std::launch::deferred, make_plan)
+                                                 : std::async(std::launch::async | std::launch::deferred, make_plan);
+      e->upload([&] {
+        plan.get();
+        renumber_points(e->h, e->plan);
+        e->plan.device_of.clear();
+      });
+    } else if (!host_only) {
+      e->upload([] {});
+    }
     *out = e.release();
   });
 }

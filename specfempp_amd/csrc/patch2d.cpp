@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <future>
 #include <numeric>
 
 #include "../../include/specfempp_amd.h"
@@ -26,7 +27,7 @@ struct Bisection {
   const std::vector<float> &cx, &cz;
   std::vector<int32_t> &order;
   int pe;
-  std::vector<std::pair<int, int>> out;
+  using Groups = std::vector<std::pair<int, int>>;
 
   int cut(int a, int b, int want) {
     float lo[2] = {cx[order[a]], cz[order[a]]}, hi[2] = {lo[0], lo[1]};
@@ -58,8 +59,9 @@ struct Bisection {
     return a + k;
   }
   // [a, b) into `parts` groups of about equal size, cut again where the
-  // rounding to whole columns left one too large
-  void split(int a, int b, int parts) {
+  // rounding to whole columns left one too large; the halves of a large range on
+  // up to `threads` host threads
+  void split(int a, int b, int parts, Groups &out, int threads) {
     if (parts <= 1 && b - a > pe) parts = 2;
     if (parts <= 1 || b - a <= 1) {
       out.push_back({a, b});
@@ -67,8 +69,17 @@ struct Bisection {
     }
     const int left = parts / 2;
     const int m = cut(a, b, std::max(1, static_cast<int>(static_cast<int64_t>(b - a) * left / parts)));
-    split(a, m, left);
-    split(m, b, parts - left);
+    if (threads < 2 || b - a < 2000) {
+      split(a, m, left, out, 1);
+      split(m, b, parts - left, out, 1);
+      return;
+    }
+    Groups right;
+    std::future<void> job = std::async(std::launch::async | std::launch::deferred,
+                                       [&] { split(m, b, parts - left, right, threads / 2); });
+    split(a, m, left, out, threads - threads / 2);
+    job.get();
+    out.insert(out.end(), right.begin(), right.end());
   }
 };
 
@@ -106,12 +117,12 @@ void add_patches(PatchPlan &plan, const HostAssembly &h, const std::vector<int32
   }
   std::vector<int32_t> order(ns);
   std::iota(order.begin(), order.end(), 0);
-  Bisection bis{cx, cz, order, pe, {}};
+  Bisection bis{cx, cz, order, pe};
   // the average size to aim at, below the limit so that cuts at whole columns
   // seldom leave a group that must be cut again
   const int target = pe == PATCH_LARGE ? 45 : 22;
-  bis.split(0, ns, (ns + target - 1) / target);
-  std::vector<std::pair<int, int>> groups = std::move(bis.out);
+  Bisection::Groups groups;
+  bis.split(0, ns, (ns + target - 1) / target, groups, 8);
 
   // colored: the points of each element that have a Stacey term, and all of
   // an element with sources, have one more contribution each
