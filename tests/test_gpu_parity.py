@@ -113,9 +113,9 @@ def test_forward_seismograms_match_oracle_and_specfem2d(case, scatter):
 @pytest.mark.parametrize("scatter", ["colored", "gather"])
 def test_non_affine_mesh_matches_oracle(scatter):
     """Interior nodes moved by up to a quarter element: the geometry varies over
-    each element, so the colored stiffness reads it per point (affine meshes use
-    one record per element) and the gather path recomputes it at every point
-    from the element's 4 control nodes, giving the oracle's bits."""
+    each element, so the patches recompute it at every point from the element's
+    4 control nodes (affine meshes use one record per element); the gather
+    scatter gives the oracle's bits."""
     from specfempp_amd import Engine2D, meshes
 
     n, h = 24, 10.0
