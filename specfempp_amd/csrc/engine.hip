@@ -685,13 +685,14 @@ struct sfx_engine {
     snap.alloc(static_cast<size_t>(h.nrec) * 125 * 6);
   }
 
-  // number_points: puts the points in device order; called once what does not
-  // depend on their order is on the device
+  // number_points: puts the points of a patch engine in device order; called once
+  // what does not depend on their order is on the device
   template <class F> void upload(F &&number_points) {
     lat = Lattice{h.nx, h.ny, h.nz, h.nx + 1, h.ny + 1, h.nz + 1, h.nint_pad};
     SFX_HIP(hipGetDevice(&device));
     SFX_HIP(hipStreamCreate(&stream));
     hipStream_t s = stream;
+    if (!patches()) gather.upload(permuted(h.gather), s);
     kappa.upload(permuted(h.kappa), s);
     mu.upload(permuted(h.mu), s);
     upload_element_properties(s);
@@ -715,11 +716,9 @@ struct sfx_engine {
       }
       rec_index.upload(ri, s);
       bnd_rec.upload(br, s);
-    }
-    number_points();
-    gather.upload(permuted(h.gather), s);
-    if (h.dim == 2) {
       if (patches()) {
+        number_points();
+        gather.upload(permuted(h.gather), s);
         const float dt = static_cast<float>(run.dt);
         const PatchSim sim{dt, static_cast<float>(dt / 2.0), static_cast<float>(dt * dt / 2.0), run.nstep,
                            run.nstep_between_samples, h.nrec, 0};

@@ -127,18 +127,12 @@ template <int PE> constexpr int patch_threads() { return (PE * 5 + 63) / 64 * 64
 
 // Sum of an interior point's contributions in order, the first one (table
 // entry ea) given: its local index l tells how many there are (the points are
-// sorted by that number).  a0, a1: the patch's stored acceleration the sum
-// starts from, or null.
+// sorted by that number).
 __device__ __forceinline__ float2 interior_force(const PatchHead &h, const uint16_t *__restrict__ tab,
-                                                 const float *st, int l, int ea, int eb, const float *a0 = nullptr,
-                                                 const float *a1 = nullptr) {
+                                                 const float *st, int l, int ea, int eb) {
 #pragma clang fp contract(off)
   const float2 *f = reinterpret_cast<const float2 *>(st);
   float2 s = f[ea];
-  if (a0) {
-    s.x = at(a0, l) + s.x;
-    s.y = at(a1, l) + s.y;
-  }
   if (l >= h.n1) {
     const float2 r = f[eb];
     s.x += r.x;
@@ -575,12 +569,11 @@ __global__ __launch_bounds__(patch_threads<PE>()) __attribute__((amdgpu_waves_pe
     for (int k = t; k < h.nbent; k += NT) out[T.bslot[h.be0 + k]] = f[tab[h.bent + k]];
   }
   const bool snapshot = h.rm0 >= 0 && L.advance && n % h.nsb == 0;
-  const float *const a0p = !EXACT && L.add_a ? S.a + h.pt0 : nullptr, *const a1p = a0p ? S.a + np + h.pt0 : nullptr;
 #pragma unroll
   for (int k = 0; k < NI; k++) {
     const int l = t + k * NT;
     if (l >= h.nint) continue;
-    const float2 s = interior_force(h, tab, se, l, ea[k], eb[k], a0p, a1p);
+    const float2 s = interior_force(h, tab, se, l, ea[k], eb[k]);
     const float a0 = s.x * mi[k][0], a1 = s.y * mi[k][1];
     if (L.advance) {
       float u0 = su[0][l], u1 = su[1][l], v0 = vi[k][0], v1 = vi[k][1], w0, w1;
@@ -604,8 +597,11 @@ __global__ __launch_bounds__(patch_threads<PE>()) __attribute__((amdgpu_waves_pe
       }
     }
     if (!L.advance || L.store_a) {
-      put(S.a + h.pt0, l, a0);
-      put(S.a + np + h.pt0, l, a1);
+      float *const a0p = S.a + h.pt0, *const a1p = S.a + np + h.pt0;
+      // a force held in the stored a joins here, out of the way of fused steps
+      const bool add = !EXACT && L.add_a;
+      put(a0p, l, add ? (s.x + at(a0p, l)) * mi[k][0] : a0);
+      put(a1p, l, add ? (s.y + at(a1p, l)) * mi[k][1] : a1);
     }
   }
 }

@@ -167,7 +167,7 @@ struct PatchLaunch {
   int pending;   // the contributions of step - 1 are summed first
   int advance;   // 1: corrector and predictor; 0: only a = M^-1 f (seam calls)
   int store_a;   // advance: keep a as well
-  int add_a;     // contracted form, no advance: the sums start from the stored a
+  int add_a;     // contracted form, no advance: the stored a joins the sums
   float *rec;    // contracted form: the Stacey elements' forces of step n go to rec + n * rec_stride, or null
   long long rec_stride;
 };
@@ -232,7 +232,7 @@ void launch_patch_step(hipStream_t s, int pe, int npatch, int nrec, bool exact, 
                        const PatchState &st, const GllConst &q, const PatchLaunch &l);
 // Boundary points, from the contributions in buffer rd: with advance the
 // corrector and predictor into state A (a too with store_a), else a only.
-// add_a: the sums start from the stored a.
+// add_a: the stored a joins the sums.
 void launch_patch_boundary(hipStream_t s, bool exact, const PatchTables &t, const PatchState &st, NewmarkConst nc,
                            int rd, int advance, int store_a, int add_a);
 void launch_patch_pair(hipStream_t s, int pe, int npatch, int nrec, const PatchTables &t, const PatchState &adj,
